@@ -201,9 +201,11 @@ def _scoring(case):
 
 
 class _DeviceArray:
-    """int32 device memory of a batch's results, for torch.as_tensor."""
+    """int32 device memory of a batch's results, for torch.as_tensor.  It holds the
+    batch, which owns the memory: a tensor made of it may outlive the state."""
 
-    def __init__(self, ptr, shape):
+    def __init__(self, batch, ptr, shape):
+        self.batch = batch
         self.__cuda_array_interface__ = {"data": (ptr, False), "shape": shape, "typestr": "<i4", "version": 2}
 
 
@@ -211,7 +213,7 @@ def _device_results(batch):
     p = ctypes.c_void_p()
     if gbsw.load_library().gbsw_batch_device_results(batch._h, ctypes.byref(p)) != 0:
         raise RuntimeError("gbsw_batch_device_results failed")
-    return torch.as_tensor(_DeviceArray(p.value, (5, batch.n)), device="cuda")
+    return torch.as_tensor(_DeviceArray(batch, p.value, (5, batch.n)), device="cuda")
 
 
 def _requests(case):
