@@ -49,8 +49,8 @@ PEAK_INT_TOPS_PACKED = MI355X_CU * 64 * MI355X_GHZ * 2 / 1000.0  # 78.6 TOP/s (i
 
 
 # launch kind -> (kernel, cell policy)
-KIND_NAMES = {2: ("k_batched", "Packed16"), 3: ("k_batched", "Wide32"), 4: ("k_batched", "PackedF16"),
-              5: ("k_split", "Packed16"), 6: ("k_split", "PackedF16")}
+KIND_NAMES = {2: ("k_batched", "Packed16"), 3: ("k_batched", "Wide32"), 4: ("k_sweep", "Sweep16"),
+              5: ("k_split", "Packed16"), 6: ("k_sweep_split", "Sweep16")}
 
 
 def log(*a):

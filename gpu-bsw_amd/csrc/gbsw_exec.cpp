@@ -106,6 +106,11 @@ int lds_for(int K, int alpha, bool p8, int bnd_bytes = 4)
     return lds_layout(prof_row_bytes(K, p8), alpha, bnd_bytes).total;
 }
 
+int sweep_lds_for(int K, int alpha, int form)
+{
+    return sweep_lds(kLanesPerPair, K, form, alpha, 4).total;
+}
+
 int grid_for(const Exec& ex, int kind, int K, int lds, int64_t nquads)
 {
     int occ = kernel_occupancy(kind, K, lds);
@@ -127,7 +132,7 @@ int launch_timed(Exec& ex, hipStream_t stream, int kind, int K, int grid, int ld
     GBSW_HIP_TRY(hipEventRecord(ex.kev[2 * slot], stream));
     GBSW_HIP_TRY(kernel_launch(kind, K, grid, lds, stream, a));
     GBSW_HIP_TRY(hipEventRecord(ex.kev[2 * slot + 1], stream));
-    ex.launches.push_back({kind, K, grid, 0, 0, 0.0});
+    ex.launches.push_back({kind & kReportedKind, K, grid, 0, 0, 0.0});
     return GBSW_OK;
 }
 
@@ -267,7 +272,7 @@ double occupancy_threshold(int model)
 double occupancy_factor(int K, int alpha, double threshold)
 {
     static std::mutex mu;
-    static std::map<int, int> cache; // workgroups per CU
+    static std::map<int, int> cache; // workgroups per CU (the usual kernel of the alphabet)
     int wg_per_cu = 0;
     {
         std::lock_guard<std::mutex> lk(mu);
@@ -276,21 +281,18 @@ double occupancy_factor(int K, int alpha, double threshold)
         if (it != cache.end()) {
             wg_per_cu = it->second;
         } else {
-            // one wave each; a small alphabet's usual tables (exact f16 high
-            // bytes) run the f16 kernels on a byte profile
-            const bool p8 = byte_profile_alphabet(alpha);
-            wg_per_cu = kernel_occupancy(with_profile(kBatched, p8), K, lds_for(K, alpha, p8));
-            if (!p8 && kernel_has(kBatchedF16, K))
-                wg_per_cu = std::max(wg_per_cu, kernel_occupancy(with_profile(kBatchedF16, true), K, lds_for(K, alpha, true)));
+            // one wave each
+            const int form = alpha <= kRegAlpha ? kProfRegs : kProfBytes;
+            wg_per_cu = kernel_occupancy(sweep_kind(kBatchedF16, form), K, sweep_lds_for(K, alpha, form));
             cache.emplace(key, wg_per_cu);
         }
     }
     return (wg_per_cu > 0 && threshold > 0) ? std::min(1.0, wg_per_cu / 4.0 / threshold) : 1.0;
 }
 
-int k_for_cols(int cols, int alpha, int model)
+int k_for_cols(int cols, int alpha, int model, int klimit)
 {
-    const int kmax = max_k_for(alpha, byte_profile_alphabet(alpha));
+    const int kmax = std::min(klimit, max_k_for(alpha, byte_profile_alphabet(alpha)));
     int nk = 0;
     const int* ks = kernel_k_list(&nk);
     int best = ks[0];
@@ -337,16 +339,15 @@ const std::vector<uint8_t>& bucket_table(int alpha, int model)
     // strip counts, hence the choice, only change at multiples of 32 columns:
     // the lengths (32(j-1), 32j] share the choice made for 32j
     std::vector<int> kblk(65536 / 32 + 1);
-    for (size_t j = 0; j < kblk.size(); ++j) kblk[j] = k_for_cols((int)(32 * j), alpha, model);
+    for (size_t j = 0; j < kblk.size(); ++j) kblk[j] = k_for_cols((int)(32 * j), alpha, model, kSweepMaxK);
     std::vector<uint8_t> t(65536);
     for (int m = 0; m < 65536; ++m) {
         const int K = kblk[(size_t)((m + 31) / 32)];
         int idx = 0;
         while (idx < nk && ks[idx] != K) ++idx;
         // pairs spanning several strips get buckets of their own, so a single-strip
-        // bucket bounds its scores by 32 x K columns; those up to kMultiShortCols
-        // columns apart from longer ones, whose bound (with DNA scores up to 3)
-        // still allows the f16 kernels
+        // bucket hands no boundary rows on; those up to kMultiShortCols columns apart
+        // from longer ones
         const bool multi = m > kVirtPerPair * K;
         const int cls = !multi ? 0 : m <= kMultiShortCols ? 1 : 2;
         t[(size_t)m] = (uint8_t)(idx + cls * nk);
@@ -392,10 +393,8 @@ int batched_grid_cap(const Exec& ex, int K, int alpha)
     // admission reserved for it
     const bool p8 = byte_profile_alphabet(alpha);
     int occ = kernel_occupancy(with_profile(kBatched, p8), K, lds_for(K, alpha, p8));
-    if (kernel_has(kBatchedF16, K)) {
-        occ = std::max(occ, kernel_occupancy(kBatchedF16, K, lds_for(K, alpha, false)));
-        occ = std::max(occ, kernel_occupancy(with_profile(kBatchedF16, true), K, lds_for(K, alpha, true)));
-    }
+    for (int form = alpha <= kRegAlpha ? kProfRegs : kProfBytes; form <= kProfWords; ++form)
+        occ = std::max(occ, kernel_occupancy(sweep_kind(kBatchedF16, form), K, sweep_lds_for(K, alpha, form)));
     return std::max(1, occ) * ex.num_cu;
 }
 
@@ -404,17 +403,33 @@ bool f16_high_byte_exact(int32_t s)
     // an integer is an f16 value with a zero low byte when it has at most three
     // significant bits (leading one and two mantissa bits) below 2^11
     const int32_t a = s < 0 ? -s : s;
-    if (a >= kF16Exact) return false;
+    if (a >= 2048) return false;
     return a == 0 || (a >> __builtin_ctz((uint32_t)a)) < 8;
 }
 
-int batched_kind(const Bucket& bk, int32_t max_sub, bool allow_f16)
+SweepChoice sweep_choice(const std::vector<int16_t>& sub, int alpha, int32_t gap_open, int32_t gap_extend,
+                         int32_t max_sub, bool bytes)
 {
-    // every cell value of a pair is at most its score plus one substitution, and
-    // the score at most (shorter length) x (best substitution)
-    const int64_t bound = (int64_t)bk.max_cols * max_sub + max_sub;
-    if (allow_f16 && kernel_has(kBatchedF16, bk.K) && bound < kF16Exact) return kBatchedF16;
-    return kBatched;
+    SweepChoice c;
+    const int32_t ge = -gap_extend, go = -gap_open, bias = ge + go;
+    int32_t lo = 1 << 30, hi = -(1 << 30);
+    for (int r = 0; r < alpha; ++r)
+        for (int q = 0; q < alpha; ++q) {
+            lo = std::min<int32_t>(lo, sub[(size_t)(r * alpha + q)] + bias);
+            hi = std::max<int32_t>(hi, sub[(size_t)(r * alpha + q)] + bias);
+        }
+    // every value stays non-negative: the smallest is a zero cell's Ho plus the
+    // smallest biased score
+    c.base = go + std::max(0, -lo) + 4;
+    const int64_t offset = (int64_t)c.base + (int64_t)ge * (kRebase + 40);
+    // the padding scores -(open + extend), which must be negative; the running
+    // offset and the scores leave most of the range to the cell values
+    c.ok = bias >= 1 && offset <= 8192 && max_sub <= 4096 && lo > -16384 && hi < 16384;
+    c.form = (bytes && lo >= 0 && hi <= 255) ? (alpha <= kRegAlpha ? kProfRegs : kProfBytes) : kProfWords;
+    // a pair below this never formed a value past 0x7C00 (largest offset, gap step
+    // and one substitution on top of its best)
+    c.sat_limit = (int32_t)(0x7C00 - offset - 2 * ge - max_sub - 4);
+    return c;
 }
 
 int sort_scratch_bytes(int64_t n, size_t* bytes)
@@ -467,7 +482,7 @@ int prepare_scoring(const Job& job, const gbsw_scoring* sc, std::vector<int16_t>
     for (int16_t v : sub) lo = std::min<int>(lo, v);
     *p8 = byte_profile_alphabet(A) && lo >= -127 && mx <= 127;
     if (f16p8) {
-        // the f16 kernels can read a byte profile (the scores' f16 high bytes)
+        // scores with at most three significant bits: held as bytes
         *f16p8 = true;
         for (int16_t v : sub) *f16p8 = *f16p8 && f16_high_byte_exact(v);
     }
@@ -481,16 +496,16 @@ namespace {
 // One length bucket's launch in the batched form.
 struct BucketPlan {
     int kind = 0, K = 0, grid = 0, lds = 0, strips = 1;
+    int32_t sat_limit = 0;
     size_t bnd_at = 0, split_at = 0; // 32-bit word offsets into ex.bnd / ex.split_buf
 };
 
 // Estimated duration of a bucket (relative): cells x (K + 2) / K (padding and
-// per-step overhead), +15 % for int16 cells, x2.5 for the split form (its strips
-// wait for each other; it issues VALU at 0.3-0.7 of the other kernels' rate).
+// per-step overhead), +40 % for the int16 kernels, and the split form's weight.
 double bucket_cost(const BucketPlan& b, const Bucket& bk)
 {
-    const int k = b.kind & ~kByteProfile;
-    const double f16 = (k == kBatchedF16 || k == kSplitF16) ? 1.0 : 1.15;
+    const int k = b.kind & 0xFF;
+    const double f16 = (k == kBatchedF16 || k == kSplitF16) ? 1.0 : 1.4;
     // a split bucket's strips wait on each other, and beside the bulk buckets it
     // runs several times longer than alone (the K = 7 split bucket of the 1M-pair
     // DNA mix: 1.0 ms alone, 6.6 ms beside them); weights 2.5 / 4 / 6 / 8 / 12
@@ -501,7 +516,7 @@ double bucket_cost(const BucketPlan& b, const Bucket& bk)
 
 bool plan_is_split(const BucketPlan& b)
 {
-    const int k = b.kind & ~kByteProfile;
+    const int k = b.kind & 0xFF;
     return k == kSplit || k == kSplitF16;
 }
 
@@ -518,33 +533,41 @@ size_t split_words_of(const Bucket& bk, const BucketPlan& b)
 }
 
 // Kernels, grids and scratch of every bucket (host only; reserves the buffers).
-int plan_batched(Exec& ex, const Job& job, int max_sub, bool p8, bool f16p8, bool asym, int kclamp, int64_t bnd_rows,
-                 std::vector<BucketPlan>& plan, std::vector<size_t>& order)
+int plan_batched(Exec& ex, const Job& job, int max_sub, bool p8, const SweepChoice& sw, bool asym, int kclamp,
+                 int64_t bnd_rows, std::vector<BucketPlan>& plan, std::vector<size_t>& order)
 {
     const size_t nb = job.buckets.size();
     plan.assign(nb, BucketPlan{});
     order.resize(nb);
-    // the unsplit kernel of a bucket and its LDS layout: the int16 kernels use
-    // the job's profile (p8), the f16 ones a byte profile when the table allows
-    // it (f16p8, a third of the LDS of DNA's int16 profile: more workgroups per
-    // CU) and else the int16 profile, which a byte-profile alphabet does not get
-    const bool allow_f16 = ex.f16 && (f16p8 || !p8);
+    // the unsplit kernel of a bucket: the sweep kernel of the job's profile form in
+    // the widest geometry that fits its LDS, else (scorings outside the sweep
+    // kernels' range, option F16 off) the int16 kernel
+    int nk = 0;
+    const int* ks = kernel_k_list(&nk);
     auto unsplit = [&](BucketPlan& b, const Bucket& bk) {
-        const int k = batched_kind(bk, max_sub, allow_f16);
-        const bool bp8 = k == kBatchedF16 ? f16p8 : p8;
-        b.kind = with_profile(k, bp8);
-        b.lds = lds_for(b.K, job.alpha, bp8);
+        b.K = std::min(kclamp, bk.K);
+        if (sw.ok) {
+            int i = 0;
+            while (i + 1 < nk && ks[i + 1] <= bk.K) ++i;
+            while (i > 0 && sweep_lds_for(ks[i], job.alpha, sw.form) > 65536) --i;
+            b.K = ks[i];
+            b.kind = sweep_kind(kBatchedF16, sw.form);
+            b.lds = sweep_lds_for(b.K, job.alpha, sw.form);
+            b.sat_limit = sw.sat_limit;
+        } else {
+            b.kind = with_profile(kBatched, p8);
+            b.lds = lds_for(b.K, job.alpha, p8);
+            b.sat_limit = 32767 - max_sub;
+        }
     };
     for (size_t i = 0; i < nb; ++i) {
         order[i] = i;
         const Bucket& bk = job.buckets[i];
         BucketPlan& b = plan[i];
-        b.K = std::min(kclamp, bk.K);
         unsplit(b, bk);
-        const bool bp8 = (b.kind & kByteProfile) != 0;
         const int64_t nquads = (bk.count + kPairsPerWave - 1) / kPairsPerWave;
         b.strips = std::max(1, (bk.max_cols + kVirtPerPair * b.K - 1) / (kVirtPerPair * b.K));
-        const int skind = with_profile((b.kind & ~kByteProfile) == kBatchedF16 ? kSplitF16 : kSplit, bp8);
+        const int skind = sw.ok ? sweep_kind(kSplitF16, sw.form) : with_profile(kSplit, p8);
         // A split item waits about four chunks for its predecessor's first
         // rows: worth it only when the bucket has too few quads to keep every
         // workgroup busy for two rounds (on the 200k-pair DNA mix: 1765 vs 827
@@ -625,7 +648,7 @@ int plan_batched(Exec& ex, const Job& job, int max_sub, bool p8, bool f16p8, boo
 }
 
 // Stream work of the batched form (recorded eagerly or into a graph).
-int record_batched(Exec& ex, const Job& job, KernelArgs a, int max_sub, const std::vector<BucketPlan>& plan,
+int record_batched(Exec& ex, const Job& job, KernelArgs a, const std::vector<BucketPlan>& plan,
                    const std::vector<size_t>& order, size_t sub_bytes)
 {
     hipStream_t st0 = ex.stream;
@@ -665,8 +688,7 @@ int record_batched(Exec& ex, const Job& job, KernelArgs a, int max_sub, const st
         a.order = job.order + bk.begin;
         a.order_n = bk.count;
         a.queue = ex.queue.as<uint32_t>() + kXcds * i;
-        const int base_kind = b.kind & ~kByteProfile;
-        a.sat_limit = (base_kind == kBatchedF16 || base_kind == kSplitF16) ? kF16Exact - max_sub : 32767 - max_sub;
+        a.sat_limit = b.sat_limit;
         std::memset(&a.split, 0, sizeof(a.split));
         if (plan_is_split(b)) {
             uint32_t* w = ex.split_buf.as<uint32_t>() + b.split_at;
@@ -772,7 +794,7 @@ int enqueue_job(Exec& ex, const Job& job, const gbsw_scoring* sc, int mode)
         // pairs more than the extra waves gain (793 vs 593 GCUPS on the 1M-pair
         // DNA mix), so it applies to profile-free alphabets only
         const int K = std::min(kclamp, k_for_cols(job.max_cols, job.alpha,
-                                                  byte_profile_alphabet(job.alpha) ? job.kmodel : kModelClassic));
+                                                  byte_profile_alphabet(job.alpha) ? job.kmodel : kModelClassic, 1 << 30));
         const int lds = lds_for(K, job.alpha, p8);
         const int64_t nquads = (job.n + kPairsPerWave - 1) / kPairsPerWave;
         a.order = nullptr;
@@ -803,12 +825,18 @@ int enqueue_job(Exec& ex, const Job& job, const gbsw_scoring* sc, int mode)
     }
     std::vector<BucketPlan> plan;
     std::vector<size_t> order;
-    rc = plan_batched(ex, job, max_sub, p8, f16p8, a.asym != 0, kclamp, a.bnd_rows, plan, order);
+    // scores of the sweep kernels: bytes where they fit an int8 profile (large
+    // alphabets) or have at most three significant bits (small ones), else 16 bits
+    SweepChoice sw = sweep_choice(sub, job.alpha, sc->gap_open, sc->gap_extend, max_sub,
+                                  byte_profile_alphabet(job.alpha) ? p8 : f16p8);
+    sw.ok = sw.ok && ex.f16;
+    a.base = sw.base;
+    rc = plan_batched(ex, job, max_sub, p8, sw, a.asym != 0, kclamp, a.bnd_rows, plan, order);
     if (rc) return rc;
     const size_t sub_bytes = sizeof(int16_t) * sub.size();
     if (!ex.graphs || ex.fixed || !job.graph) {
         GBSW_HIP_TRY(hipEventRecord(ex.ev_start, st0));
-        rc = record_batched(ex, job, a, max_sub, plan, order, sub_bytes);
+        rc = record_batched(ex, job, a, plan, order, sub_bytes);
         if (rc) return rc;
         GBSW_HIP_TRY(hipEventRecord(ex.ev_stop, st0));
         return GBSW_OK;
@@ -821,7 +849,7 @@ int enqueue_job(Exec& ex, const Job& job, const gbsw_scoring* sc, int mode)
     if (!G.exec || G.key != key) {
         G.reset();
         GBSW_HIP_TRY(hipStreamBeginCapture(st0, hipStreamCaptureModeRelaxed));
-        rc = record_batched(ex, job, a, max_sub, plan, order, sub_bytes);
+        rc = record_batched(ex, job, a, plan, order, sub_bytes);
         hipGraph_t graph = nullptr;
         const hipError_t ce = hipStreamEndCapture(st0, &graph);
         if (rc) {

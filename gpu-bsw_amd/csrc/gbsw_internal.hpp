@@ -92,7 +92,7 @@ struct Exec {
     int streams = kDefaultStreams; // streams for the length buckets (1 = serialised)
     // creates the auxiliary streams the first n streams need
     int ensure_streams(int n);
-    bool f16 = true;               // exact f16 kernels where the score bound allows
+    bool f16 = true;               // sweep kernels where the scoring fits their range
     bool split = true;             // multi-strip buckets run their strips on several workgroups
     bool split_misplaced = false;  // a split launch ran workgroups of one XCD counter on different
                                    // XCCs: the split form stays off for this Exec
@@ -170,8 +170,9 @@ constexpr int kModelOccupancy = 1;
 // 2.5, 2.0, 3.0, 4.0, 1.5 waves
 constexpr int kGeometryModels = 6;
 double occupancy_threshold(int model);
-// K for a shorter sequence of `cols` residues.
-int k_for_cols(int cols, int alpha, int model);
+// K for a shorter sequence of `cols` residues, at most klimit.
+int k_for_cols(int cols, int alpha, int model, int klimit);
+constexpr int kSweepMaxK = 16; // widest sweep kernel with four pairs per wave
 // Bucket ids: position of K in kernel_k_list, plus once the list's length for
 // pairs that span several strips with at most kMultiShortCols columns, twice for
 // longer ones (bucket_ids() in all).
@@ -181,17 +182,24 @@ const std::vector<uint8_t>& bucket_table(int alpha, int model);
 // Key bits of the device radix sort: bucket id << 16 | (65535 - longer length).
 constexpr int kSortBits = 22;
 // Multi-strip pairs up to this many columns form buckets of their own (ids nk ..
-// 2nk-1), longer ones the ids 2nk .. 3nk-1: 512 x 3 + 3 < 2048 keeps DNA buckets
-// of the first class on the exact f16 kernels.
+// 2nk-1), longer ones the ids 2nk .. 3nk-1, so that a wave's pairs and a bucket's
+// strips are of like length.
 constexpr int kMultiShortCols = 512;
 // Fill job.buckets from per-pair lengths (host), ordered by ascending K.
 void count_buckets(Job& job, const int32_t* len_ref, const int32_t* len_qry);
 // Workgroups of a full-occupancy batched launch for K columns per lane (the grid
 // of a bucket is min(this, ceil(pairs / kPairsPerWave))).
 int batched_grid_cap(const Exec& ex, int K, int alpha);
-// Kernel of a batched bucket: the f16 kernel when its score bound allows, else
-// the int16 one.
-int batched_kind(const Bucket& bk, int32_t max_sub, bool allow_f16);
+// Whether a scoring runs the sweep kernels (gbsw_sweep.hpp), and how: the profile
+// form, the offset of all cell values, and the score from which a pair may have
+// left the 16-bit range.  bytes: the scores may be held as bytes.
+struct SweepChoice {
+    bool ok = false;
+    int form = 0; // ProfileForm
+    int32_t base = 0, sat_limit = 0;
+};
+SweepChoice sweep_choice(const std::vector<int16_t>& sub, int alpha, int32_t gap_open, int32_t gap_extend,
+                         int32_t max_sub, bool bytes);
 // Scratch bytes of the radix sort for n pairs.
 int sort_scratch_bytes(int64_t n, size_t* bytes);
 

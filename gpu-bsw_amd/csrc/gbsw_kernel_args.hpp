@@ -106,7 +106,8 @@ struct KernelArgs {
     int32_t sat_limit;         // scores >= this may have saturated int16
     int32_t asym;              // 1: sub[] is not symmetric (the reverse pass then finds its own maximum
                                //    when its orientation differs from the forward pass's)
-    SplitArgs split;           // k_split only
+    int32_t base;              // sweep kernels: offset of all cell values (gbsw_sweep.hpp)
+    SplitArgs split;           // split forms only
 };
 
 // Dynamic LDS layout of one 64-lane workgroup; W = profile columns per row
@@ -169,6 +170,44 @@ __host__ __device__ inline LdsLayout lds_layout(int32_t row_bytes, int32_t alpha
     L.ring_bnd_off = L.ring_code_off + kRingCodes * 2;
     L.group_bytes = align_up(L.ring_bnd_off + kRingBnd * bnd_bytes, 128);
     L.total = L.group_off + kPairsPerWave * L.group_bytes;
+    return L;
+}
+
+// Dynamic LDS layout of a workgroup (one wave) of the sweep kernels.  G lanes
+// align one pair: 2G virtual lanes of K columns, 64/G pairs per wave.
+constexpr int kRegAlpha = 4;   // residue codes a register table holds
+constexpr int kSweepUnroll = 4; // steps per iteration, and the look-ahead of the ring reads
+constexpr int kRebase = 128;   // steps between two subtractions of the running offset
+// Where a sweep kernel keeps the substitution scores: byte tables in registers,
+// a byte profile or a 16-bit profile in LDS.
+enum ProfileForm { kProfRegs = 0, kProfBytes = 1, kProfWords = 2 };
+
+// Ring entries: the 2G - 1 rows before a chunk's first step, the chunk, the next
+// one, and the rows of an outgoing boundary that wait for their flush.
+__host__ __device__ constexpr int32_t sweep_ring(int32_t G) { return G == 16 ? 128 : 256; }
+__host__ __device__ constexpr int32_t sweep_row_bytes(int32_t G, int32_t K, int form)
+{
+    return form == kProfRegs ? 0 : form == kProfBytes ? 2 * G * kstride8(K) : 4 * G * kstride(K);
+}
+struct SweepLds {
+    int32_t lut_off, sub_off, colmax_off, row_tab_off, col_tab_off, group_off, group_bytes;
+    int32_t prof_bytes, ring_code_off, ring_bnd_off, total;
+};
+__host__ __device__ inline SweepLds sweep_lds(int32_t G, int32_t K, int form, int32_t alpha, int32_t bnd_bytes)
+{
+    SweepLds L;
+    L.lut_off = 0;                                              // 256 B
+    L.sub_off = 256;                                            // alpha^2 int16
+    L.colmax_off = L.sub_off + align_up(2 * alpha * alpha, 16); // 32 int16
+    L.row_tab_off = L.colmax_off + 2 * 32;                      // 257 uint16
+    L.col_tab_off = align_up(L.row_tab_off + 2 * 257, 4);       // 257 dwords (register form)
+    L.group_off = align_up(L.col_tab_off + (form == kProfRegs ? 4 * 257 : 0), 128);
+    L.prof_bytes = align_up((alpha + 1) * sweep_row_bytes(G, K, form), 128);
+    L.ring_code_off = L.prof_bytes;
+    // every code entry twice; the register form's entries are dwords (two rows)
+    L.ring_bnd_off = L.ring_code_off + 2 * sweep_ring(G) * (form == kProfRegs ? 4 : 2);
+    L.group_bytes = align_up(L.ring_bnd_off + (sweep_ring(G) + kSweepUnroll) * bnd_bytes, 128);
+    L.total = L.group_off + (kWave / G) * L.group_bytes;
     return L;
 }
 

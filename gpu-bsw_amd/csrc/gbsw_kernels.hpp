@@ -11,16 +11,29 @@ enum KernelKind {
     kPlainReverse = 1,
     kBatched = 2,
     kBatchedWide = 3,
-    kBatchedF16 = 4,
+    kBatchedF16 = 4, // k_sweep: 16-bit cells, f16 maxima
     kSplit = 5,    // k_split, int16 cells
-    kSplitF16 = 6, // k_split, f16 cells
+    kSplitF16 = 6, // k_sweep_split
 };
-// Flag on a kind: the instantiation with an int8 profile (no f16 form).
+// Flag on a kind: the scores are held as bytes (profile or register tables).
 constexpr int kByteProfile = 0x100;
 inline int with_profile(int kind, bool bytes8) { return bytes8 ? (kind | kByteProfile) : kind; }
 
-// largest score + one substitution an f16 kernel may meet (exact integers in f16)
-constexpr int kF16Exact = 2048;
+// The sweep kernels (gbsw_sweep.hpp) are kBatchedF16 and kSplitF16 with these
+// flags.  kRegTables: the scores of a lane's columns in registers (at most
+// kRegAlpha residue codes) instead of a profile in LDS.  kWideGroup: one pair per
+// wave (64 lanes) instead of four (16 lanes each).
+constexpr int kWideGroup = 0x200;
+constexpr int kRegTables = 0x400;
+constexpr int kReportedKind = 0x1FF; // the part of a kind that launch statistics report
+inline int sweep_kind(int kind, int form)
+{
+    return form == kProfRegs ? kind | kByteProfile | kRegTables : form == kProfBytes ? kind | kByteProfile : kind;
+}
+// kernel of a form, nullptr where it is not compiled (gbsw_sweep_*.hip)
+const void* sweep_kernel_regs(bool split, bool wide, int K);
+const void* sweep_kernel_bytes(bool split, bool wide, int K);
+const void* sweep_kernel_words(bool split, bool wide, int K);
 
 bool kernel_supported(int K);
 bool kernel_has(int kind, int K);

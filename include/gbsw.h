@@ -80,8 +80,8 @@ int gbsw_context_destroy(gbsw_context* ctx);
  * STREAMS: streams the length buckets of the batched form run on, 1..8 (default
  *          4, or the GBSW_STREAMS environment variable); 1 serialises them, so
  *          every launch is timed alone.
- * F16:     1 (default; GBSW_F16=0 turns it off): length buckets whose scores
- *          provably stay below 2048 run an exact integer-valued f16 kernel;
+ * F16:     1 (default; GBSW_F16=0 turns it off): length buckets run the kernels
+ *          whose maxima are three-operand f16 instructions on integers (exact);
  *          0: every bucket runs the int16 kernel.  Results are identical. */
 #define GBSW_OPT_STREAMS 1
 #define GBSW_OPT_F16 2

@@ -1,0 +1,118 @@
+"""The sweep kernels (batched form) against the oracle at the sizes where they can
+go wrong: column counts around a lane block, a strip and a wave; row counts around
+a chunk, the period of the running offset and a group's fill; every profile form;
+and scores around the top of the 16-bit range.  Bit-exact on all five outputs;
+the int16 kernels (option F16 off) must agree on the same pairs."""
+import random
+
+import numpy as np
+import pytest
+
+import oracle_lib as ol
+import gbsw
+from gbsw.scoring import AA_ORDER, BLOSUM62
+
+pytestmark = pytest.mark.gpu
+FIELDS = gbsw.FIELDS
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = gbsw.Context(0)
+    yield c
+    c.close()
+
+
+def mutate(rng, s, letters):
+    out = []
+    for c in s:
+        u = rng.random()
+        if u < 0.08:
+            out.append(rng.choice(letters))
+        elif u < 0.10:
+            continue
+        elif u < 0.12:
+            out.append(c + rng.choice(letters))
+        else:
+            out.append(c)
+    return "".join(out)
+
+
+def edge_pairs(seed, letters, cols, rows):
+    rng = random.Random(seed)
+    refs, qrys = [], []
+    for c in cols:
+        for r in rows:
+            long, short = max(c, r), min(c, r)
+            a = "".join(rng.choice(letters) for _ in range(long))
+            at = rng.randint(0, long - short)
+            b = mutate(rng, a[at:at + short], letters) if rng.random() < 0.7 else \
+                "".join(rng.choice(letters) for _ in range(short))
+            b = (b + "".join(rng.choice(letters) for _ in range(short)))[:short]
+            refs.append(a)
+            qrys.append(b)
+            if rng.random() < 0.3:
+                refs[-1], qrys[-1] = qrys[-1], refs[-1]
+    return refs, qrys
+
+
+def check(ctx, refs, qrys, oracle_sc, sc, label):
+    rb, ro = gbsw.pack(refs)
+    qb, qo = gbsw.pack(qrys)
+    exp = ol.align_batch(rb, ro, qb, qo, oracle_sc)
+    try:
+        for f16, split in ((1, 1), (1, 0), (0, 0)):
+            print("case", label, "f16", f16, "split", split, flush=True)
+            ctx.set_option(gbsw.OPT_F16, f16)
+            ctx.set_option(gbsw.OPT_SPLIT, split)
+            got = ctx.align_packed(rb, ro, qb, qo, sc, "batched")
+            for f in FIELDS:
+                bad = np.nonzero(got[f] != exp[f])[0]
+                assert len(bad) == 0, (label, f16, split, f, len(bad), int(bad[0]), len(refs[bad[0]]),
+                                       len(qrys[bad[0]]), {g: (int(got[g][bad[0]]), int(exp[g][bad[0]])) for g in FIELDS})
+    finally:
+        ctx.set_option(gbsw.OPT_F16, 1)
+        ctx.set_option(gbsw.OPT_SPLIT, 1)
+    return exp
+
+
+COLS = (1, 2, 31, 32, 33, 63, 64, 65, 127, 128, 129, 159, 160, 161, 255, 256, 257, 383, 385, 511, 512, 513, 1025)
+ROWS = (1, 16, 32, 97, 128, 129, 161, 225, 256, 257, 289, 600, 1200)
+DNA_FORMS = [("ACGT", (3, -3, -6, -1)),       # register tables
+             ("ACG", (1, -4, -6, 0)),         # no extension cost: no running offset
+             ("ACGT", (4, -4, -40, -24)),     # a large one
+             ("ACGTN", (3, -3, -6, -1)),      # byte profile
+             ("ACGTNRYKMSWB", (2, -3, -5, -2)),
+             ("ACGT", (9, -11, -13, -2)),     # 16-bit profile
+             ("ACGT", (2, -200, -6, -1)),     # 16-bit, negative after the bias
+             ("ACGT", (3, -3, -1, -4)),       # extending costs more than opening
+             ("ACGT", (3, -3, -600, -600))]   # outside the sweep kernels' range
+
+
+@pytest.mark.parametrize("form", range(len(DNA_FORMS)))
+def test_dna_tile_edges(ctx, form):
+    letters, scoring = DNA_FORMS[form]
+    refs, qrys = edge_pairs(900 + form, letters, COLS, ROWS)
+    check(ctx, refs, qrys, ol.dna_scoring(*scoring), gbsw.dna_scoring(*scoring), "dna %s %s" % (letters, scoring))
+
+
+@pytest.mark.parametrize("gaps", [(-6, -1), (-11, -1), (-1, -1), (0, 0)])
+def test_protein_tile_edges(ctx, gaps):
+    refs, qrys = edge_pairs(950 - gaps[0], AA_ORDER[:20], COLS, ROWS)
+    check(ctx, refs, qrys, ol.aa_scoring(BLOSUM62, *gaps), gbsw.protein_scoring(BLOSUM62, *gaps), "protein %s" % (gaps,))
+
+
+@pytest.mark.parametrize("letters", ["ACGT", "ACGTN"])
+def test_scores_around_the_16_bit_range(ctx, letters):
+    """Identical stretches of 96 per residue: scores from 30,000 to 34,000 cross the
+    limit from which a pair is recomputed with int32 cells, beside ordinary pairs."""
+    rng = random.Random(77)
+    refs, qrys = [], []
+    for n in list(range(312, 356)) + [900, 1500]:
+        core = "".join(rng.choice(letters) for _ in range(n))
+        refs.append("".join(rng.choice(letters) for _ in range(rng.randint(0, 200))) + core)
+        qrys.append(core)
+        refs.append("".join(rng.choice(letters) for _ in range(400)))
+        qrys.append(refs[-1][100:100 + rng.randint(1, 120)])
+    exp = check(ctx, refs, qrys, ol.dna_scoring(96, -96, -192, -64), gbsw.dna_scoring(96, -96, -192, -64), letters)
+    assert exp["score"].max() > 100_000 and ((exp["score"] > 30_000) & (exp["score"] < 33_000)).sum() > 10
