@@ -47,7 +47,7 @@ struct gbsw_batch {
     gbsw_context* ctx = nullptr;
     Job job;
     DeviceBuffer ref, ref_off, qry, qry_off, out, order;
-    DeviceBuffer bucket_of_len, keys, keys_sorted, vals, sort_temp;
+    DeviceBuffer keys, keys_sorted, vals, sort_temp;
     std::vector<int32_t> len_ref, len_qry;
     uint8_t lut[256];
     uint8_t code_of[24]; // protein: reference code of each residue code present
@@ -197,7 +197,6 @@ static int batch_fill(gbsw_batch* b, gbsw_context* ctx, Exec& ex, int32_t alphab
     if (e == hipSuccess) e = b->vals.reserve(4 * np);
     if (e == hipSuccess) e = b->order.reserve(4 * np);
     if (e == hipSuccess) e = b->sort_temp.reserve(sort_bytes);
-    if (e == hipSuccess) e = b->bucket_of_len.reserve(65536);
     if (e == hipSuccess && ref_bytes) e = hipMemcpy(b->ref.ptr, rp, ref_bytes, hipMemcpyHostToDevice);
     if (e == hipSuccess && qry_bytes) e = hipMemcpy(b->qry.ptr, qp, qry_bytes, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(b->ref_off.ptr, ro.data(), sizeof(uint64_t) * (size_t)(n + 1), hipMemcpyHostToDevice);
@@ -226,14 +225,11 @@ static int batch_fill(gbsw_batch* b, gbsw_context* ctx, Exec& ex, int32_t alphab
         job.code_of = alphabet == GBSW_PROTEIN ? b->code_of : nullptr;
     }
     count_buckets(job, b->len_ref.data(), b->len_qry.data());
-    e = hipMemcpy(b->bucket_of_len.ptr, bucket_table(job.alpha, job.kmodel).data(), 65536, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return fail(GBSW_E_DEVICE, std::string("batch upload: ") + hipGetErrorString(e));
     job.ref = b->ref.as<uint8_t>();
     job.qry = b->qry.as<uint8_t>();
     job.ref_off = b->ref_off.as<uint64_t>();
     job.qry_off = b->qry_off.as<uint64_t>();
     job.out = b->out.as<int32_t>();
-    job.bucket_of_len = b->bucket_of_len.as<uint8_t>();
     job.keys = b->keys.as<uint32_t>();
     job.keys_sorted = b->keys_sorted.as<uint32_t>();
     job.vals = b->vals.as<int32_t>();
@@ -301,7 +297,6 @@ int noalloc_carve(gbsw_context* ctx, int64_t n, uint64_t ref_bytes, uint64_t qry
     take(x.sub, sizeof(int16_t) * 1024);
     take(x.lut, 256);
     take(x.colmax, sizeof(int16_t) * 32);
-    take(b->bucket_of_len, 65536);
     take(b->ref, std::max<uint64_t>(ref_bytes, 16));
     take(b->qry, std::max<uint64_t>(qry_bytes, 16));
     take(b->ref_off, sizeof(uint64_t) * (np + 1));
@@ -708,29 +703,18 @@ int gbsw_batch_autotune(gbsw_batch* b, const gbsw_scoring* sc, int32_t repeats, 
     gbsw_context* ctx = b->ctx;
     GBSW_HIP_TRY(hipSetDevice(ctx->device));
     Job& job = b->job;
-    auto use_model = [&](int m) -> int {
-        GBSW_HIP_TRY(hipMemcpy(b->bucket_of_len.ptr, bucket_table(job.alpha, m).data(), 65536, hipMemcpyHostToDevice));
-        job.kmodel = m;
-        count_buckets(job, b->len_ref.data(), b->len_qry.data());
-        b->graph.reset(); // its launches hold the previous map's bucket slices
-        return GBSW_OK;
-    };
+    // (the plan of the next align follows the model)
+    auto use_model = [&](int m) { job.kmodel = m; };
     // the batch's current model first; another one must beat it by more than
     // kTuneMargin (run-to-run noise of a batch is about 1 %)
     constexpr double kTuneMargin = 0.015;
     const int current = job.kmodel;
     int best = -1;
     double best_ms = 1e300;
-    std::vector<const std::vector<uint8_t>*> tried;
     for (int i = 0; i < kGeometryModels; ++i) {
         const int m = i == 0 ? current : (i <= current ? i - 1 : i);
-        // models whose length -> geometry map is one already timed add nothing
-        const std::vector<uint8_t>* t = &bucket_table(job.alpha, m);
-        bool seen = false;
-        for (const auto* u : tried) seen = seen || *u == *t;
-        if (seen) continue;
-        tried.push_back(t);
-        int rc = use_model(m);
+        use_model(m);
+        int rc = GBSW_OK;
         double m_ms = 1e300;
         for (int r = 0; !rc && r < repeats + 1; ++r) {
             rc = gbsw_batch_align(b, sc, GBSW_BATCHED);
@@ -739,8 +723,7 @@ int gbsw_batch_autotune(gbsw_batch* b, const gbsw_scoring* sc, int32_t repeats, 
         if (rc) return rc;
         if (best < 0 || m_ms < best_ms * (1.0 - kTuneMargin)) { best_ms = m_ms; best = m; }
     }
-    int rc = use_model(best);
-    if (rc) return rc;
+    use_model(best);
     ctx->ex.kmodel = best; // batches created afterwards start from it
     if (model) *model = best;
     if (ms) *ms = best_ms;

@@ -106,9 +106,9 @@ int lds_for(int K, int alpha, bool p8, int bnd_bytes = 4)
     return lds_layout(prof_row_bytes(K, p8), alpha, bnd_bytes).total;
 }
 
-int sweep_lds_for(int K, int alpha, int form)
+int sweep_lds_for(int K, int alpha, int form, int G)
 {
-    return sweep_lds(kLanesPerPair, K, form, alpha, 4).total;
+    return sweep_lds(G, K, form, alpha, 4).total;
 }
 
 int grid_for(const Exec& ex, int kind, int K, int lds, int64_t nquads)
@@ -265,34 +265,19 @@ double occupancy_threshold(int model)
     return (model > 0 && model < kGeometryModels) ? thr[model] : 0.0;
 }
 
-// Share of the VALU issue rate a geometry reaches at its occupancy: the large
-// DNA buckets issue 0.96 VALU instructions per CU per cycle at 4 waves per SIMD,
-// 0.82 at 2.75, 0.78 at 2 and 0.62 at 1.5 (rocprofv3 counters), so
-// min(1, waves per SIMD / threshold), threshold 2.5 by default.
-double occupancy_factor(int K, int alpha, double threshold)
+// Share of the VALU issue rate `waves` per SIMD reach: the int16 kernels' large
+// buckets issue 0.96 VALU instructions per CU per cycle at 4 waves per SIMD, 0.82
+// at 2.75, 0.78 at 2 and 0.62 at 1.5 (rocprofv3 counters), so min(1, waves /
+// threshold), threshold 2.5 by default.
+double issue_share(double waves, double threshold)
 {
-    static std::mutex mu;
-    static std::map<int, int> cache; // workgroups per CU (the usual kernel of the alphabet)
-    int wg_per_cu = 0;
-    {
-        std::lock_guard<std::mutex> lk(mu);
-        const int key = K * 64 + alpha;
-        auto it = cache.find(key);
-        if (it != cache.end()) {
-            wg_per_cu = it->second;
-        } else {
-            // one wave each
-            const int form = alpha <= kRegAlpha ? kProfRegs : kProfBytes;
-            wg_per_cu = kernel_occupancy(sweep_kind(kBatchedF16, form), K, sweep_lds_for(K, alpha, form));
-            cache.emplace(key, wg_per_cu);
-        }
-    }
-    return (wg_per_cu > 0 && threshold > 0) ? std::min(1.0, wg_per_cu / 4.0 / threshold) : 1.0;
+    return (waves > 0 && threshold > 0) ? std::min(1.0, waves / threshold) : 1.0;
 }
 
-int k_for_cols(int cols, int alpha, int model, int klimit)
+int k_for_cols(int cols, int alpha, int model)
 {
-    const int kmax = std::min(klimit, max_k_for(alpha, byte_profile_alphabet(alpha)));
+    const bool p8 = byte_profile_alphabet(alpha);
+    const int kmax = max_k_for(alpha, p8);
     int nk = 0;
     const int* ks = kernel_k_list(&nk);
     int best = ks[0];
@@ -303,99 +288,43 @@ int k_for_cols(int cols, int alpha, int model, int klimit)
         const int64_t strips = std::max<int64_t>(1, (cols + kVirtPerPair * K - 1) / (kVirtPerPair * K));
         // padded columns and the per-step cost, per strip
         double cost = (double)(strips * (K + 2) * 4 + (strips - 1));
-        if (model != kModelClassic) cost /= occupancy_factor(K, alpha, occupancy_threshold(model));
+        if (model != kModelClassic) // (one wave per workgroup)
+            cost /= issue_share(kernel_occupancy(with_profile(kBatched, p8), K, lds_for(K, alpha, p8)) / 4.0,
+                                occupancy_threshold(model));
         if (cost < best_cost) { best_cost = cost; best = K; }
     }
     return best;
 }
 
-int bucket_ids()
-{
-    int nk = 0;
-    kernel_k_list(&nk);
-    return 3 * nk;
-}
-
-StripWidths strip_widths()
-{
-    StripWidths sw;
-    std::memset(&sw, 0, sizeof(sw));
-    int nk = 0;
-    const int* ks = kernel_k_list(&nk);
-    for (int b = 0; b < std::min(64, bucket_ids()); ++b) sw.w[b] = (uint16_t)(kVirtPerPair * ks[b % nk]);
-    return sw;
-}
-
-const std::vector<uint8_t>& bucket_table(int alpha, int model)
-{
-    static std::mutex mu;
-    static std::map<int, std::vector<uint8_t>> cache;
-    std::lock_guard<std::mutex> lk(mu);
-    const int key = alpha * 64 + model;
-    auto it = cache.find(key);
-    if (it != cache.end()) return it->second;
-    int nk = 0;
-    const int* ks = kernel_k_list(&nk);
-    // strip counts, hence the choice, only change at multiples of 32 columns:
-    // the lengths (32(j-1), 32j] share the choice made for 32j
-    std::vector<int> kblk(65536 / 32 + 1);
-    for (size_t j = 0; j < kblk.size(); ++j) kblk[j] = k_for_cols((int)(32 * j), alpha, model, kSweepMaxK);
-    std::vector<uint8_t> t(65536);
-    for (int m = 0; m < 65536; ++m) {
-        const int K = kblk[(size_t)((m + 31) / 32)];
-        int idx = 0;
-        while (idx < nk && ks[idx] != K) ++idx;
-        // pairs spanning several strips get buckets of their own, so a single-strip
-        // bucket hands no boundary rows on; those up to kMultiShortCols columns apart
-        // from longer ones
-        const bool multi = m > kVirtPerPair * K;
-        const int cls = !multi ? 0 : m <= kMultiShortCols ? 1 : 2;
-        t[(size_t)m] = (uint8_t)(idx + cls * nk);
-    }
-    return cache.emplace(key, std::move(t)).first->second;
-}
-
 void count_buckets(Job& job, const int32_t* len_ref, const int32_t* len_qry)
 {
-    const std::vector<uint8_t>& tab = bucket_table(job.alpha, job.kmodel);
-    int nk = 0;
-    const int* ks = kernel_k_list(&nk);
-    const int nb = bucket_ids();
-    std::vector<int64_t> count((size_t)nb, 0), cells((size_t)nb, 0);
-    std::vector<int32_t> mcols((size_t)nb, 0);
+    Bucket sum[kClasses];
     for (int64_t p = 0; p < job.n; ++p) {
         const int32_t la = len_ref[p], lb = len_qry[p];
-        const int32_t m = std::min(la, lb);
-        const int bi = tab[(size_t)std::min<int32_t>(m, 65535)];
-        count[(size_t)bi] += 1;
-        cells[(size_t)bi] += (int64_t)la * lb;
-        mcols[(size_t)bi] = std::max(mcols[(size_t)bi], m);
+        sum[length_class(std::min(la, lb))].add(std::min(la, lb), std::max(la, lb));
     }
+    place_buckets(job, sum);
+}
+
+void place_buckets(Job& job, const Bucket* by_class)
+{
     job.buckets.clear();
     int64_t at = 0;
-    for (int i = 0; i < nb; ++i) {
-        if (count[(size_t)i] == 0) continue;
-        Bucket bk;
-        bk.K = ks[i % nk];
-        bk.begin = at;
-        bk.count = count[(size_t)i];
-        bk.cells = cells[(size_t)i];
-        bk.max_cols = mcols[(size_t)i];
-        at += bk.count;
-        job.buckets.push_back(bk);
+    for (int c = kClasses - 1; c >= 0; --c) { // the sort order: longest class first
+        if (by_class[c].count == 0) continue;
+        job.buckets.push_back(by_class[c]);
+        job.buckets.back().begin = at;
+        at += by_class[c].count;
     }
 }
 
-int batched_grid_cap(const Exec& ex, int K, int alpha)
+int wide_grid_cap(const Exec& ex, int alpha)
 {
-    // the largest occupancy of the geometry's kernels and profile layouts, so
-    // that a launch's grid (hence its boundary rows) never exceeds what
-    // admission reserved for it
-    const bool p8 = byte_profile_alphabet(alpha);
-    int occ = kernel_occupancy(with_profile(kBatched, p8), K, lds_for(K, alpha, p8));
+    int occ = 1;
     for (int form = alpha <= kRegAlpha ? kProfRegs : kProfBytes; form <= kProfWords; ++form)
-        occ = std::max(occ, kernel_occupancy(sweep_kind(kBatchedF16, form), K, sweep_lds_for(K, alpha, form)));
-    return std::max(1, occ) * ex.num_cu;
+        occ = std::max(occ, kernel_occupancy(sweep_kind(kBatchedF16, form, kWideGroup), 1,
+                                             sweep_lds_for(1, alpha, form, kWave)));
+    return occ * ex.num_cu;
 }
 
 bool f16_high_byte_exact(int32_t s)
@@ -493,26 +422,18 @@ int prepare_scoring(const Job& job, const gbsw_scoring* sc, std::vector<int16_t>
 
 namespace {
 
-// One length bucket's launch in the batched form.
+// One launch of the batched form: adjacent length classes.
 struct BucketPlan {
-    int kind = 0, K = 0, grid = 0, lds = 0, strips = 1;
+    Bucket bk;
+    int kind = 0, K = 0, grid = 0, lds = 0, strips = 1; // K: the widest geometry of the launch
+    int G = kLanesPerPair; // lanes per pair (64: one pair per wave)
     int32_t sat_limit = 0;
+    std::vector<SetRange> ranges;    // sweep launches: geometries by position within the launch
+    double work = 0, unit = 0;       // estimated cycles: of the whole launch on the full GPU, of its longest item alone
     size_t bnd_at = 0, split_at = 0; // 32-bit word offsets into ex.bnd / ex.split_buf
+    int pairs_per_wave() const { return kWave / G; }
+    int64_t sets() const { return (bk.count + pairs_per_wave() - 1) / pairs_per_wave(); }
 };
-
-// Estimated duration of a bucket (relative): cells x (K + 2) / K (padding and
-// per-step overhead), +40 % for the int16 kernels, and the split form's weight.
-double bucket_cost(const BucketPlan& b, const Bucket& bk)
-{
-    const int k = b.kind & 0xFF;
-    const double f16 = (k == kBatchedF16 || k == kSplitF16) ? 1.0 : 1.4;
-    // a split bucket's strips wait on each other, and beside the bulk buckets it
-    // runs several times longer than alone (the K = 7 split bucket of the 1M-pair
-    // DNA mix: 1.0 ms alone, 6.6 ms beside them); weights 2.5 / 4 / 6 / 8 / 12
-    // measured 3,658-3,672 / 3,703-3,708 / 3,715-3,729 / 3,717-3,726 / 3,713 GCUPS
-    const double split = (k == kSplit || k == kSplitF16) ? 6.0 : 1.0;
-    return (double)bk.cells * (b.K + 2) / b.K * f16 * split;
-}
 
 bool plan_is_split(const BucketPlan& b)
 {
@@ -520,136 +441,310 @@ bool plan_is_split(const BucketPlan& b)
     return k == kSplit || k == kSplitF16;
 }
 
-// 32-bit words of a split bucket's bookkeeping: keys (2 x count u64), progress
-// words (2 slots per workgroup, u64), done counters (2 x quads), release epochs
+// 32-bit words of a split launch's bookkeeping: keys (2 x count u64), progress
+// words (2 slots per workgroup, u64), done counters (2 x sets), release epochs
 // (one per slot), the placement table (kXcds) and the strip gates (count), padded
-// to a multiple of 64 (256 bytes) so that the next bucket's 64-bit keys and
+// to a multiple of 64 (256 bytes) so that the next launch's 64-bit keys and
 // progress words stay 8-byte aligned.
-size_t split_words_of(const Bucket& bk, const BucketPlan& b)
+size_t split_words_of(const BucketPlan& b)
 {
-    const size_t nquads = (size_t)((bk.count + kPairsPerWave - 1) / kPairsPerWave);
-    const size_t words = 5 * (size_t)bk.count + 2 * nquads + 3 * (size_t)(2 * b.grid) + kXcds;
+    const size_t words = 5 * (size_t)b.bk.count + 2 * (size_t)b.sets() + 3 * (size_t)(2 * b.grid) + kXcds;
     return (words + 63) & ~(size_t)63;
 }
 
-// Kernels, grids and scratch of every bucket (host only; reserves the buffers).
-int plan_batched(Exec& ex, const Job& job, int max_sub, bool p8, const SweepChoice& sw, bool asym, int kclamp,
-                 int64_t bnd_rows, std::vector<BucketPlan>& plan, std::vector<size_t>& order)
+// Cycles of one step of a wave with K columns per lane, with other waves on its
+// SIMD and alone (measured: 126 and 194 cycles at K = 1, 193 at K = 5 beside others,
+// 391 / 455 / 602 at K = 5 / 6 / 8 alone); a strip with boundary rows takes more.
+double step_issue(int K, bool ms) { return 25.0 * K + 80 + (ms ? 20 : 0); }
+double step_alone(int K, bool ms) { return 58.0 * K + 135 + (ms ? 55 : 0); }
+// Forward plus reverse pass, in forward passes.
+constexpr double kPasses = 1.6;
+// A strip of the split form starts once its predecessor has published the rows of
+// its first three chunks, which leave the predecessor's last virtual lane 2G steps
+// after they enter it.
+int split_lag(int G) { return 2 * G + 3 * kChunk; }
+// Geometries of the sweep kernels, ascending.
+#define GBSW_ITEM(k) k,
+constexpr int kSweepK16[] = {GBSW_SWEEP_K16(GBSW_ITEM) GBSW_SWEEP_K16_WIDE(GBSW_ITEM)};
+constexpr int kSweepK64[] = {GBSW_SWEEP_K64(GBSW_ITEM)};
+constexpr int kSweepSplitK[] = {GBSW_SWEEP_K64_SPLIT(GBSW_ITEM)};
+#undef GBSW_ITEM
+constexpr int kSweepNarrowMax = 8; // widest geometry of the narrow four-pair kernel
+
+// Estimates of one class in one geometry: work (wave cycles over all SIMDs) and
+// the longest item's time.
+struct GeoCost {
+    double work = 1e300, unit = 1e300;
+    int K = 0, strips = 1;
+};
+GeoCost geo_cost(const Exec& ex, const Bucket& bk, int G, int K, bool split)
 {
-    const size_t nb = job.buckets.size();
-    plan.assign(nb, BucketPlan{});
-    order.resize(nb);
-    // the unsplit kernel of a bucket: the sweep kernel of the job's profile form in
-    // the widest geometry that fits its LDS, else (scorings outside the sweep
-    // kernels' range, option F16 off) the int16 kernel
-    int nk = 0;
-    const int* ks = kernel_k_list(&nk);
-    auto unsplit = [&](BucketPlan& b, const Bucket& bk) {
-        b.K = std::min(kclamp, bk.K);
-        if (sw.ok) {
-            int i = 0;
-            while (i + 1 < nk && ks[i + 1] <= bk.K) ++i;
-            while (i > 0 && sweep_lds_for(ks[i], job.alpha, sw.form) > 65536) --i;
-            b.K = ks[i];
-            b.kind = sweep_kind(kBatchedF16, sw.form);
-            b.lds = sweep_lds_for(b.K, job.alpha, sw.form);
-            b.sat_limit = sw.sat_limit;
-        } else {
-            b.kind = with_profile(kBatched, p8);
-            b.lds = lds_for(b.K, job.alpha, p8);
-            b.sat_limit = 32767 - max_sub;
+    const int vl = 2 * G;
+    GeoCost c;
+    c.K = K;
+    c.strips = std::max(1, (bk.max_cols + vl * K - 1) / (vl * K));
+    const double n = (double)std::max<int64_t>(1, bk.count);
+    const double strips = c.strips == 1 ? 1.0 : std::max(1.0, (double)bk.cols / n / (vl * K) + 0.5);
+    const double steps = (double)bk.rows / n + vl - 1, longest = bk.max_rows + vl - 1;
+    c.work = n * G / kWave * strips * steps * step_issue(K, c.strips > 1) * kPasses * (split ? 1.4 : 1.0) /
+             (4.0 * ex.num_cu);
+    c.unit = (split ? longest + (c.strips - 1) * (double)split_lag(G) : c.strips * longest) *
+             step_alone(K, c.strips > 1) * kPasses;
+    return c;
+}
+
+// The launches of a job whose scoring runs the sweep kernels.
+//
+// Which geometry a class takes.  Four pairs per wave issue the fewest instructions
+// per cell; one pair per wave finishes a pair about four times sooner and takes any
+// number of strips; its strips on several waves (the split form) finish it sooner
+// still.  The sort order puts long classes first, so the forms are three adjacent
+// stretches of it (split, one pair per wave, four pairs per wave: wide, then narrow
+// geometries), one launch each.  A job lasts at least as long as its instructions
+// take on the whole GPU and as its longest item takes alone; the stretches are
+// those of least max + kOverlap x min of the two.
+void plan_sweeps(const Exec& ex, const Job& job, const SweepChoice& sw, bool may_split, std::vector<BucketPlan>& plan)
+{
+    constexpr double kOverlap = 0.35;
+    const std::vector<Bucket>& cls = job.buckets;
+    const size_t n = cls.size();
+    const double thr = occupancy_threshold(job.kmodel);
+    auto lds = [&](int G, int K) { return sweep_lds_for(K, job.alpha, sw.form, G); };
+    // share of the issue rate of a launch whose widest geometry is K
+    auto share = [&](int flags, int G, int K) {
+        const int l = lds(G, K);
+        if (l > 65536) return 0.0;
+        return issue_share(kernel_occupancy(sweep_kind(kBatchedF16, sw.form, flags), K, l) / 4.0, thr);
+    };
+    struct Option {
+        std::vector<GeoCost> cost; // per class
+        std::vector<double> work, unit; // sums / maxima over [0, i) (or [i, n) for four pairs per wave)
+        int cap = 0;
+    };
+    auto prefix = [&](Option& o) {
+        o.work.assign(n + 1, 0.0);
+        o.unit.assign(n + 1, 0.0);
+        for (size_t i = 0; i < n; ++i) {
+            o.work[i + 1] = o.work[i] + o.cost[i].work;
+            o.unit[i + 1] = std::max(o.unit[i], o.cost[i].unit);
         }
     };
-    for (size_t i = 0; i < nb; ++i) {
-        order[i] = i;
-        const Bucket& bk = job.buckets[i];
-        BucketPlan& b = plan[i];
-        unsplit(b, bk);
-        const int64_t nquads = (bk.count + kPairsPerWave - 1) / kPairsPerWave;
-        b.strips = std::max(1, (bk.max_cols + kVirtPerPair * b.K - 1) / (kVirtPerPair * b.K));
-        const int skind = sw.ok ? sweep_kind(kSplitF16, sw.form) : with_profile(kSplit, p8);
-        // A split item waits about four chunks for its predecessor's first
-        // rows: worth it only when the bucket has too few quads to keep every
-        // workgroup busy for two rounds (on the 200k-pair DNA mix: 1765 vs 827
-        // GCUPS at 1.4 quads per workgroup; 988 vs 1275 on protein at 2.7).
-        const int64_t full = (int64_t)std::max(1, kernel_occupancy(b.kind, b.K, b.lds)) * ex.num_cu;
-        // (an asymmetric table may need a third pass per pair, which the split
-        // form's strip items do not schedule)
-        if (ex.split && !ex.split_misplaced && !asym && b.strips > 1 && nquads < 2 * full && kernel_has(skind, b.K)) {
-            // every XCD's counter needs workgroups: a multiple of kXcds, no more
-            // than the items a pipelined quad can keep busy, and two boundary
-            // slots per workgroup
-            b.kind = skind;
-            const int occ = std::max(1, kernel_occupancy(skind, b.K, b.lds));
-            const int64_t busy = (nquads * b.strips + kXcds - 1) / kXcds * kXcds;
-            b.grid = (int)std::max<int64_t>(kXcds, std::min<int64_t>(occ * ex.num_cu / kXcds * kXcds, busy));
-        } else {
-            b.grid = grid_for(ex, b.kind, b.K, b.lds, nquads);
+    // four pairs per wave: the widest geometry (its LDS decides the launch's
+    // occupancy) is that of the first class
+    Option four;
+    size_t first = n; // classes before it have no such geometry
+    four.cost.resize(n);
+    four.work.assign(n + 1, 0.0);
+    four.unit.assign(n + 1, 0.0);
+    for (size_t i = n; i-- > 0;) {
+        int K = 0;
+        for (int k : kSweepK16)
+            if (cls[i].max_cols <= kVirtPerPair * k) { K = k; break; }
+        const double s = K ? share(K > kSweepNarrowMax ? kWideLanes : 0, kLanesPerPair, K) : 0.0;
+        if (s <= 0) break;
+        first = i;
+        four.cost[i] = geo_cost(ex, cls[i], kLanesPerPair, K, false);
+        four.work[i] = four.work[i + 1] + four.cost[i].work / s;
+        four.unit[i] = std::max(four.unit[i + 1], four.cost[i].unit);
+    }
+    // one pair per wave: per widest geometry, the strips of least work or of the
+    // shortest item; split: one geometry per launch
+    std::vector<Option> one, split;
+    for (int cap : kSweepK64) {
+        const double s = share(kWideGroup, kWave, cap);
+        if (s <= 0) break;
+        for (int quick = 0; quick < 2; ++quick) {
+            Option o;
+            o.cap = cap;
+            for (const Bucket& bk : cls) {
+                GeoCost best;
+                for (int K : kSweepK64) {
+                    if (K > cap) break;
+                    const GeoCost c = geo_cost(ex, bk, kWave, K, false);
+                    if (quick ? c.unit < best.unit : c.work < best.work) best = c;
+                }
+                best.work /= s;
+                o.cost.push_back(best);
+            }
+            prefix(o);
+            one.push_back(std::move(o));
         }
     }
+    if (may_split)
+        for (int K : kSweepSplitK) {
+            if (lds(kWave, K) > 65536) break;
+            const int kind = sweep_kind(kSplitF16, sw.form, kWideGroup);
+            const double s = issue_share(kernel_occupancy(kind, K, lds(kWave, K)) / 4.0, thr);
+            Option o;
+            o.cap = K;
+            for (const Bucket& bk : cls) {
+                o.cost.push_back(geo_cost(ex, bk, kWave, K, true));
+                o.cost.back().work /= s;
+            }
+            prefix(o);
+            split.push_back(std::move(o));
+        }
+    double best = 1e300;
+    size_t i64 = 0, i16 = n, which_one = 0, which_split = 0;
+    // launches beyond the first cost little beside a large job and show in a small one
+    constexpr double kLaunch = 12000;
+    for (size_t o = 0; o < one.size(); ++o)
+        for (size_t b = first; b <= n; ++b) { // [b, n) four pairs per wave
+            std::vector<double> unit_tail(b + 1, 0.0); // longest one-pair item of [i, b)
+            for (size_t i = b; i-- > 0;) unit_tail[i] = std::max(unit_tail[i + 1], one[o].cost[i].unit);
+            const double w4 = four.work[b], u4 = four.unit[b];
+            auto consider = [&](size_t a, size_t s) { // [0, a) split
+                double w = w4 + one[o].work[b] - one[o].work[a], u = std::max(u4, unit_tail[a]);
+                if (a) {
+                    w += split[s].work[a];
+                    u = std::max(u, split[s].unit[a]);
+                }
+                const double m = std::max(w, u) + kOverlap * std::min(w, u) +
+                                 kLaunch * ((a > 0 ? 1 : 0) + (b > a ? 1 : 0) + (n > b ? 1 : 0));
+                if (m < best) { best = m; i64 = a; i16 = b; which_one = o; which_split = s; }
+            };
+            consider(0, 0);
+            for (size_t s = 0; s < split.size(); ++s)
+                for (size_t a = 1; a <= b; ++a) consider(a, s);
+        }
+
+    auto add = [&](size_t from, size_t to, int G, int flags, const Option& o, bool is_split) {
+        if (from >= to) return;
+        BucketPlan b;
+        b.G = G;
+        b.sat_limit = sw.sat_limit;
+        b.bk.begin = cls[from].begin;
+        for (size_t i = from; i < to; ++i) {
+            const GeoCost& c = o.cost[i];
+            b.bk.add(cls[i]);
+            b.K = std::max(b.K, c.K);
+            b.strips = std::max(b.strips, c.strips);
+            b.work += c.work;
+            b.unit = std::max(b.unit, c.unit);
+            const int32_t end = (int32_t)b.bk.count;
+            if (!b.ranges.empty() && b.ranges.back().K == c.K) b.ranges.back().end = end;
+            else b.ranges.push_back({end, c.K});
+        }
+        b.kind = sweep_kind(is_split ? kSplitF16 : kBatchedF16, sw.form, flags);
+        b.lds = lds(G, b.K);
+        plan.push_back(b);
+    };
+    size_t narrow = i16;
+    while (narrow < n && four.cost[narrow].K > kSweepNarrowMax) ++narrow;
+    if (i64) add(0, i64, kWave, kWideGroup, split[which_split], true);
+    add(i64, i16, kWave, kWideGroup, one[which_one], false);
+    add(i16, narrow, kLanesPerPair, kWideLanes, four, false);
+    add(narrow, n, kLanesPerPair, 0, four, false);
+}
+
+// The launches of a job on the int16 kernels (scorings outside the sweep kernels'
+// range, option F16 off): one per geometry.  A multi-strip launch is split when it
+// has too few quads to keep every workgroup busy for two rounds (on the 200k-pair
+// DNA mix: 1765 vs 827 GCUPS at 1.4 quads per workgroup; 988 vs 1275 on protein at
+// 2.7).
+void plan_int16(const Exec& ex, const Job& job, int max_sub, bool p8, int kclamp, bool may_split,
+                std::vector<BucketPlan>& plan)
+{
+    for (const Bucket& bk : job.buckets) {
+        const int K = std::min(kclamp, k_for_cols(bk.max_cols, job.alpha, job.kmodel));
+        const int strips = std::max(1, (bk.max_cols + kVirtPerPair * K - 1) / (kVirtPerPair * K));
+        if (plan.empty() || plan.back().K != K || (plan.back().strips > 1) != (strips > 1)) {
+            plan.push_back(BucketPlan{});
+            BucketPlan& b = plan.back();
+            b.bk.begin = bk.begin;
+            b.K = K;
+            b.kind = with_profile(kBatched, p8);
+            b.lds = lds_for(K, job.alpha, p8);
+            b.sat_limit = 32767 - max_sub;
+        }
+        BucketPlan& b = plan.back();
+        b.bk.add(bk);
+        b.strips = std::max(b.strips, strips);
+        const GeoCost c = geo_cost(ex, bk, kLanesPerPair, K, false);
+        b.work += 1.4 * c.work;
+        b.unit = std::max(b.unit, 1.4 * c.unit);
+    }
+    for (BucketPlan& b : plan) {
+        const int64_t full = (int64_t)std::max(1, kernel_occupancy(b.kind, b.K, b.lds)) * ex.num_cu;
+        const int skind = with_profile(kSplit, p8);
+        if (may_split && b.strips > 1 && b.sets() < 2 * full && kernel_has(skind, b.K)) b.kind = skind;
+    }
+}
+
+// Kernels, grids and scratch of every launch (host only; reserves the buffers).
+int plan_batched(Exec& ex, const Job& job, int max_sub, bool p8, const SweepChoice& sw, bool asym, int kclamp,
+                 std::vector<BucketPlan>& plan)
+{
+    plan.clear();
+    // (an asymmetric table may need a third pass per pair, which strip items lack)
+    const bool may_split = ex.split && !ex.split_misplaced && !asym;
+    auto set_grid = [&](BucketPlan& b) {
+        if (plan_is_split(b)) {
+            // a multiple of kXcds: every XCD's counter serves every kXcds-th set, with a
+            // workgroup for each of their strips at most, and two boundary slots each
+            const int occ = std::max(1, kernel_occupancy(b.kind, b.K, b.lds));
+            const int64_t busy = (b.sets() + kXcds - 1) / kXcds * b.strips * kXcds;
+            b.grid = (int)std::max<int64_t>(kXcds, std::min<int64_t>((int64_t)occ * ex.num_cu / kXcds * kXcds, busy));
+        } else {
+            b.grid = grid_for(ex, b.kind, b.K, b.lds, b.sets());
+        }
+    };
     // boundary rows and split bookkeeping (keys: 2 x count u64, prog: slots u64,
-    // done: 2 x quads u32, rel: slots u32, xcc, gate: count u32) in 32-bit words
+    // done: 2 x sets u32, rel: slots u32, xcc, gate: count u32) in 32-bit words
     size_t bnd_words = 0, split_words = 0;
     auto sizes = [&]() {
         bnd_words = split_words = 0;
-        for (size_t i = 0; i < nb; ++i) {
-            const Bucket& bk = job.buckets[i];
-            BucketPlan& b = plan[i];
+        for (BucketPlan& b : plan) {
             b.bnd_at = bnd_words;
+            const size_t per_wg = (size_t)b.pairs_per_wave() * (size_t)std::max(1, b.bk.max_rows);
             if (plan_is_split(b)) {
-                bnd_words += (size_t)2 * b.grid * kPairsPerWave * (size_t)bnd_rows;
+                bnd_words += (size_t)2 * b.grid * per_wg;
                 b.split_at = split_words;
-                split_words += split_words_of(bk, b);
+                split_words += split_words_of(b);
             } else if (b.strips > 1) {
-                // (a bucket whose pairs all fit one strip hands no boundary rows on)
-                bnd_words += (size_t)b.grid * kPairsPerWave * (size_t)bnd_rows;
+                // (a launch whose pairs all fit one strip hands no boundary rows on)
+                bnd_words += (size_t)b.grid * per_wg;
             }
         }
     };
-    sizes();
+    auto make = [&](bool split) {
+        plan.clear();
+        if (sw.ok) plan_sweeps(ex, job, sw, split, plan);
+        else plan_int16(ex, job, max_sub, p8, kclamp, split, plan);
+        for (BucketPlan& b : plan) set_grid(b);
+        sizes();
+    };
+    make(may_split);
     if (ex.fixed) {
-        // preallocated buffers (a serving slot): admission reserved the unsplit
-        // boundary rows; split buckets go back to the unsplit form, widest first,
-        // until everything fits
-        while (bnd_words * sizeof(uint32_t) > ex.bnd.bytes || split_words * sizeof(uint32_t) > ex.split_buf.bytes) {
-            size_t w = nb;
-            for (size_t i = 0; i < nb; ++i)
-                if (plan_is_split(plan[i]) && (w == nb || plan[i].grid > plan[w].grid)) w = i;
-            if (w == nb) break;
-            unsplit(plan[w], job.buckets[w]);
-            plan[w].grid = grid_for(ex, plan[w].kind, plan[w].K, plan[w].lds,
-                                    (job.buckets[w].count + kPairsPerWave - 1) / kPairsPerWave);
-            sizes();
-        }
+        // preallocated buffers (a serving slot): without the split form where its
+        // boundary slots and bookkeeping do not fit
+        if (bnd_words * sizeof(uint32_t) > ex.bnd.bytes || split_words * sizeof(uint32_t) > ex.split_buf.bytes) make(false);
         // then the widest multi-strip grids shrink (a persistent grid of any size
         // drains its queue) until the boundary rows fit
         while (bnd_words * sizeof(uint32_t) > ex.bnd.bytes) {
-            size_t w = nb;
-            for (size_t i = 0; i < nb; ++i)
-                if (!plan_is_split(plan[i]) && plan[i].strips > 1 && plan[i].grid > 1 &&
-                    (w == nb || plan[i].grid > plan[w].grid))
-                    w = i;
-            if (w == nb) return fail(GBSW_E_RANGE, "strip boundary rows exceed the preallocated scratch");
-            plan[w].grid = std::max(1, plan[w].grid / 2);
+            BucketPlan* w = nullptr;
+            for (BucketPlan& b : plan)
+                if (!plan_is_split(b) && b.strips > 1 && b.grid > 1 && (!w || b.grid > w->grid)) w = &b;
+            if (!w) return fail(GBSW_E_RANGE, "strip boundary rows exceed the preallocated scratch");
+            w->grid = std::max(1, w->grid / 2);
             sizes();
         }
     }
-    // Buckets run concurrently on the streams, the ones whose single work item
-    // takes longest (largest K) first, so a bucket with few long pairs overlaps
-    // the bulk instead of running alone at the end (ordering by estimated total
-    // instead measured 4 % slower on the 1M-pair DNA mix); record_batched puts
-    // each on the least-loaded stream.
-    std::sort(order.begin(), order.end(), [&](size_t x, size_t y) { return job.buckets[x].K > job.buckets[y].K; });
-    if (ex.queue.bytes < sizeof(uint32_t) * kXcds * std::max<size_t>(nb, 1))
-        GBSW_HIP_TRY(ex.queue.reserve(sizeof(uint32_t) * kXcds * std::max<size_t>(nb, 1)));
+    // Launches run concurrently on the streams, the ones whose single work item
+    // takes longest first, so that few long pairs overlap the bulk instead of running
+    // alone at the end; record_batched puts each on the least-loaded stream.
+    std::sort(plan.begin(), plan.end(), [](const BucketPlan& x, const BucketPlan& y) {
+        return x.unit != y.unit ? x.unit > y.unit : x.bk.begin < y.bk.begin;
+    });
+    const size_t nb = std::max<size_t>(plan.size(), 1);
+    if (ex.queue.bytes < sizeof(uint32_t) * kXcds * nb) GBSW_HIP_TRY(ex.queue.reserve(sizeof(uint32_t) * kXcds * nb));
     if (split_words) GBSW_HIP_TRY(ex.split_buf.reserve(split_words * sizeof(uint32_t)));
     GBSW_HIP_TRY(ex.bnd.reserve(std::max<size_t>(bnd_words, 1) * sizeof(uint32_t)));
     return GBSW_OK;
 }
 
 // Stream work of the batched form (recorded eagerly or into a graph).
-int record_batched(Exec& ex, const Job& job, KernelArgs a, const std::vector<BucketPlan>& plan,
-                   const std::vector<size_t>& order, size_t sub_bytes)
+int record_batched(Exec& ex, const Job& job, KernelArgs a, const std::vector<BucketPlan>& plan, size_t sub_bytes)
 {
     hipStream_t st0 = ex.stream;
     const uint8_t* th = ex.tables_host.as<uint8_t>();
@@ -659,45 +754,46 @@ int record_batched(Exec& ex, const Job& job, KernelArgs a, const std::vector<Buc
                                 st0));
     GBSW_HIP_TRY(zero_u32(ex.status.as<uint32_t>(), kStatusWords, st0));
     // device binning: keys, then a stable radix sort into the work order
-    GBSW_HIP_TRY(bin_keys(job.ref_off, job.qry_off, job.n, job.bucket_of_len, strip_widths(), job.keys, job.vals, st0));
+    GBSW_HIP_TRY(bin_keys(job.ref_off, job.qry_off, job.n, job.keys, job.vals, st0));
     size_t tb = job.sort_temp_bytes;
     GBSW_HIP_TRY(sort_pairs(job.sort_temp, tb, job.keys, job.keys_sorted, job.vals, job.order, (int)job.n, kSortBits,
                             st0));
     const size_t nb = plan.size();
     GBSW_HIP_TRY(zero_u32(ex.queue.as<uint32_t>(), (int)(kXcds * nb), st0));
     size_t split_words = 0;
-    for (size_t i = 0; i < nb; ++i)
-        if (plan_is_split(plan[i]))
-            split_words = std::max(split_words, plan[i].split_at + split_words_of(job.buckets[i], plan[i]));
+    for (const BucketPlan& b : plan)
+        if (plan_is_split(b)) split_words = std::max(split_words, b.split_at + split_words_of(b));
     if (split_words) GBSW_HIP_TRY(zero_u32(ex.split_buf.as<uint32_t>(), (int)split_words, st0));
     const int ns = std::max(1, std::min(kAuxStreams + 1, ex.streams));
     GBSW_HIP_TRY(hipEventRecord(ex.ev_fork, st0));
     for (int i = 0; i < ns - 1; ++i) GBSW_HIP_TRY(hipStreamWaitEvent(ex.aux[i], ex.ev_fork, 0));
-    // each bucket (in the plan's order) goes to the stream with the least
-    // estimated work queued so far (bucket_cost): a short bucket then does not
-    // wait behind a long one and run alone at the end
+    // each launch (in the plan's order) goes to the stream with the least estimated
+    // work queued so far (its share of the whole GPU, or its longest item): a short
+    // bucket then does not wait behind a long one and run alone at the end
     std::vector<double> load((size_t)ns, 0.0);
-    for (size_t j = 0; j < order.size(); ++j) {
-        const size_t i = order[j];
+    for (size_t i = 0; i < plan.size(); ++i) {
         size_t si = 0;
         for (size_t q = 1; q < load.size(); ++q)
             if (load[q] < load[si]) si = q;
-        load[si] += bucket_cost(plan[i], job.buckets[i]);
-        const Bucket& bk = job.buckets[i];
         const BucketPlan& b = plan[i];
+        const Bucket& bk = b.bk;
+        load[si] += std::max(b.work, b.unit);
         a.order = job.order + bk.begin;
         a.order_n = bk.count;
         a.queue = ex.queue.as<uint32_t>() + kXcds * i;
+        a.bnd_rows = std::max(1, bk.max_rows);
+        a.kmax = b.K;
+        a.nranges = (int32_t)std::min<size_t>(kMaxRanges, b.ranges.size());
+        for (int32_t r = 0; r < a.nranges; ++r) a.ranges[r] = b.ranges[(size_t)r];
         a.sat_limit = b.sat_limit;
         std::memset(&a.split, 0, sizeof(a.split));
         if (plan_is_split(b)) {
             uint32_t* w = ex.split_buf.as<uint32_t>() + b.split_at;
-            const int64_t nquads = (bk.count + kPairsPerWave - 1) / kPairsPerWave;
             const int64_t nslots = 2 * (int64_t)b.grid;
             a.split.keys = (uint64_t*)w;
             a.split.prog = (uint64_t*)(w + 4 * bk.count);
             a.split.done = w + 4 * bk.count + 2 * nslots;
-            a.split.rel = a.split.done + 2 * nquads;
+            a.split.rel = a.split.done + 2 * b.sets();
             a.split.xcc = a.split.rel + nslots;
             a.split.gate = a.split.xcc + kXcds;
             if (((uintptr_t)a.split.keys | (uintptr_t)a.split.prog) & 7)
@@ -740,10 +836,11 @@ std::string graph_key(const Exec& ex, const Job& job, const gbsw_scoring* sc, co
     k.append((const char*)jf, sizeof(jf));
     for (size_t i = 0; i < plan.size(); ++i) {
         const BucketPlan& b = plan[i];
-        const Bucket& bk = job.buckets[i];
+        const Bucket& bk = b.bk;
         const int64_t f[] = {b.kind, b.K, b.grid, b.lds, b.strips, (int64_t)b.bnd_at, (int64_t)b.split_at,
-                             bk.begin, bk.count, bk.max_cols};
+                             bk.begin, bk.count, bk.max_cols, bk.max_rows};
         k.append((const char*)f, sizeof(f));
+        k.append((const char*)b.ranges.data(), sizeof(SetRange) * b.ranges.size());
     }
     return k;
 }
@@ -794,7 +891,7 @@ int enqueue_job(Exec& ex, const Job& job, const gbsw_scoring* sc, int mode)
         // pairs more than the extra waves gain (793 vs 593 GCUPS on the 1M-pair
         // DNA mix), so it applies to profile-free alphabets only
         const int K = std::min(kclamp, k_for_cols(job.max_cols, job.alpha,
-                                                  byte_profile_alphabet(job.alpha) ? job.kmodel : kModelClassic, 1 << 30));
+                                                  byte_profile_alphabet(job.alpha) ? job.kmodel : kModelClassic));
         const int lds = lds_for(K, job.alpha, p8);
         const int64_t nquads = (job.n + kPairsPerWave - 1) / kPairsPerWave;
         a.order = nullptr;
@@ -824,19 +921,18 @@ int enqueue_job(Exec& ex, const Job& job, const gbsw_scoring* sc, int mode)
         return GBSW_OK;
     }
     std::vector<BucketPlan> plan;
-    std::vector<size_t> order;
     // scores of the sweep kernels: bytes where they fit an int8 profile (large
     // alphabets) or have at most three significant bits (small ones), else 16 bits
     SweepChoice sw = sweep_choice(sub, job.alpha, sc->gap_open, sc->gap_extend, max_sub,
                                   byte_profile_alphabet(job.alpha) ? p8 : f16p8);
     sw.ok = sw.ok && ex.f16;
     a.base = sw.base;
-    rc = plan_batched(ex, job, max_sub, p8, sw, a.asym != 0, kclamp, a.bnd_rows, plan, order);
+    rc = plan_batched(ex, job, max_sub, p8, sw, a.asym != 0, kclamp, plan);
     if (rc) return rc;
     const size_t sub_bytes = sizeof(int16_t) * sub.size();
     if (!ex.graphs || ex.fixed || !job.graph) {
         GBSW_HIP_TRY(hipEventRecord(ex.ev_start, st0));
-        rc = record_batched(ex, job, a, plan, order, sub_bytes);
+        rc = record_batched(ex, job, a, plan, sub_bytes);
         if (rc) return rc;
         GBSW_HIP_TRY(hipEventRecord(ex.ev_stop, st0));
         return GBSW_OK;
@@ -849,7 +945,7 @@ int enqueue_job(Exec& ex, const Job& job, const gbsw_scoring* sc, int mode)
     if (!G.exec || G.key != key) {
         G.reset();
         GBSW_HIP_TRY(hipStreamBeginCapture(st0, hipStreamCaptureModeRelaxed));
-        rc = record_batched(ex, job, a, plan, order, sub_bytes);
+        rc = record_batched(ex, job, a, plan, sub_bytes);
         hipGraph_t graph = nullptr;
         const hipError_t ce = hipStreamEndCapture(st0, &graph);
         if (rc) {

@@ -56,13 +56,30 @@ struct PinnedBuffer {
     template <class T> T* as() const { return (T*)ptr; }
 };
 
-// One length bucket of the batched form: a kernel geometry and a slice of the
-// sorted work order.
+// The pairs of one length class (or several): a slice of the sorted work order.
 struct Bucket {
-    int K = 0;
     int64_t begin = 0, count = 0;
-    int64_t cells = 0;
-    int32_t max_cols = 0; // longest shorter sequence: bounds the bucket's scores
+    int64_t cells = 0, rows = 0, cols = 0; // sums over the pairs
+    int32_t max_cols = 0, max_rows = 0;    // longest shorter and longest longer sequence
+    // one pair, by its shorter and longer length
+    void add(int32_t shorter, int32_t longer)
+    {
+        count += 1;
+        cells += (int64_t)shorter * longer;
+        cols += shorter;
+        rows += longer;
+        max_cols = shorter > max_cols ? shorter : max_cols;
+        max_rows = longer > max_rows ? longer : max_rows;
+    }
+    void add(const Bucket& o)
+    {
+        count += o.count;
+        cells += o.cells;
+        cols += o.cols;
+        rows += o.rows;
+        max_cols = o.max_cols > max_cols ? o.max_cols : max_cols;
+        max_rows = o.max_rows > max_rows ? o.max_rows : max_rows;
+    }
 };
 
 struct LaunchRec {
@@ -147,7 +164,6 @@ struct Job {
     int32_t max_rows = 0, max_cols = 0;
     int64_t cells = 0;
     std::vector<Bucket> buckets;     // batched form (host counts)
-    const uint8_t* bucket_of_len = nullptr; // device table for the keys kernel
     uint32_t* keys = nullptr;
     uint32_t* keys_sorted = nullptr;
     int32_t* vals = nullptr;
@@ -170,26 +186,16 @@ constexpr int kModelOccupancy = 1;
 // 2.5, 2.0, 3.0, 4.0, 1.5 waves
 constexpr int kGeometryModels = 6;
 double occupancy_threshold(int model);
-// K for a shorter sequence of `cols` residues, at most klimit.
-int k_for_cols(int cols, int alpha, int model, int klimit);
-constexpr int kSweepMaxK = 16; // widest sweep kernel with four pairs per wave
-// Bucket ids: position of K in kernel_k_list, plus once the list's length for
-// pairs that span several strips with at most kMultiShortCols columns, twice for
-// longer ones (bucket_ids() in all).
-int bucket_ids();
-// Host table shorter-length -> bucket id, 65536 entries, cached per (alpha, model).
-const std::vector<uint8_t>& bucket_table(int alpha, int model);
-// Key bits of the device radix sort: bucket id << 16 | (65535 - longer length).
-constexpr int kSortBits = 22;
-// Multi-strip pairs up to this many columns form buckets of their own (ids nk ..
-// 2nk-1), longer ones the ids 2nk .. 3nk-1, so that a wave's pairs and a bucket's
-// strips are of like length.
-constexpr int kMultiShortCols = 512;
-// Fill job.buckets from per-pair lengths (host), ordered by ascending K.
+// K of the int16 kernels for a shorter sequence of `cols` residues.
+int k_for_cols(int cols, int alpha, int model);
+// Share of the VALU issue rate that `waves` per SIMD reach under a model's threshold.
+double issue_share(double waves, double threshold);
+// Fill job.buckets from per-pair lengths (host), or from the sums per length class:
+// the classes that occur, in work order (longest first).
 void count_buckets(Job& job, const int32_t* len_ref, const int32_t* len_qry);
-// Workgroups of a full-occupancy batched launch for K columns per lane (the grid
-// of a bucket is min(this, ceil(pairs / kPairsPerWave))).
-int batched_grid_cap(const Exec& ex, int K, int alpha);
+void place_buckets(Job& job, const Bucket* by_class);
+// Workgroups of a full-occupancy one-pair-per-wave launch.
+int wide_grid_cap(const Exec& ex, int alpha);
 // Whether a scoring runs the sweep kernels (gbsw_sweep.hpp), and how: the profile
 // form, the offset of all cell values, and the score from which a pair may have
 // left the 16-bit range.  bytes: the scores may be held as bytes.

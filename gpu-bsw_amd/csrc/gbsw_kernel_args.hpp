@@ -82,6 +82,35 @@ __host__ __device__ constexpr bool split_rerun_needed(const int32_t* status)
 // wave runs on (gfx942 / gfx950).
 constexpr int kXccIdReg = (3 << 11) | (0 << 6) | 20;
 
+// Length classes: pairs by their shorter sequence, the columns of the DP.  Upper
+// bounds: 64 .. 256 in steps of 32 and 320 .. 512 in steps of 64 (one strip of a
+// sweep kernel with four pairs per wave and 2 .. 8, 10, 12, 14, 16 columns per
+// virtual lane), then steps of 128 to 1024, 512 to 8192, 1024 to 16384, and 4096.
+constexpr int kClasses = 50;
+__host__ __device__ constexpr int length_class(int m)
+{
+    return m <= 64      ? 0
+           : m <= 256   ? (m - 33) / 32
+           : m <= 512   ? 7 + (m - 257) / 64
+           : m <= 1024  ? 11 + (m - 513) / 128
+           : m <= 8192  ? 15 + (m - 1025) / 512
+           : m <= 16384 ? 29 + (m - 8193) / 1024
+                        : 37 + (m - 16385) / 4096;
+}
+// Sort key of a pair: classes of longer pairs first, in a class the most rows
+// first (longest-processing-time order for the work queues, and like row counts
+// in a wave).  kRowBits bits of row count in steps of 32.
+constexpr int kRowBits = 9;
+constexpr int kSortBits = 6 + kRowBits;
+static_assert(kClasses <= 64, "class bits of the sort key");
+
+// Work of a sweep launch: sets of pairs in work order, the sets that start below
+// pair `end` in geometry K (columns per virtual lane).
+constexpr int kMaxRanges = 16;
+struct SetRange {
+    int32_t end, K;
+};
+
 struct KernelArgs {
     const uint8_t* ref;
     const uint64_t* ref_off;   // n+1 exclusive prefix offsets
@@ -107,6 +136,9 @@ struct KernelArgs {
     int32_t asym;              // 1: sub[] is not symmetric (the reverse pass then finds its own maximum
                                //    when its orientation differs from the forward pass's)
     int32_t base;              // sweep kernels: offset of all cell values (gbsw_sweep.hpp)
+    int32_t kmax;              // widest geometry of the launch (its LDS layout)
+    int32_t nranges;
+    SetRange ranges[kMaxRanges];
     SplitArgs split;           // split forms only
 };
 

@@ -30,6 +30,9 @@
 //    chosen after the pass.
 //  reverse: the same DP on the reversed prefixes; among cells with H = score, the
 //    smallest reversed column, then its first row (kernel.cpp:3-45, 577-581).
+#include <array>
+#include <map>
+#include <mutex>
 #include <type_traits>
 
 #include "gbsw_device.hpp"
@@ -1062,10 +1065,10 @@ static const void* kernel_for(int kind, int K)
 {
     const int base = kind & 0xFF;
     if (base == kBatchedF16 || base == kSplitF16) {
-        const bool split = base == kSplitF16, wide = (kind & kWideGroup) != 0;
-        return (kind & kRegTables) ? sweep_kernel_regs(split, wide, K)
-               : (kind & kByteProfile) ? sweep_kernel_bytes(split, wide, K)
-                                       : sweep_kernel_words(split, wide, K);
+        const bool wide = (kind & kWideGroup) != 0;
+        if (kind & kRegTables) return wide ? sweep_kernel_regs_wide(kind, K) : sweep_kernel_regs(kind, K);
+        if (kind & kByteProfile) return wide ? sweep_kernel_bytes_wide(kind, K) : sweep_kernel_bytes(kind, K);
+        return wide ? sweep_kernel_words_wide(kind, K) : sweep_kernel_words(kind, K);
     }
     return (kind & kByteProfile) ? kernel_for_profile<true>(kind & ~kByteProfile, K)
                                  : kernel_for_profile<false>(kind, K);
@@ -1097,12 +1100,23 @@ const int* kernel_k_list(int* count)
 }
 
 // Workgroups of one kernel that fit on a CU at this LDS size (0 on error).
+// Remembered: a plan asks for a few hundred of them.
 int kernel_occupancy(int kind, int K, int lds_bytes)
 {
+    static std::mutex mu;
+    static std::map<std::array<int, 3>, int> known;
+    const std::array<int, 3> key = {kind, K, lds_bytes};
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        const auto it = known.find(key);
+        if (it != known.end()) return it->second;
+    }
     const void* f = kernel_for(kind, K);
     if (!f) return 0;
     int nb = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, kWave, (size_t)lds_bytes) != hipSuccess) return 0;
+    std::lock_guard<std::mutex> lk(mu);
+    known[key] = nb;
     return nb;
 }
 

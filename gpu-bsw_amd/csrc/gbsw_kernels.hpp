@@ -22,18 +22,30 @@ inline int with_profile(int kind, bool bytes8) { return bytes8 ? (kind | kBytePr
 // The sweep kernels (gbsw_sweep.hpp) are kBatchedF16 and kSplitF16 with these
 // flags.  kRegTables: the scores of a lane's columns in registers (at most
 // kRegAlpha residue codes) instead of a profile in LDS.  kWideGroup: one pair per
-// wave (64 lanes) instead of four (16 lanes each).
+// wave (64 lanes) instead of four (16 lanes each).  kWideLanes: the four-pair
+// kernel of the wide geometries (K from 10).  A kernel without kSplitF16 holds
+// every geometry of its list; a split one is compiled per K.
 constexpr int kWideGroup = 0x200;
 constexpr int kRegTables = 0x400;
+constexpr int kWideLanes = 0x800;
 constexpr int kReportedKind = 0x1FF; // the part of a kind that launch statistics report
-inline int sweep_kind(int kind, int form)
+inline int sweep_kind(int kind, int form, int flags)
 {
+    kind |= flags;
     return form == kProfRegs ? kind | kByteProfile | kRegTables : form == kProfBytes ? kind | kByteProfile : kind;
 }
+// Geometries of the sweep kernels.
+#define GBSW_SWEEP_K16(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8)
+#define GBSW_SWEEP_K16_WIDE(X) X(10) X(12) X(14) X(16)
+#define GBSW_SWEEP_K64(X) X(1) X(2) X(3) X(4) X(5) X(6) X(8)
+#define GBSW_SWEEP_K64_SPLIT(X) X(1) X(2) X(3) X(4) X(6) X(8)
 // kernel of a form, nullptr where it is not compiled (gbsw_sweep_*.hip)
-const void* sweep_kernel_regs(bool split, bool wide, int K);
-const void* sweep_kernel_bytes(bool split, bool wide, int K);
-const void* sweep_kernel_words(bool split, bool wide, int K);
+const void* sweep_kernel_regs(int kind, int K);
+const void* sweep_kernel_bytes(int kind, int K);
+const void* sweep_kernel_words(int kind, int K);
+const void* sweep_kernel_regs_wide(int kind, int K);
+const void* sweep_kernel_bytes_wide(int kind, int K);
+const void* sweep_kernel_words_wide(int kind, int K);
 
 bool kernel_supported(int K);
 bool kernel_has(int kind, int K);
@@ -44,12 +56,8 @@ hipError_t kernel_launch(int kind, int K, int grid, int lds_bytes, hipStream_t s
 hipError_t zero_u32(uint32_t* p, int n, hipStream_t stream);
 
 // gbsw_binning.hip
-// Columns of one strip (32 x K) of each bucket id.
-struct StripWidths {
-    uint16_t w[64];
-};
-hipError_t bin_keys(const uint64_t* ref_off, const uint64_t* qry_off, int64_t n, const uint8_t* bucket_of_len,
-                    const StripWidths& widths, uint32_t* keys, int32_t* vals, hipStream_t stream);
+hipError_t bin_keys(const uint64_t* ref_off, const uint64_t* qry_off, int64_t n, uint32_t* keys, int32_t* vals,
+                    hipStream_t stream);
 // OR into mask[8] the set of byte values in p[0, n) (p 16-byte aligned).
 hipError_t byte_presence(const uint8_t* p, uint64_t n, uint32_t* mask, hipStream_t stream);
 hipError_t sort_pairs(void* temp, size_t& temp_bytes, const uint32_t* kin, uint32_t* kout, const int32_t* vin,

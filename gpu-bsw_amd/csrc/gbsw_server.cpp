@@ -58,7 +58,8 @@ Clock::time_point trace_epoch()
     return t0;
 }
 
-constexpr int kMaxBuckets = 64;
+constexpr int kMaxBuckets = 64; // launches of a micro-batch
+constexpr int kWideFromClass = length_class(129); // pairs that may take several strips of one wave
 // Pinned host memory that kernels read in place: mapped, and coherent so that a
 // region rewritten by the host after an earlier read is never served stale.
 constexpr unsigned kDeviceReadFlags = hipHostMallocMapped | hipHostMallocCoherent;
@@ -173,10 +174,8 @@ struct AlphabetTables {
     int32_t alpha = 0;
     int kmax = 0;
     uint8_t lut[256];
-    std::vector<uint8_t> bucket_of_len; // host copy (65536)
-    std::vector<int> bucket_k;          // K of each bucket index
-    std::vector<int> bucket_full;       // full-occupancy grid of each bucket index
-    DeviceBuffer d_bucket_of_len, d_accept;
+    int wide_full = 1; // full-occupancy grid of the one-pair-per-wave kernel
+    DeviceBuffer d_accept;
 };
 
 struct Request {
@@ -190,9 +189,7 @@ struct Request {
     // summary for whole-request admission
     int64_t residues = 0, cells = 0;
     int32_t max_rows = 0, max_cols = 0;
-    int64_t bucket_count[kMaxBuckets] = {0};
-    int64_t bucket_cells[kMaxBuckets] = {0};
-    int32_t bucket_maxcols[kMaxBuckets] = {0};
+    Bucket buckets[kClasses];
     // progress (guarded by the server mutex)
     int64_t next = 0;
     int parts = 0, parts_pending = 0;
@@ -338,21 +335,9 @@ int gbsw_server::init_tables(int which)
         for (int c = 0; c < 256; ++c) accept[c] = c < 91;
     }
     t.kmax = max_k_for(t.alpha, byte_profile_alphabet(t.alpha));
-    t.bucket_of_len = bucket_table(t.alpha, slots[0]->ex.kmodel);
-    int nk = 0;
-    const int* ks = kernel_k_list(&nk);
-    const int nb = bucket_ids();
-    if (nb > kMaxBuckets) return fail(GBSW_E_INTERNAL, "too many kernel geometries");
-    t.bucket_k.resize((size_t)nb);
-    t.bucket_full.resize((size_t)nb);
-    for (int i = 0; i < nb; ++i) {
-        t.bucket_k[(size_t)i] = ks[i % nk];
-        t.bucket_full[(size_t)i] = batched_grid_cap(slots[0]->ex, ks[i % nk], t.alpha);
-    }
-    int rc = alloc_into(t.d_bucket_of_len, 65536, device_bytes);
-    if (!rc) rc = alloc_into(t.d_accept, 256, device_bytes);
+    t.wide_full = wide_grid_cap(slots[0]->ex, t.alpha);
+    const int rc = alloc_into(t.d_accept, 256, device_bytes);
     if (rc) return rc;
-    GBSW_HIP_TRY(hipMemcpy(t.d_bucket_of_len.ptr, t.bucket_of_len.data(), 65536, hipMemcpyHostToDevice));
     GBSW_HIP_TRY(hipMemcpy(t.d_accept.ptr, accept, 256, hipMemcpyHostToDevice));
     return GBSW_OK;
 }
@@ -379,7 +364,7 @@ int gbsw_server::init_slot(Slot& s)
     // split-form bookkeeping: keys, strip gates and counters of every pair, the
     // progress words of up to two boundary slots per workgroup of a full grid
     // per bucket, and each bucket's padding to 256 bytes
-    const size_t split_words = 5 * P + 2 * (P / kPairsPerWave + kMaxBuckets) +
+    const size_t split_words = 5 * P + 2 * (P + kMaxBuckets) +
                                6 * (size_t)kMaxBuckets * 16 * s.ex.num_cu + (size_t)(kXcds + 64) * kMaxBuckets;
     if (!rc) rc = alloc_into(s.ex.split_buf, 4 * split_words, device_bytes);
     s.ex.fixed = true;
@@ -411,17 +396,15 @@ void gbsw_server::admit(Slot& s)
     const int c = oldest_class();
     ScoreClass& C = classes[(size_t)c];
     const AlphabetTables& T = tabs[C.tables];
-    const int nb = (int)T.bucket_k.size();
     const int64_t cap_pairs = cfg.pairs_per_slot, cap_res = cfg.residues_per_slot;
     const int64_t cap_bnd = cfg.boundary_bytes_per_slot;
-    int64_t cnt[kMaxBuckets] = {0}, cel[kMaxBuckets] = {0};
-    int32_t mcol[kMaxBuckets] = {0};
-    int64_t pairs = 0, res = 0, quads = 0, cells = 0;
+    Bucket sum[kClasses];
+    int64_t pairs = 0, res = 0, wide = 0, cells = 0;
     int32_t max_rows = 0, max_cols = 0;
-    auto quads_of = [&](int b, int64_t count) {
-        return std::min<int64_t>(T.bucket_full[(size_t)b], (count + kPairsPerWave - 1) / kPairsPerWave);
+    // boundary rows: one workgroup per pair of several strips, up to a full grid
+    auto bnd_need = [&](int64_t wide, int32_t rows) {
+        return std::min<int64_t>(T.wide_full, std::max<int64_t>(1, wide)) * (int64_t)std::max(1, rows) * 4;
     };
-    auto bnd_need = [&](int64_t q, int32_t rows) { return q * kPairsPerWave * (int64_t)std::max(1, rows) * 4; };
     s.parts.clear();
     s.sc = C.sc;
     s.tables = C.tables;
@@ -431,16 +414,12 @@ void gbsw_server::admit(Slot& s)
         int64_t take = 0;
         if (r->next == 0) {
             // whole request at once when it fits
-            int64_t q2 = 0;
-            for (int b = 0; b < nb; ++b) q2 += quads_of(b, cnt[b] + r->bucket_count[b]);
+            int64_t w2 = wide;
+            for (int c = kWideFromClass; c < kClasses; ++c) w2 += r->buckets[c].count;
             const int32_t rows2 = std::max(max_rows, r->max_rows);
-            if (pairs + r->n <= cap_pairs && res + r->residues <= cap_res && bnd_need(q2, rows2) <= cap_bnd) {
-                for (int b = 0; b < nb; ++b) {
-                    cnt[b] += r->bucket_count[b];
-                    cel[b] += r->bucket_cells[b];
-                    mcol[b] = std::max(mcol[b], r->bucket_maxcols[b]);
-                }
-                quads = q2;
+            if (pairs + r->n <= cap_pairs && res + r->residues <= cap_res && bnd_need(w2, rows2) <= cap_bnd) {
+                for (int c = 0; c < kClasses; ++c) sum[c].add(r->buckets[c]);
+                wide = w2;
                 max_rows = rows2;
                 max_cols = std::max(max_cols, r->max_cols);
                 res += r->residues;
@@ -453,17 +432,15 @@ void gbsw_server::admit(Slot& s)
             for (int64_t p = r->next; p < r->n; ++p) {
                 const int32_t la = (int32_t)(r->ro[(size_t)p + 1] - r->ro[(size_t)p]);
                 const int32_t lb = (int32_t)(r->qo[(size_t)p + 1] - r->qo[(size_t)p]);
-                const int b = T.bucket_of_len[(size_t)std::min(la, lb)];
-                const int64_t q2 = quads - quads_of(b, cnt[b]) + quads_of(b, cnt[b] + 1);
+                const int c = length_class(std::min(la, lb));
+                const int64_t w2 = wide + (c >= kWideFromClass ? 1 : 0);
                 const int32_t rows2 = std::max(max_rows, std::max(la, lb));
-                if (pairs + take + 1 > cap_pairs || res + la + lb > cap_res || bnd_need(q2, rows2) > cap_bnd) {
+                if (pairs + take + 1 > cap_pairs || res + la + lb > cap_res || bnd_need(w2, rows2) > cap_bnd) {
                     full = true;
                     break;
                 }
-                cnt[b] += 1;
-                cel[b] += (int64_t)la * lb;
-                mcol[b] = std::max(mcol[b], std::min(la, lb));
-                quads = q2;
+                sum[c].add(std::min(la, lb), std::max(la, lb));
+                wide = w2;
                 max_rows = rows2;
                 max_cols = std::max(max_cols, std::min(la, lb));
                 res += la + lb;
@@ -504,19 +481,7 @@ void gbsw_server::admit(Slot& s)
     j.max_rows = max_rows;
     j.max_cols = max_cols;
     j.cells = cells;
-    j.buckets.clear();
-    int64_t at = 0;
-    for (int b = 0; b < nb; ++b) {
-        if (!cnt[b]) continue;
-        Bucket bk;
-        bk.K = T.bucket_k[(size_t)b];
-        bk.begin = at;
-        bk.count = cnt[b];
-        bk.cells = cel[b];
-        bk.max_cols = mcol[b];
-        at += cnt[b];
-        j.buckets.push_back(bk);
-    }
+    place_buckets(j, sum);
     s.busy = true;
     s.launch_seq = ++launch_counter;
     ++busy_slots;
@@ -600,7 +565,6 @@ int gbsw_server::launch(Slot& s)
     j.ref_off = s.meta.as<uint64_t>();
     j.qry_off = s.meta.as<uint64_t>() + (n + 1);
     j.out = s.out.as<int32_t>();
-    j.bucket_of_len = T.d_bucket_of_len.as<uint8_t>();
     j.keys = s.keys.as<uint32_t>();
     j.keys_sorted = s.keys_sorted.as<uint32_t>();
     j.vals = s.vals.as<int32_t>();
@@ -887,10 +851,7 @@ int gbsw_server_submit(gbsw_server* srv, const gbsw_scoring* sc, int64_t n, cons
             delete r;
             return fail(GBSW_E_RANGE, "sequences longer than 65000 residues are not supported");
         }
-        const int b = T.bucket_of_len[(size_t)std::min(la, lb)];
-        r->bucket_count[b] += 1;
-        r->bucket_cells[b] += (int64_t)(la * lb);
-        r->bucket_maxcols[b] = std::max<int32_t>(r->bucket_maxcols[b], (int32_t)std::min(la, lb));
+        r->buckets[length_class((int)std::min(la, lb))].add((int32_t)std::min(la, lb), (int32_t)std::max(la, lb));
         r->cells += (int64_t)(la * lb);
         r->max_rows = std::max<int32_t>(r->max_rows, (int32_t)std::max(la, lb));
         r->max_cols = std::max<int32_t>(r->max_cols, (int32_t)std::min(la, lb));

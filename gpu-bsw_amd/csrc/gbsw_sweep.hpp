@@ -209,8 +209,9 @@ struct SweepFetch {
 };
 constexpr int kNoRow = 256; // its entry of the row table is the padding row
 
-// The rings.  MS: the wave has pairs of several strips (boundary entries in use).
-template <class A, int G, int PF, bool MS>
+// The rings.  ROWB: bytes of a profile row.  MS: the wave has pairs of several
+// strips (boundary entries in use).
+template <class A, int G, int PF, int ROWB, bool MS>
 struct SweepRows {
     static constexpr int N = kChunk / G > 1 ? kChunk / G : 1; // rows per lane and chunk
     static constexpr int R = sweep_ring(G);
@@ -246,7 +247,8 @@ struct SweepRows {
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             const int x = chunk * kChunk + l + G * i;
-            const uint16_t e = row_tab[f.b[i]];
+            const uint32_t c = row_tab[f.b[i]];
+            const uint16_t e = (uint16_t)(PF == kProfRegs ? c : c * (uint32_t)ROWB);
             const int at = x & (R - 1);
             if constexpr (PF == kProfRegs) {
                 // entry r is a whole v_perm selector, for a lane's rows r (low half) and
@@ -270,16 +272,16 @@ struct SweepRows {
     }
 };
 
-// Row table: byte -> ring entry of its row (profile offset, or selector half).
+// Row table: byte -> code of its row (register form: its half of the selector).
 // Column table (register form): byte -> the four biased scores of its column.
 template <int PF>
-__device__ __forceinline__ void stage_byte_tables(const KernelArgs& a, const SweepSmem& sm, int rowstride)
+__device__ __forceinline__ void stage_byte_tables(const KernelArgs& a, const SweepSmem& sm)
 {
     const int alpha = a.alpha, sbias = -(a.gap_open + a.gap_extend);
     for (int i = threadIdx.x; i <= kNoRow; i += kWave) {
         int c = i < kNoRow ? (int)sm.lut()[i] : alpha;
         c = c > alpha ? alpha : c; // bytes outside the alphabet read the padding row
-        sm.row_tab()[i] = PF == kProfRegs ? (uint16_t)(c == alpha ? kPadSelector : 0x0C00 | c) : (uint16_t)(c * rowstride);
+        sm.row_tab()[i] = PF == kProfRegs ? (uint16_t)(c == alpha ? kPadSelector : 0x0C00 | c) : (uint16_t)c;
         if constexpr (PF == kProfRegs) {
             uint32_t w = 0;
             for (int r = 0; r < alpha; ++r)
@@ -339,7 +341,7 @@ struct SweepProf {
 // io.bnd_in / io.bnd_out as they are published, else every strip with the
 // boundary rows in bnd_g.  Winner keys as in gbsw_pass.hpp.
 template <class A, int G, int K, int PF, bool REV, bool SPLIT = false>
-__device__ PassResult sweep(const KernelArgs& a, const SweepSmem& sm, const Task& t, int32_t target,
+__device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem& sm, const Task& t, int32_t target,
                             typename A::B* bnd_g, const StripIO& io = StripIO{})
 {
     using V = typename A::V;
@@ -370,7 +372,8 @@ __device__ PassResult sweep(const KernelArgs& a, const SweepSmem& sm, const Task
     }
     strips_max = __builtin_amdgcn_readfirstlane(strips_max);
     steps_max = __builtin_amdgcn_readfirstlane(steps_max);
-    const bool multi_strip = strips_max > 1;
+    // (the host gives four-pair waves pairs of one strip only)
+    const bool multi_strip = G == kWave && strips_max > 1;
     const int strip_lo = SPLIT ? io.strip : 0;
 
     const U gs = A::uni(ge), cs = A::uni(ge - go), hand_u = A::uni(ge * (K - 1));
@@ -477,7 +480,7 @@ __device__ PassResult sweep(const KernelArgs& a, const SweepSmem& sm, const Task
         // two forms are separate loops so that neither holds the other's registers
         auto chunks = [&](auto ms) {
             constexpr bool MS = decltype(ms)::value;
-            using Rows = SweepRows<A, G, PF, MS>;
+            using Rows = SweepRows<A, G, PF, rowstride, MS>;
             // row ring: 2G padding rows, rows [0, 32) now, [32, 64) in flight
             for (int c = -(VL / kChunk); c < 0; ++c)
                 Rows::store(Rows::none(), c, l, ring_code, ring_bnd, row_tab, base, ge, go);
@@ -636,8 +639,12 @@ __device__ PassResult sweep(const KernelArgs& a, const SweepSmem& sm, const Task
                 }
             }
         };
-        if (multi_strip) chunks(std::true_type{});
-        else chunks(std::false_type{});
+        if constexpr (G == kWave) {
+            if (multi_strip) chunks(std::true_type{});
+            else chunks(std::false_type{});
+        } else {
+            chunks(std::false_type{});
+        }
         if (multi_strip) {
             // the last chunk's rows; complete before the next strip reads them
             __syncthreads();
@@ -708,30 +715,69 @@ __device__ PassResult sweep(const KernelArgs& a, const SweepSmem& sm, const Task
     return r;
 }
 
-template <class A, int G, int K, int PF>
+template <class A, int G, int PF>
 __device__ __forceinline__ SweepSmem sweep_smem(uint8_t* mem, const KernelArgs& a)
 {
-    SweepLds L = sweep_lds(G, K, PF, a.alpha, (int)sizeof(typename A::B));
+    SweepLds L = sweep_lds(G, a.kmax, PF, a.alpha, (int)sizeof(typename A::B));
     // an opaque group offset keeps the compiler from splitting the layout's rounding
     // constants into the profile address (see make_smem of the int16 kernels)
     asm volatile("" : "+s"(L.group_off));
     return SweepSmem{mem, L};
 }
 
-// Waves per SIMD the register allocation leaves room for.
-constexpr int sweep_waves(int K) { return K <= 6 ? 4 : K <= 12 ? 3 : 2; }
-
-// Persistent workgroups (one wave) pull sets of 64/G length-sorted pairs from a
-// device work queue and run forward then reverse back to back.
+// Both passes of one set of pairs, and its results.
 template <class A, int G, int K, int PF>
-__global__ __launch_bounds__(64, sweep_waves(K)) void k_sweep(KernelArgs a)
+__device__ __forceinline__ void sweep_set(const KernelArgs& a, const SweepSmem& sm, int64_t p, typename A::B* bnd_g)
+{
+    const int l = threadIdx.x & (G - 1);
+    // the forward pass, then (asymmetric tables, wave-uniform) the forward-style
+    // pass over the reversed boxes that need their own maximum: one call site
+    Task tf = forward_task(a, p);
+    FwdOut f{0, 0, 0};
+    RevPlan rp;
+#pragma nounroll
+    for (int fp = 0;; ++fp) {
+        const PassResult rf = sweep<A, G, K, PF, false>(a, sm, tf, 0, bnd_g);
+        if (fp == 0) {
+            f = forward_result<G>(a, p, rf.key);
+            rp = reverse_plan<G>(a, sm, p, f);
+            if (__ballot(rp.gen) == 0) break;
+            tf = rp.gen ? rp.t : empty_task(a, 1);
+        } else {
+            reverse_plan_finish<G>(a, p, rf.key, rp);
+            break;
+        }
+    }
+    const PassResult rr = sweep<A, G, K, PF, true>(a, sm, rp.t, rp.target, bnd_g);
+    int32_t rb, qb;
+    reverse_result(a, p, f, rp.t, rp.target, rr.key, &rb, &qb);
+    if (p >= 0 && l == 0 && f.score >= 0 && !rp.saturated) {
+        a.out[kOutScore * a.n + p] = f.score;
+        a.out[kOutRefEnd * a.n + p] = f.ref_end;
+        a.out[kOutQueryEnd * a.n + p] = f.query_end;
+        a.out[kOutRefBegin * a.n + p] = rb;
+        a.out[kOutQueryBegin * a.n + p] = qb;
+    }
+}
+
+// Persistent workgroups (one wave) pull sets of 64/G pairs from a device work queue,
+// longest first, and run forward then reverse back to back.  One launch holds every
+// geometry of its list: the sets' geometries come from a.ranges, so the waves run
+// through all of them without a gap and the launch has one tail.  (One launch per
+// geometry, sixteen on the 1M-pair DNA mix, left each its own tail and the hardware
+// queues unevenly loaded: 26.3-27.5 ms against 25.7 ms; 150k pairs 9.4 against 5.0.)
+// WIDE: the four-pair geometries of K >= 10, whose registers leave room for fewer
+// waves.
+constexpr int sweep_group_waves(int G, bool WIDE) { return G == 16 && WIDE ? 3 : 4; }
+template <class A, int G, int PF, bool WIDE>
+__global__ __launch_bounds__(64, sweep_group_waves(G, WIDE)) void k_sweep(KernelArgs a)
 {
     extern __shared__ __align__(16) uint8_t smem_raw[];
     constexpr int PW = kWave / G;
-    const SweepSmem sm = sweep_smem<A, G, K, PF>(smem_raw, a);
+    const SweepSmem sm = sweep_smem<A, G, PF>(smem_raw, a);
     stage_tables(a, sm);
-    stage_byte_tables<PF>(a, sm, sweep_row_bytes(G, K, PF));
-    const int l = threadIdx.x & (G - 1), g = threadIdx.x / G;
+    stage_byte_tables<PF>(a, sm);
+    const int g = threadIdx.x / G;
     typename A::B* bnd_g = (typename A::B*)a.bnd + ((int64_t)blockIdx.x * PW + g) * a.bnd_rows;
     const int64_t nsets = (a.order_n + PW - 1) / PW;
     for (;;) {
@@ -740,34 +786,18 @@ __global__ __launch_bounds__(64, sweep_waves(K)) void k_sweep(KernelArgs a)
         q = (uint32_t)__builtin_amdgcn_readfirstlane((int)q);
         if ((int64_t)q >= nsets) break;
         const int64_t p = slot_pair(a, (int64_t)q * PW + g);
-        // the forward pass, then (asymmetric tables, wave-uniform) the forward-style
-        // pass over the reversed boxes that need their own maximum: one call site
-        Task tf = forward_task(a, p);
-        FwdOut f{0, 0, 0};
-        RevPlan rp;
-#pragma nounroll
-        for (int fp = 0;; ++fp) {
-            const PassResult rf = sweep<A, G, K, PF, false>(a, sm, tf, 0, bnd_g);
-            if (fp == 0) {
-                f = forward_result<G>(a, p, rf.key);
-                rp = reverse_plan<G>(a, sm, p, f);
-                if (__ballot(rp.gen) == 0) break;
-                tf = rp.gen ? rp.t : empty_task(a, 1);
-            } else {
-                reverse_plan_finish<G>(a, p, rf.key, rp);
-                break;
-            }
+        int K = 0;
+        for (int r = a.nranges - 1; r >= 0; --r)
+            if ((int64_t)q * PW < a.ranges[r].end) K = a.ranges[r].K;
+#define GBSW_CASE(k) case k: sweep_set<A, G, k, PF>(a, sm, p, bnd_g); break;
+        if constexpr (G == kWave) {
+            switch (K) { GBSW_SWEEP_K64(GBSW_CASE) }
+        } else if constexpr (WIDE) {
+            switch (K) { GBSW_SWEEP_K16_WIDE(GBSW_CASE) }
+        } else {
+            switch (K) { GBSW_SWEEP_K16(GBSW_CASE) }
         }
-        const PassResult rr = sweep<A, G, K, PF, true>(a, sm, rp.t, rp.target, bnd_g);
-        int32_t rb, qb;
-        reverse_result(a, p, f, rp.t, rp.target, rr.key, &rb, &qb);
-        if (p >= 0 && l == 0 && f.score >= 0 && !rp.saturated) {
-            a.out[kOutScore * a.n + p] = f.score;
-            a.out[kOutRefEnd * a.n + p] = f.ref_end;
-            a.out[kOutQueryEnd * a.n + p] = f.query_end;
-            a.out[kOutRefBegin * a.n + p] = rb;
-            a.out[kOutQueryBegin * a.n + p] = qb;
-        }
+#undef GBSW_CASE
     }
 }
 
@@ -778,13 +808,13 @@ __global__ __launch_bounds__(64, sweep_waves(K)) void k_sweep(KernelArgs a)
 // taken from the counter earlier, which holds its workgroup until it finishes,
 // and is bounded by kSpinTicks besides.
 template <class A, int G, int K, int PF>
-__global__ __launch_bounds__(64, sweep_waves(K)) void k_sweep_split(KernelArgs a)
+__global__ __launch_bounds__(64, K <= 6 ? 4 : 3) void k_sweep_split(KernelArgs a)
 {
     extern __shared__ __align__(16) uint8_t smem_raw[];
     constexpr int PW = kWave / G;
-    const SweepSmem sm = sweep_smem<A, G, K, PF>(smem_raw, a);
+    const SweepSmem sm = sweep_smem<A, G, PF>(smem_raw, a);
     stage_tables(a, sm);
-    stage_byte_tables<PF>(a, sm, sweep_row_bytes(G, K, PF));
+    stage_byte_tables<PF>(a, sm);
     const int l = threadIdx.x & (G - 1), g = threadIdx.x / G;
     const int x = (int)(blockIdx.x % kXcds);
     const SplitArgs& sp = a.split;
@@ -884,7 +914,3 @@ __global__ __launch_bounds__(64, sweep_waves(K)) void k_sweep_split(KernelArgs a
 }
 
 } // namespace gbsw
-
-// ---- the kernels of one profile form (each form is a translation unit of its own)
-#define GBSW_SWEEP_CASE(k) case k: return (const void*)&k_sweep<Sweep16, GBSW_SWEEP_G, k, GBSW_SWEEP_PF>;
-#define GBSW_SWEEP_SPLIT_CASE(k) case k: return (const void*)&k_sweep_split<Sweep16, GBSW_SWEEP_G, k, GBSW_SWEEP_PF>;

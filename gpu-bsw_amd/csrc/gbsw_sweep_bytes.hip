@@ -1,31 +1,11 @@
-// gbsw_sweep_bytes.hip -- sweep kernels: byte profile.
+// gbsw_sweep_bytes.hip -- sweep kernels with four pairs per wave: byte profile.
 #include "gbsw_sweep.hpp"
 
 namespace gbsw {
 
-#define GBSW_SWEEP_PF kProfBytes
-#ifndef GBSW_SWEEP_K16
-#define GBSW_SWEEP_K16(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(10) X(12) X(14) X(16)
-#endif
-#ifndef GBSW_SWEEP_SPLIT_K16
-#define GBSW_SWEEP_SPLIT_K16(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(10) X(12) X(14) X(16)
-#endif
-
-const void* sweep_kernel_bytes(bool split, bool wide, int K)
+const void* sweep_kernel_bytes(int kind, int)
 {
-    if (wide) return nullptr;
-#define GBSW_SWEEP_G 16
-    if (split) {
-        switch (K) {
-            GBSW_SWEEP_SPLIT_K16(GBSW_SWEEP_SPLIT_CASE)
-        default: return nullptr;
-        }
-    }
-    switch (K) {
-        GBSW_SWEEP_K16(GBSW_SWEEP_CASE)
-    default: return nullptr;
-    }
-#undef GBSW_SWEEP_G
+    return (kind & kWideLanes) ? (const void*)&k_sweep<Sweep16, 16, kProfBytes, true> : (const void*)&k_sweep<Sweep16, 16, kProfBytes, false>;
 }
 
 } // namespace gbsw

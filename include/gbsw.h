@@ -85,18 +85,18 @@ int gbsw_context_destroy(gbsw_context* ctx);
  *          0: every bucket runs the int16 kernel.  Results are identical. */
 #define GBSW_OPT_STREAMS 1
 #define GBSW_OPT_F16 2
-/* GEOMETRY: how a pair's shorter length picks its kernel geometry (K columns per
- *          lane), for batches created afterwards.  0: fewest padded columns and
- *          steps, strips x (K + 2); 1 (default; GBSW_KMODEL=m selects model m):
- *          that cost divided by min(1, waves per SIMD / 2.5), the share of the
- *          VALU issue rate the geometry's occupancy allows; 2..5: the same with
- *          2.0, 3.0, 4.0 or 1.5 waves (gbsw_batch_autotune picks among them).  Applies to the length buckets of
+/* GEOMETRY: how kernel geometries (columns per lane, lanes per pair) are weighed,
+ *          for batches created afterwards.  0: by their instructions alone; 1
+ *          (default; GBSW_KMODEL=m selects model m): instructions divided by
+ *          min(1, waves per SIMD / 2.5), the share of the VALU issue rate the
+ *          geometry's occupancy allows; 2..5: the same with 2.0, 3.0, 4.0 or 1.5
+ *          waves (gbsw_batch_autotune picks among them).  Applies to
  *          gbsw_batch_align(GBSW_BATCHED), and to the plain form for protein
  *          (the plain form uses 0 for DNA).  Results are identical. */
 #define GBSW_OPT_GEOMETRY 3
 /* SPLIT:   1 (default; GBSW_SPLIT=0 turns it off): length buckets of pairs that
- *          span several strips, with too few pairs to occupy the GPU twice
- *          over, run each strip as its own work item, on several workgroups of
+ *          span several strips, where a single pair would outlast the rest of
+ *          the job, run each strip as its own work item, on several workgroups of
  *          one XCD in a pipeline (a strip follows the boundary rows of the one
  *          before as they are written); 0: one workgroup runs a pair's strips
  *          one after another.  Results are identical. */
