@@ -6,6 +6,7 @@
 // forward launch, host newMin, reverse launch, copies back).
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -354,6 +355,8 @@ SweepChoice sweep_choice(const std::vector<int16_t>& sub, int alpha, int32_t gap
     // the padding scores -(open + extend), which must be negative; the running
     // offset and the scores leave most of the range to the cell values
     c.ok = bias >= 1 && offset <= 8192 && max_sub <= 4096 && lo > -16384 && hi < 16384;
+    // int32 cells: any range; the profile holds the biased scores in 16 bits
+    c.wide_ok = bias >= 1 && lo > -32768 && hi < 32768;
     c.form = (bytes && lo >= 0 && hi <= 255) ? (alpha <= kRegAlpha ? kProfRegs : kProfBytes) : kProfWords;
     // a pair below this never formed a value past 0x7C00 (largest offset, gap step
     // and one substitution on top of its best)
@@ -743,6 +746,24 @@ int plan_batched(Exec& ex, const Job& job, int max_sub, bool p8, const SweepChoi
     return GBSW_OK;
 }
 
+// The split form's bookkeeping of launch b, at its place in ex.split_buf.
+int set_split_args(const Exec& ex, const BucketPlan& b, KernelArgs& a)
+{
+    uint32_t* w = ex.split_buf.as<uint32_t>() + b.split_at;
+    const int64_t nslots = 2 * (int64_t)b.grid;
+    a.split.keys = (uint64_t*)w;
+    a.split.prog = (uint64_t*)(w + 4 * b.bk.count);
+    a.split.done = w + 4 * b.bk.count + 2 * nslots;
+    a.split.rel = a.split.done + 2 * b.sets();
+    a.split.xcc = a.split.rel + nslots;
+    a.split.gate = a.split.xcc + kXcds;
+    if (((uintptr_t)a.split.keys | (uintptr_t)a.split.prog) & 7)
+        return fail(GBSW_E_INTERNAL, "split bookkeeping of a launch is not 8-byte aligned");
+    a.split.strips = b.strips;
+    a.split.slots = (int32_t)(nslots / kXcds);
+    return GBSW_OK;
+}
+
 // Stream work of the batched form (recorded eagerly or into a graph).
 int record_batched(Exec& ex, const Job& job, KernelArgs a, const std::vector<BucketPlan>& plan, size_t sub_bytes)
 {
@@ -787,20 +808,8 @@ int record_batched(Exec& ex, const Job& job, KernelArgs a, const std::vector<Buc
         for (int32_t r = 0; r < a.nranges; ++r) a.ranges[r] = b.ranges[(size_t)r];
         a.sat_limit = b.sat_limit;
         std::memset(&a.split, 0, sizeof(a.split));
-        if (plan_is_split(b)) {
-            uint32_t* w = ex.split_buf.as<uint32_t>() + b.split_at;
-            const int64_t nslots = 2 * (int64_t)b.grid;
-            a.split.keys = (uint64_t*)w;
-            a.split.prog = (uint64_t*)(w + 4 * bk.count);
-            a.split.done = w + 4 * bk.count + 2 * nslots;
-            a.split.rel = a.split.done + 2 * b.sets();
-            a.split.xcc = a.split.rel + nslots;
-            a.split.gate = a.split.xcc + kXcds;
-            if (((uintptr_t)a.split.keys | (uintptr_t)a.split.prog) & 7)
-                return fail(GBSW_E_INTERNAL, "split bookkeeping of a bucket is not 8-byte aligned");
-            a.split.strips = b.strips;
-            a.split.slots = (int32_t)(nslots / kXcds);
-        }
+        if (plan_is_split(b))
+            if (int rc = set_split_args(ex, b, a)) return rc;
         hipStream_t st = si == 0 ? st0 : ex.aux[si - 1];
         int rc = launch_timed(ex, st, b.kind, b.K, b.grid, b.lds, a, ex.bnd.as<uint32_t>() + b.bnd_at);
         if (rc) return rc;
@@ -974,6 +983,106 @@ int enqueue_job(Exec& ex, const Job& job, const gbsw_scoring* sc, int mode)
     return GBSW_OK;
 }
 
+namespace {
+
+// The pairs in ex.redo again with int32 cells; blocks, and leaves the status words
+// in ex.status_host.
+int redo_int32(Exec& ex, const Job& job, const gbsw_scoring* sc, int64_t count)
+{
+    KernelArgs a = base_args(ex, job, sc);
+    a.order = ex.redo.as<int32_t>();
+    a.order_n = count;
+    a.sat_limit = INT_MAX;
+    BucketPlan b;
+    b.bk.count = count;
+    b.bk.max_cols = job.max_cols;
+    b.bk.max_rows = job.max_rows;
+    std::vector<int16_t> sub;
+    int max_sub = 0;
+    bool p8 = false, f16p8 = false;
+    int rc = prepare_scoring(job, sc, sub, &max_sub, &p8, &f16p8);
+    if (rc) return rc;
+    const SweepChoice sw = sweep_choice(sub, job.alpha, sc->gap_open, sc->gap_extend, max_sub, false);
+    if (sw.wide_ok) {
+        // One pair per wave; few pairs (up to a wave per SIMD) as strips of the split
+        // form: 400 long reads, a few of them past the range, 773 -> 21.5 ms with
+        // the few no longer on one 16-lane group each.  (An int32 step takes about
+        // twice a 16-bit one.)
+        a.base = sw.base;
+        b.G = kWave;
+        auto geometry = [&](int K, bool split) {
+            b.K = K;
+            b.kind = kBatchedWide | kWideGroup | (split ? kSplitStrips : 0);
+            b.strips = std::max(1, (job.max_cols + 2 * kWave * K - 1) / (2 * kWave * K));
+            b.lds = sweep_lds(kWave, K, kProfWords, job.alpha, 8).total;
+        };
+        constexpr int kMost = 4; // widest geometry of the int32 kernels
+        geometry(kMost, false);
+        const bool few = count <= 4 * (int64_t)ex.num_cu;
+        if (few && b.strips > 1 && ex.split && !ex.split_misplaced && !a.asym) {
+            double best = 1e300;
+            int K = kMost;
+            for (int k = 2; k <= kMost; k += 2) {
+                const double strips = std::ceil(job.max_cols / (2.0 * kWave * k));
+                const double t = (job.max_rows + (strips - 1) * split_lag(kWave)) * step_alone(2 * k, true);
+                if (t < best) { best = t; K = k; }
+            }
+            geometry(K, true);
+        }
+    } else {
+        int nk = 0;
+        const int* wk = wide_k_list(&nk);
+        b.K = wk[nk - 1];
+        for (int i = 0; i < nk; ++i)
+            if (kVirtPerPair * wk[i] >= job.max_cols) { b.K = wk[i]; break; }
+        b.kind = with_profile(kBatchedWide, ex.p8);
+        b.lds = lds_for(b.K, job.alpha, ex.p8, 8);
+    }
+    const size_t per_wg = (size_t)b.pairs_per_wave() * (size_t)a.bnd_rows * 8;
+    auto set_grid = [&]() {
+        if (b.kind & kSplitStrips) {
+            const int occ = std::max(1, kernel_occupancy(b.kind, b.K, b.lds));
+            const int64_t busy = (b.sets() + kXcds - 1) / kXcds * b.strips * kXcds;
+            b.grid = (int)std::max<int64_t>(kXcds, std::min<int64_t>((int64_t)occ * ex.num_cu / kXcds * kXcds, busy));
+        } else {
+            b.grid = grid_for(ex, b.kind, b.K, b.lds, b.sets());
+        }
+    };
+    set_grid();
+    if (ex.fixed && (b.kind & kSplitStrips) &&
+        (2 * (size_t)b.grid * per_wg > ex.bnd.bytes || split_words_of(b) * 4 > ex.split_buf.bytes)) {
+        b.kind &= ~kSplitStrips;
+        set_grid();
+    }
+    const bool split = (b.kind & kSplitStrips) != 0;
+    if (ex.fixed && !split && (size_t)b.grid * per_wg > ex.bnd.bytes) {
+        const int cap = (int)std::min<size_t>(ex.bnd.bytes / per_wg, INT_MAX);
+        if (cap < 1) return fail(GBSW_E_RANGE, "int32 boundary rows exceed the preallocated scratch");
+        b.grid = std::min(b.grid, cap);
+    }
+    GBSW_HIP_TRY(ex.bnd.reserve((size_t)(split ? 2 : 1) * b.grid * per_wg));
+    a.queue = ex.queue.as<uint32_t>();
+    GBSW_HIP_TRY(zero_u32(a.queue, kXcds, ex.stream));
+    a.kmax = b.K;
+    a.nranges = 1;
+    a.ranges[0] = {(int32_t)count, b.K};
+    if (split) {
+        GBSW_HIP_TRY(ex.split_buf.reserve(split_words_of(b) * sizeof(uint32_t)));
+        GBSW_HIP_TRY(zero_u32(ex.split_buf.as<uint32_t>(), (int)split_words_of(b), ex.stream));
+        if ((rc = set_split_args(ex, b, a))) return rc;
+    }
+    rc = launch_timed(ex, ex.stream, b.kind, b.K, b.grid, b.lds, a, ex.bnd.ptr);
+    if (rc) return rc;
+    ex.launches.back().pairs = count;
+    GBSW_HIP_TRY(hipMemcpyAsync(ex.status_host.ptr, ex.status.ptr, sizeof(int32_t) * kStatusWords,
+                                hipMemcpyDeviceToHost, ex.stream));
+    GBSW_HIP_TRY(hipEventRecord(ex.ev_stop, ex.stream));
+    GBSW_HIP_TRY(hipEventSynchronize(ex.ev_stop));
+    return GBSW_OK;
+}
+
+} // namespace
+
 int complete_job(Exec& ex, const Job& job, const gbsw_scoring* sc, double* device_ms)
 {
     GBSW_HIP_TRY(hipEventSynchronize(ex.ev_stop));
@@ -991,37 +1100,17 @@ int complete_job(Exec& ex, const Job& job, const gbsw_scoring* sc, double* devic
         return rc;
     }
     if (status[kStatusSaturated] > 0) {
-        // pairs whose int16 score reached the saturation limit: recompute them
+        // pairs whose 16-bit score reached the saturation limit: recompute them
         // (forward + reverse) with int32 cells
-        int nk = 0;
-        const int* wk = wide_k_list(&nk);
-        int K = wk[nk - 1];
-        for (int i = 0; i < nk; ++i)
-            if (kVirtPerPair * wk[i] >= job.max_cols) { K = wk[i]; break; }
-        const int lds = lds_for(K, job.alpha, ex.p8, 8);
-        const int64_t count = status[kStatusSaturated];
-        KernelArgs a = base_args(ex, job, sc);
-        a.order = ex.redo.as<int32_t>();
-        a.order_n = count;
-        a.sat_limit = INT_MAX;
-        a.queue = ex.queue.as<uint32_t>();
-        GBSW_HIP_TRY(zero_u32(a.queue, 1, ex.stream));
-        const int kw = with_profile(kBatchedWide, ex.p8);
-        int grid = grid_for(ex, kw, K, lds, (count + kPairsPerWave - 1) / kPairsPerWave);
-        const size_t per_wg = kPairsPerWave * (size_t)a.bnd_rows * 8;
-        if (ex.fixed && (size_t)grid * per_wg > ex.bnd.bytes) {
-            const int cap = (int)std::min<size_t>(ex.bnd.bytes / per_wg, INT_MAX);
-            if (cap < 1) return fail(GBSW_E_RANGE, "int32 boundary rows exceed the preallocated scratch");
-            grid = std::min(grid, cap);
+        int rc = redo_int32(ex, job, sc, status[kStatusSaturated]);
+        if (!rc && split_rerun_needed(status)) {
+            // (as above: unsplit from now on; the status words of the first try go)
+            ex.split_misplaced = true;
+            GBSW_HIP_TRY(zero_u32(ex.status.as<uint32_t>(), kStatusWords, ex.stream));
+            const int32_t count = status[kStatusSaturated];
+            rc = redo_int32(ex, job, sc, count);
         }
-        GBSW_HIP_TRY(ex.bnd.reserve((size_t)grid * per_wg));
-        int rc = launch_timed(ex, ex.stream, kw, K, grid, lds, a, ex.bnd.ptr);
         if (rc) return rc;
-        ex.launches.back().pairs = count;
-        GBSW_HIP_TRY(hipMemcpyAsync(ex.status_host.ptr, ex.status.ptr, sizeof(int32_t) * kStatusWords,
-                                    hipMemcpyDeviceToHost, ex.stream));
-        GBSW_HIP_TRY(hipEventRecord(ex.ev_stop, ex.stream));
-        GBSW_HIP_TRY(hipEventSynchronize(ex.ev_stop));
         ex.late_results = true;
     }
     float ms = 0.f;

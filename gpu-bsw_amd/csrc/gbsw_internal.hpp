@@ -201,6 +201,7 @@ int wide_grid_cap(const Exec& ex, int alpha);
 // left the 16-bit range.  bytes: the scores may be held as bytes.
 struct SweepChoice {
     bool ok = false;
+    bool wide_ok = false; // the int32 sweep kernels
     int form = 0; // ProfileForm
     int32_t base = 0, sat_limit = 0;
 };

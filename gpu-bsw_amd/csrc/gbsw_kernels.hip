@@ -1064,6 +1064,7 @@ static const void* kernel_for_profile(int kind, int K)
 static const void* kernel_for(int kind, int K)
 {
     const int base = kind & 0xFF;
+    if (base == kBatchedWide && (kind & kWideGroup)) return sweep_kernel_int32(kind, K);
     if (base == kBatchedF16 || base == kSplitF16) {
         const bool wide = (kind & kWideGroup) != 0;
         if (kind & kRegTables) return wide ? sweep_kernel_regs_wide(kind, K) : sweep_kernel_regs(kind, K);

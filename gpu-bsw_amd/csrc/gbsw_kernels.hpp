@@ -46,6 +46,10 @@ const void* sweep_kernel_words(int kind, int K);
 const void* sweep_kernel_regs_wide(int kind, int K);
 const void* sweep_kernel_bytes_wide(int kind, int K);
 const void* sweep_kernel_words_wide(int kind, int K);
+// int32 cells (kBatchedWide | kWideGroup, with kSplitStrips the split form)
+constexpr int kSplitStrips = 0x1000;
+#define GBSW_SWEEP_K32(X) X(2) X(4)
+const void* sweep_kernel_int32(int kind, int K);
 
 bool kernel_supported(int K);
 bool kernel_has(int kind, int K);

@@ -195,6 +195,85 @@ struct Sweep16 {
     __device__ static B zero_bnd() { return 0u; }
 };
 
+// Sweep32: the same two virtual lanes as two int32 registers, for pairs whose score
+// may exceed the 16-bit range.
+struct Sweep32 {
+    struct V {
+        int32_t l, h;
+    };
+    using U = int32_t;
+    using B = uint2; // (H, E)
+    static constexpr bool kWide = true;
+    __device__ static U uni(int32_t x) { return x; }
+    __device__ static V from(U u) { return V{u, u}; }
+    __device__ static V splat(int32_t x) { return V{x, x}; }
+    __device__ static V addu(V a, U u) { return V{a.l + u, a.h + u}; }
+    __device__ static V subu(V a, U u) { return V{a.l - u, a.h - u}; }
+    template <bool SIGNED>
+    __device__ static V add(V a, V b) { return V{a.l + b.l, a.h + b.h}; }
+    __device__ static V vmax(V a, V b) { return V{max(a.l, b.l), max(a.h, b.h)}; }
+    __device__ static V max3(V a, V b, V c) { return V{max(max(a.l, b.l), c.l), max(max(a.h, b.h), c.h)}; }
+    __device__ static V max3u(V a, V b, U c) { return V{max(max(a.l, b.l), c), max(max(a.h, b.h), c)}; }
+    __device__ static V vmax3(V a, V b, V c) { return max3(a, b, c); }
+    template <int G>
+    __device__ static void left(V x, V y, V d, V& xo, V& yo)
+    {
+        uint32_t xl, xh, yl, yh;
+        group_left<G>((uint32_t)x.l, (uint32_t)y.l, (uint32_t)d.l, xl, yl);
+        group_left<G>((uint32_t)x.h, (uint32_t)y.h, (uint32_t)d.h, xh, yh);
+        xo = V{(int32_t)xl, (int32_t)xh};
+        yo = V{(int32_t)yl, (int32_t)yh};
+    }
+    __device__ static V fix_h(V x, B bnd, const GroupFix& f)
+    {
+        return V{f.first ? (int32_t)bnd.x : x.l, f.first ? x.l : x.h};
+    }
+    __device__ static V fix_e(V x, B bnd, const GroupFix& f)
+    {
+        return V{f.first ? (int32_t)bnd.y : x.l, f.first ? x.l : x.h};
+    }
+    __device__ static B bnd_zero(int32_t zh, int32_t ze) { return make_uint2((uint32_t)zh, (uint32_t)ze); }
+    __device__ static B first_bnd(U z, int32_t go) { return bnd_zero(z - go, z); }
+    __device__ static B bnd_add(B b, int32_t zh, int32_t ze) { return make_uint2(b.x + (uint32_t)zh, b.y + (uint32_t)ze); }
+    __device__ static B bnd_sub(B b, int32_t zh, int32_t ze) { return make_uint2(b.x - (uint32_t)zh, b.y - (uint32_t)ze); }
+    __device__ static B bnd_out(V h, V e) { return make_uint2((uint32_t)h.h, (uint32_t)e.h); }
+    __device__ static V bytes(uint32_t w) { return V{(int32_t)(w & 0xFFFFu), (int32_t)(w >> 16)}; }
+    __device__ static V words(const uint32_t* plo, const uint32_t* phi, int k)
+    {
+        const int sh = (k & 1) * 16;
+        return V{(int32_t)(int16_t)(plo[k / 2] >> sh), (int32_t)(int16_t)(phi[k / 2] >> sh)};
+    }
+    __device__ static bool exceeds(V x, V thr) { return x.l > thr.l || x.h > thr.h; }
+    __device__ static V ltmask(V a, V b) { return V{a.l < b.l ? -1 : 0, a.h < b.h ? -1 : 0}; }
+    __device__ static V sel(V m, V a, V b) { return V{m.l ? a.l : b.l, m.h ? a.h : b.h}; }
+    __device__ static V sel_step(V m, int s, V b) { return V{m.l ? s : b.l, m.h ? s : b.h}; }
+    __device__ static V less1(V x) { return V{max(x.l - 1, 0), max(x.h - 1, 0)}; }
+    __device__ static int32_t lo(V x) { return x.l; }
+    __device__ static int32_t hi(V x) { return x.h; }
+    template <int G>
+    __device__ static V group_max(V x)
+    {
+        int32_t m = max(x.l, x.h);
+        m = max(m, (int32_t)row_ror<1>((uint32_t)m));
+        m = max(m, (int32_t)row_ror<2>((uint32_t)m));
+        m = max(m, (int32_t)row_ror<4>((uint32_t)m));
+        m = max(m, (int32_t)row_ror<8>((uint32_t)m));
+        if constexpr (G == 64) {
+            int32_t r = 0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) r = max(r, __builtin_amdgcn_readlane(m, 16 * q));
+            m = r;
+        }
+        return V{m, m};
+    }
+    __device__ static B load_bnd(const B* p)
+    {
+        const uint64_t v = __hip_atomic_load((const uint64_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return make_uint2((uint32_t)v, (uint32_t)(v >> 32));
+    }
+    __device__ static B zero_bnd() { return make_uint2(0u, 0u); }
+};
+
 // Bits 0 .. n - 1 (n clamped to [0, 32]): the columns of a block inside the pair.
 __device__ __forceinline__ uint32_t sweep_cols(int n)
 {
@@ -768,9 +847,10 @@ __device__ __forceinline__ void sweep_set(const KernelArgs& a, const SweepSmem& 
 // queues unevenly loaded: 26.3-27.5 ms against 25.7 ms; 150k pairs 9.4 against 5.0.)
 // WIDE: the four-pair geometries of K >= 10, whose registers leave room for fewer
 // waves.
-constexpr int sweep_group_waves(int G, bool WIDE) { return G == 16 && WIDE ? 3 : 4; }
+template <class A>
+constexpr int sweep_group_waves(int G, bool WIDE) { return A::kWide ? 2 : G == 16 && WIDE ? 3 : 4; }
 template <class A, int G, int PF, bool WIDE>
-__global__ __launch_bounds__(64, sweep_group_waves(G, WIDE)) void k_sweep(KernelArgs a)
+__global__ __launch_bounds__(64, sweep_group_waves<A>(G, WIDE)) void k_sweep(KernelArgs a)
 {
     extern __shared__ __align__(16) uint8_t smem_raw[];
     constexpr int PW = kWave / G;
@@ -790,7 +870,9 @@ __global__ __launch_bounds__(64, sweep_group_waves(G, WIDE)) void k_sweep(Kernel
         for (int r = a.nranges - 1; r >= 0; --r)
             if ((int64_t)q * PW < a.ranges[r].end) K = a.ranges[r].K;
 #define GBSW_CASE(k) case k: sweep_set<A, G, k, PF>(a, sm, p, bnd_g); break;
-        if constexpr (G == kWave) {
+        if constexpr (A::kWide) {
+            switch (K) { GBSW_SWEEP_K32(GBSW_CASE) }
+        } else if constexpr (G == kWave) {
             switch (K) { GBSW_SWEEP_K64(GBSW_CASE) }
         } else if constexpr (WIDE) {
             switch (K) { GBSW_SWEEP_K16_WIDE(GBSW_CASE) }
@@ -808,7 +890,7 @@ __global__ __launch_bounds__(64, sweep_group_waves(G, WIDE)) void k_sweep(Kernel
 // taken from the counter earlier, which holds its workgroup until it finishes,
 // and is bounded by kSpinTicks besides.
 template <class A, int G, int K, int PF>
-__global__ __launch_bounds__(64, K <= 6 ? 4 : 3) void k_sweep_split(KernelArgs a)
+__global__ __launch_bounds__(64, A::kWide ? 2 : K <= 6 ? 4 : 3) void k_sweep_split(KernelArgs a)
 {
     extern __shared__ __align__(16) uint8_t smem_raw[];
     constexpr int PW = kWave / G;
