@@ -150,6 +150,7 @@ struct Sweep16 {
     // the left neighbour's values, less the offset between the two lanes
     template <int G>
     __device__ static void left(V x, V y, V d, V& xo, V& yo) { group_left<G>(x, y, d, xo, yo); }
+    __device__ static void keep(V& x) { asm volatile("" : "+v"(x)); }
     __device__ static V fix_h(V x, B bnd, const GroupFix& f) { return __builtin_amdgcn_perm(x, bnd, f.selh); }
     __device__ static V fix_e(V x, B bnd, const GroupFix& f) { return __builtin_amdgcn_perm(x, bnd, f.sele); }
     // zero-score boundary at offsets zh (H) and ze (E); entries less / plus offsets
@@ -215,6 +216,7 @@ struct Sweep32 {
     __device__ static V max3(V a, V b, V c) { return V{max(max(a.l, b.l), c.l), max(max(a.h, b.h), c.h)}; }
     __device__ static V max3u(V a, V b, U c) { return V{max(max(a.l, b.l), c), max(max(a.h, b.h), c)}; }
     __device__ static V vmax3(V a, V b, V c) { return max3(a, b, c); }
+    __device__ static void keep(V& x) { asm volatile("" : "+v"(x.l), "+v"(x.h)); }
     template <int G>
     __device__ static void left(V x, V y, V d, V& xo, V& yo)
     {
@@ -456,7 +458,9 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
     const int strip_lo = SPLIT ? io.strip : 0;
 
     const U gs = A::uni(ge), cs = A::uni(ge - go), hand_u = A::uni(ge * (K - 1));
-    const V hand = A::from(hand_u);
+    // (opaque: kept in vector registers, where the DPP subtraction takes it)
+    V hand = A::from(hand_u);
+    A::keep(hand);
     const int v_lo = l, v_hi = l + G;
     uint64_t cand_lo = 0, cand_hi = 0;
     // forward: the lane's threshold (true scores); reverse: the score to reach.
@@ -605,14 +609,23 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
                 using Code = std::conditional_t<PF == kProfRegs, uint32_t, uint16_t>;
                 const Code* rc0 = (const Code*)ring_code + ((s0 - (PF == kProfRegs ? v_lo : v_hi)) & (R - 1));
                 const Bd* pb0 = ring_bnd + (s0 & (R - 1));
-                auto fetch = [&](StepIn& in, const Code* rc, const Bd* pb) {
+                // a step's row codes (profile forms: read two steps ahead, the profile
+                // words they address one step ahead)
+                struct Rc {
+                    uint32_t lo, hi;
+                };
+                auto codes = [&](const Code* rc) {
+                    if constexpr (PF == kProfRegs) return Rc{*rc, 0u};
+                    else return Rc{rc[G], rc[0]};
+                };
+                auto fetch = [&](StepIn& in, const Rc c, const Bd* pb) {
                     if constexpr (PF == kProfRegs) {
-                        in.w[0] = *rc;
+                        in.w[0] = c.lo;
                     } else {
                         using P = SweepProf<G, K, PF>;
                         uint32_t wl[P::NW], wh[P::NW];
-                        P::load(gb + rc[G], v_lo, wl);
-                        P::load(gb + rc[0], v_hi, wh);
+                        P::load(gb + c.lo, v_lo, wl);
+                        P::load(gb + c.hi, v_hi, wh);
 #pragma unroll
                         for (int q = 0; q < P::NW; ++q) { in.w[q] = wl[q]; in.w[P::NW + q] = wh[q]; }
                     }
@@ -698,17 +711,20 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
                     // offset of column 0 at step s0; steps past steps_max only meet padding rows
                     U z = A::uni(base + ge * ((s0 & (kRebase - 1)) + 1));
                     StepIn ia, ib;
-                    fetch(ia, rc, pb);
+                    fetch(ia, codes(rc), pb);
+                    Rc cn = codes(rc + 1);
                     for (int s = s0; s < s_end; s += UN) {
                         // a row of the iteration may improve the best (reach the target) only if E
                         // leaving the lane exceeds this: best - o - g (K - 1) at the first step's offset
                         const V thr = A::addu(REV ? tgt1 : bt, z + cs);
 #pragma unroll
                         for (int u = 0; u < UN; u += 2) {
-                            fetch(ib, rc + 1, pb + 1);
+                            fetch(ib, cn, pb + 1);
+                            cn = codes(rc + 2);
                             step(s + u, ia, z, thr);
                             z += gs;
-                            fetch(ia, rc + 2, pb + 2);
+                            fetch(ia, cn, pb + 2);
+                            cn = codes(rc + 3);
                             step(s + u + 1, ib, z, thr);
                             z += gs;
                             rc += 2;
