@@ -359,8 +359,9 @@ SweepChoice sweep_choice(const std::vector<int16_t>& sub, int alpha, int32_t gap
     c.wide_ok = bias >= 1 && lo > -32768 && hi < 32768;
     c.form = (bytes && lo >= 0 && hi <= 255) ? (alpha <= kRegAlpha ? kProfRegs : kProfBytes) : kProfWords;
     // a pair below this never formed a value past 0x7C00 (largest offset, gap step
-    // and one substitution on top of its best)
-    c.sat_limit = (int32_t)(0x7C00 - offset - 2 * ge - max_sub - 4);
+    // and one substitution on top of its best; the strict reverse pass keeps kRevLow
+    // below zero)
+    c.sat_limit = (int32_t)(0x7C00 - kRevLow - offset - 2 * ge - max_sub - 4);
     return c;
 }
 

@@ -209,6 +209,7 @@ __host__ __device__ inline LdsLayout lds_layout(int32_t row_bytes, int32_t alpha
 // align one pair: 2G virtual lanes of K columns, 64/G pairs per wave.
 constexpr int kRegAlpha = 4;   // residue codes a register table holds
 constexpr int kSweepUnroll = 4; // steps per iteration, and the look-ahead of the ring reads
+constexpr int kRevLow = 2048;  // floor of the strict reverse pass, below zero
 constexpr int kRebase = 128;   // steps between two subtractions of the running offset
 // Where a sweep kernel keeps the substitution scores: byte tables in registers,
 // a byte profile or a 16-bit profile in LDS.

@@ -14,6 +14,7 @@ struct Task {
     int32_t nr, nc;           // rows / columns computed
     int32_t nr_full, nc_full; // extents the reversed indices count back from
     int32_t rev;              // 1: both sequences are read backwards (reverse pass)
+    int32_t ubound;           // reverse pass: upper bound of the columns' substitution scores together
 };
 
 __device__ __forceinline__ uint32_t inv_prio(uint32_t p)
@@ -156,6 +157,7 @@ __device__ __forceinline__ Task empty_task(const KernelArgs& a, int rev)
     t.rows = a.ref; t.cols = a.qry;
     t.nr = t.nc = t.nr_full = t.nc_full = 0;
     t.rev = rev;
+    t.ubound = 0;
     return t;
 }
 
@@ -164,6 +166,7 @@ __device__ __forceinline__ Task forward_task(const KernelArgs& a, int64_t p)
     if (p < 0) return empty_task(a, 0);
     Task t;
     t.rev = 0;
+    t.ubound = 0;
     const uint8_t* A = a.ref + a.ref_off[p];
     const uint8_t* B = a.qry + a.qry_off[p];
     const int32_t la = (int32_t)(a.ref_off[p + 1] - a.ref_off[p]);
@@ -242,6 +245,7 @@ __device__ __forceinline__ Task reverse_task(const KernelArgs& a, int64_t p, con
     if (p < 0 || f.score <= 0) return empty_task(a, 1);
     Task t;
     t.rev = 1;
+    t.ubound = ubound;
     const uint8_t* A = a.ref + a.ref_off[p];
     const uint8_t* B = a.qry + a.qry_off[p];
     const bool rev_rows_a = !(f.ref_end < f.query_end);
@@ -276,6 +280,7 @@ __device__ __forceinline__ Task reverse_task_full(const KernelArgs& a, int64_t p
 {
     Task t;
     t.rev = 1;
+    t.ubound = 0;
     const uint8_t* A = a.ref + a.ref_off[p];
     const uint8_t* B = a.qry + a.qry_off[p];
     if (f.ref_end < f.query_end) { t.rows = B; t.nr = f.query_end; t.cols = A; t.nc = f.ref_end; } // 444-451

@@ -45,6 +45,17 @@
 // every 32 steps to one below the best of its whole group (a smaller value cannot
 // win; an equal one still can, by a smaller row).
 //
+// Reverse pass.  Where both passes have the same sequence as rows, every alignment
+// that reaches the target starts on row 0 of the reversed box (the forward winner is
+// the first row with that score) and its partial scores stay positive.  The strict
+// form therefore floors values at -kRevLow instead of zero once all lanes have left
+// the rows before row 0: alignments that start on later rows stay far below, no
+// hit is lost, and none appears (such an alignment is worth at most the target
+// less kRevLow).  Every 32 steps the pass ends if no value in flight is positive and
+// within reach of the target, given what the columns after it can add at most.  (The
+// static row bound of reverse_task alone: 1M-pair DNA mix 25.6 -> 24.4 ms, 10k long
+// proteins, whose box is three times as high as the alignment, 71.9 -> 64.3 ms.)
+//
 // What bounds it: VALU issue (one instruction per SIMD and four cycles, packed or
 // not).  A step of K columns takes 6 K + about 8 instructions and, in the forward
 // pass, 2.5 K + 6 more in the steps that may improve the best.  Measured against the
@@ -133,9 +144,11 @@ struct Sweep16 {
     __device__ static U uni(int32_t x) { return (uint32_t)x * 0x00010001u; }
     __device__ static V from(U u) { return u; }
     __device__ static V splat(int32_t x) { return uni(x); }
+    __device__ static V pair(int32_t lo, int32_t hi) { return pack16(lo, hi); }
     __device__ static V bytes(uint32_t w) { return w; } // scores picked by v_perm, one per half
     __device__ static V addu(V a, U u) { return a + u; }
     __device__ static V subu(V a, U u) { return a - u; }
+    __device__ static V sub_each(V a, U u) { return raw(as_u(a) - as_u(u)); } // no borrow between the halves
     // + scores: 32-bit while they are non-negative, else per half
     template <bool SIGNED>
     __device__ static V add(V a, V b)
@@ -208,8 +221,10 @@ struct Sweep32 {
     __device__ static U uni(int32_t x) { return x; }
     __device__ static V from(U u) { return V{u, u}; }
     __device__ static V splat(int32_t x) { return V{x, x}; }
+    __device__ static V pair(int32_t lo, int32_t hi) { return V{lo, hi}; }
     __device__ static V addu(V a, U u) { return V{a.l + u, a.h + u}; }
     __device__ static V subu(V a, U u) { return V{a.l - u, a.h - u}; }
+    __device__ static V sub_each(V a, U u) { return subu(a, u); }
     template <bool SIGNED>
     __device__ static V add(V a, V b) { return V{a.l + b.l, a.h + b.h}; }
     __device__ static V vmax(V a, V b) { return V{max(a.l, b.l), max(a.h, b.h)}; }
@@ -304,7 +319,8 @@ struct SweepRows {
         for (int i = 0; i < N; ++i) { f.b[i] = kNoRow; f.d[i] = A::zero_bnd(); }
         return f;
     }
-    __device__ static F fetch(const Task& t, int chunk, int l, const typename A::B* bnd, bool use_bnd)
+    // nbnd: boundary rows to read; the others take (none, none)
+    __device__ static F fetch(const Task& t, int chunk, int l, const typename A::B* bnd, int nbnd, int none)
     {
         F f;
 #pragma unroll
@@ -314,7 +330,7 @@ struct SweepRows {
             f.b[i] = v ? (int32_t)t.rows[t.rev ? t.nr_full - 1 - x : x] : kNoRow;
             // the boundary rows were stored by this workgroup during the previous strip,
             // or by another one of its XCD: an agent-scope load hits no stale L1 line
-            f.d[i] = (MS && v && use_bnd) ? A::load_bnd(bnd + x) : A::zero_bnd();
+            f.d[i] = (MS && l < kChunk && x < nbnd) ? A::load_bnd(bnd + x) : A::bnd_zero(none, none);
         }
         return f;
     }
@@ -423,7 +439,7 @@ struct SweepProf {
 // boundary rows in bnd_g.  Winner keys as in gbsw_pass.hpp.
 template <class A, int G, int K, int PF, bool REV, bool SPLIT = false>
 __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem& sm, const Task& t, int32_t target,
-                            typename A::B* bnd_g, const StripIO& io = StripIO{})
+                                            bool strict, typename A::B* bnd_g, const StripIO& io = StripIO{})
 {
     using V = typename A::V;
     using U = typename A::U;
@@ -433,7 +449,9 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
     constexpr int UN = K <= 8 ? kSweepUnroll : 2;
     const int lane = threadIdx.x, g = lane / G, l = lane & (G - 1);
     const int alpha = a.alpha;
-    const int ge = -a.gap_extend, go = -a.gap_open, base = a.base, sbias = ge + go;
+    const int ge = -a.gap_extend, go = -a.gap_open, sbias = ge + go;
+    // offset of the floor (base) and of zero scores (zero)
+    const int base = a.base, low = REV && strict ? kRevLow : 0, zero = base + low;
     const GroupFix fix = group_fix(l);
     uint8_t* gb = sm.group(g);
     uint16_t* ring_code = (uint16_t*)(gb + sm.L.ring_code_off);
@@ -466,6 +484,8 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
     // forward: the lane's threshold (true scores); reverse: the score to reach.
     // Groups without a pair take one that no cell reaches.
     V bt = A::splat(strips_g > strip_lo ? 0 : kUnreached);
+    int ahead = t.ubound;      // reverse: what the columns from the strip's first on can still add
+    int avail = 0x7FFFFFFF;    // boundary rows the strip before left (the rest are dead)
     const int tgt = target > 0 ? target : kUnreached;
     const V tgt1 = A::splat(tgt - 1);
 
@@ -526,17 +546,44 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
         }
         need_rows(2 * kChunk);
 
+        // reverse, strict: the least score (less one) from which a row of the lane may
+        // still reach the target
+        V dead = A::splat(kUnreached);
+        if constexpr (REV) {
+            if (strict) {
+                int own[2] = {0, 0};
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    const int cl = col_code(strip_base + v_lo * K + k), ch = col_code(strip_base + v_hi * K + k);
+                    own[0] += cl >= 0 ? (int)sm.colmax()[cl] : 0;
+                    own[1] += ch >= 0 ? (int)sm.colmax()[ch] : 0;
+                }
+                int sum[2] = {own[0], own[1]}; // inclusive prefix sums over the lanes
+#pragma unroll
+                for (int x = 1; x < G; x <<= 1) {
+                    const int u0 = __shfl_up(sum[0], x, G), u1 = __shfl_up(sum[1], x, G);
+                    if (l >= x) { sum[0] += u0; sum[1] += u1; }
+                }
+                const int all0 = __shfl(sum[0], G - 1, G), all1 = __shfl(sum[1], G - 1, G);
+                if (target > 0 && live) {
+                    const int r0 = ahead - (sum[0] - own[0]), r1 = ahead - all0 - (sum[1] - own[1]);
+                    dead = A::pair(max(0, tgt - 1 - r0), max(0, tgt - 1 - r1));
+                }
+                ahead -= all0 + all1;
+            }
+        }
+
         // state before step 0: zero scores at the offsets of step -1
         V Ho[K], F[K];
         V snap[REV ? 1 : K];
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            Ho[k] = A::from(A::uni(base + ge * k) + cs);
-            F[k] = A::from(A::uni(base));
+            Ho[k] = A::from(A::uni(zero + ge * k) + cs);
+            F[k] = A::from(A::uni(zero));
         }
 #pragma unroll
         for (int k = 0; k < (REV ? 1 : K); ++k) snap[k] = A::from(A::uni(0));
-        V Eout = A::from(A::uni(base + ge * K)), Hd0 = A::from(A::uni(base - go));
+        V Eout = A::from(A::uni(zero + ge * K)), Hd0 = A::from(A::uni(zero - go));
         V bstep = A::from(A::uni(0)); // step of the first row reaching the lane's best
         int32_t rt_lo = 0x7FFFFFFF, rr_lo = 0, rt_hi = 0x7FFFFFFF, rr_hi = 0; // reverse hits
         bool dirty = false; // some lane's best moved since the group's was last shared
@@ -567,15 +614,21 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
             // row ring: 2G padding rows, rows [0, 32) now, [32, 64) in flight
             for (int c = -(VL / kChunk); c < 0; ++c)
                 Rows::store(Rows::none(), c, l, ring_code, ring_bnd, row_tab, base, ge, go);
-            Rows::store(Rows::fetch(t, 0, l, bnd_rd, use_bnd), 0, l, ring_code, ring_bnd, row_tab, base, ge, go);
-            typename Rows::F pf = Rows::fetch(t, 1, l, bnd_rd, use_bnd);
+            // boundary rows to read, and the entry of the first strip's rows (zero
+            // scores; strict: from row 2G on the floor)
+            const int nbnd = use_bnd ? min(avail, t.nr) : 0;
+            auto first_rows = [&](const int chunk) { return !use_bnd && chunk * kChunk < VL ? low : 0; };
+            Rows::store(Rows::fetch(t, 0, l, bnd_rd, nbnd, first_rows(0)), 0, l, ring_code, ring_bnd, row_tab, base, ge, go);
+            typename Rows::F pf = Rows::fetch(t, 1, l, bnd_rd, nbnd, first_rows(1));
+            const int last_in = use_bnd ? min(avail, steps_max) : 0; // live boundary rows enter until then
+            int s_stop = steps_max; // steps run
             for (int s0 = 0; s0 < steps_max; s0 += kChunk) {
                 // refill: rows of chunk (s0/32 + 1) enter the ring, chunk + 2 is requested
                 {
                     const int ck = s0 / kChunk + 1;
                     Rows::store(pf, ck, l, ring_code, ring_bnd, row_tab, base, ge, go);
                     if constexpr (MS) need_rows((ck + 2) * kChunk);
-                    pf = Rows::fetch(t, ck + 1, l, bnd_rd, use_bnd);
+                    pf = Rows::fetch(t, ck + 1, l, bnd_rd, nbnd, first_rows(ck + 1));
                 }
                 __syncthreads();
                 // rows leaving the last virtual lane during the previous chunk
@@ -598,6 +651,19 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
                 if (!REV && dirty) {
                     share_best();
                     dirty = false;
+                }
+                // strict reverse pass: over once no value in flight can reach the target (a
+                // split strip with a successor runs on: its rows are announced one by one)
+                if (REV && strict && s0 >= VL && s0 >= last_in && !(SPLIT && strip + 1 < strips_max)) {
+                    V m = A::vmax(Hd0, Ho[0]);
+#pragma unroll
+                    for (int k = 1; k < K; ++k) m = A::vmax(m, Ho[k]);
+                    // (Hd0 has the smallest offset of them)
+                    const U zd = A::uni(zero + ge * ((s0 & (kRebase - 1)) - 1)) + cs;
+                    if (__ballot(A::exceeds(m, A::addu(dead, zd))) == 0) {
+                        s_stop = s0;
+                        break;
+                    }
                 }
                 const int s_end = min(s0 + kChunk, steps_max);
                 struct StepIn {
@@ -631,9 +697,9 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
                     }
                     if constexpr (MS) in.bnd = *pb;
                 };
-                auto step = [&](const int s, const StepIn& in, const U z, const V thr) {
+                auto step = [&](const int s, const StepIn& in, const U z, const U zf, const V thr) {
                     // left inputs at this lane's column -1 and, for E, column 0
-                    const Bd bnd = MS ? in.bnd : A::first_bnd(z, go);
+                    const Bd bnd = MS ? in.bnd : A::first_bnd(zf, go);
                     V xH, xE;
                     A::template left<G>(Ho[K - 1], Eout, hand, xH, xE);
                     xH = A::fix_h(xH, bnd, fix);
@@ -656,7 +722,7 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
                         Hd = Ho[k];
                         const V H = A::max3(D, E, F[k]);
                         const V ho = A::addu(H, cs);
-                        E = A::max3u(E, ho, z + (U)(k + 1) * gs);
+                        E = A::max3u(E, ho, zf + (U)(k + 1) * gs);
                         F[k] = A::vmax(F[k], ho);
                         Ho[k] = ho;
                     }
@@ -687,7 +753,7 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
                             uint32_t m_lo = 0, m_hi = 0;
 #pragma unroll
                             for (int k = K - 1; k >= 0; --k) {
-                                const V h = A::subu(Ho[k], zc + (U)k * gs);
+                                const V h = A::sub_each(Ho[k], zc + (U)k * gs); // (may be negative)
                                 m_lo = 2 * m_lo + (A::lo(h) == tgt ? 1u : 0u);
                                 m_hi = 2 * m_hi + (A::hi(h) == tgt ? 1u : 0u);
                             }
@@ -709,7 +775,9 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
                     const Code* rc = rc0;
                     const Bd* pb = pb0;
                     // offset of column 0 at step s0; steps past steps_max only meet padding rows
-                    U z = A::uni(base + ge * ((s0 & (kRebase - 1)) + 1));
+                    U z = A::uni(zero + ge * ((s0 & (kRebase - 1)) + 1));
+                    // and that of the floor: zero scores while lanes may still be above row 0
+                    const U down = A::uni(REV && s0 >= VL ? low : 0);
                     StepIn ia, ib;
                     fetch(ia, codes(rc), pb);
                     Rc cn = codes(rc + 1);
@@ -721,11 +789,11 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
                         for (int u = 0; u < UN; u += 2) {
                             fetch(ib, cn, pb + 1);
                             cn = codes(rc + 2);
-                            step(s + u, ia, z, thr);
+                            step(s + u, ia, z, z - down, thr);
                             z += gs;
                             fetch(ia, cn, pb + 2);
                             cn = codes(rc + 3);
-                            step(s + u + 1, ib, z, thr);
+                            step(s + u + 1, ib, z, z - down, thr);
                             z += gs;
                             rc += 2;
                             pb += 2;
@@ -733,17 +801,21 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
                     }
                 }
             }
+            return s_stop;
         };
+        int s_stop;
         if constexpr (G == kWave) {
-            if (multi_strip) chunks(std::true_type{});
-            else chunks(std::false_type{});
+            if (multi_strip) s_stop = chunks(std::true_type{});
+            else s_stop = chunks(std::false_type{});
         } else {
-            chunks(std::false_type{});
+            s_stop = chunks(std::false_type{});
         }
         if (multi_strip) {
-            // the last chunk's rows; complete before the next strip reads them
+            // the last chunk's rows; complete before the next strip reads them (after an
+            // early end the rows below s_stop - (2G - 1) are there, and no others count)
             __syncthreads();
-            flush_bnd(((steps_max - 1) & ~(kChunk - 1)) - (VL - 1));
+            if (s_stop == steps_max) flush_bnd(((steps_max - 1) & ~(kChunk - 1)) - (VL - 1));
+            avail = s_stop == steps_max ? 0x7FFFFFFF : max(0, s_stop - (VL - 1));
             if constexpr (SPLIT) {
                 if (strip + 1 < strips_max) publish_word(io.prog_out, io.epoch_out | 0xFFFFFFFFull);
             } else {
@@ -832,7 +904,7 @@ __device__ __forceinline__ void sweep_set(const KernelArgs& a, const SweepSmem& 
     RevPlan rp;
 #pragma nounroll
     for (int fp = 0;; ++fp) {
-        const PassResult rf = sweep<A, G, K, PF, false>(a, sm, tf, 0, bnd_g);
+        const PassResult rf = sweep<A, G, K, PF, false>(a, sm, tf, 0, false, bnd_g);
         if (fp == 0) {
             f = forward_result<G>(a, p, rf.key);
             rp = reverse_plan<G>(a, sm, p, f);
@@ -843,7 +915,8 @@ __device__ __forceinline__ void sweep_set(const KernelArgs& a, const SweepSmem& 
             break;
         }
     }
-    const PassResult rr = sweep<A, G, K, PF, true>(a, sm, rp.t, rp.target, bnd_g);
+    const bool strict = __ballot(rp.gen || (p >= 0 && f.score > 0 && reverse_swaps(a, p, f))) == 0;
+    const PassResult rr = sweep<A, G, K, PF, true>(a, sm, rp.t, rp.target, strict, bnd_g);
     int32_t rb, qb;
     reverse_result(a, p, f, rp.t, rp.target, rr.key, &rb, &qb);
     if (p >= 0 && l == 0 && f.score >= 0 && !rp.saturated) {
@@ -948,6 +1021,7 @@ __global__ __launch_bounds__(64, A::kWide ? 2 : K <= 6 ? 4 : 3) void k_sweep_spl
 
         Task t;
         FwdOut f{0, 0, 0};
+        bool strict = false;
         if (!rev) {
             t = forward_task(a, p);
         } else {
@@ -956,6 +1030,8 @@ __global__ __launch_bounds__(64, A::kWide ? 2 : K <= 6 ? 4 : 3) void k_sweep_spl
             const uint64_t fk = p >= 0 ? __hip_atomic_load(fkey + ws, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
             f = forward_result<G>(a, p, fk, s == 0);
             t = reverse_task(a, p, f, column_bound<G>(a, sm, p, f));
+            // (from the ends alone: the same for every strip of the set)
+            strict = __ballot(p >= 0 && f.score > 0 && reverse_swaps(a, p, f)) == 0;
             // a pair whose target an earlier strip reached drops out of the rest of its
             // strips, monotonically along them (k_split): strip s > 0 waits for strip
             // s - 1's decision and publishes its own
@@ -985,8 +1061,8 @@ __global__ __launch_bounds__(64, A::kWide ? 2 : K <= 6 ? 4 : 3) void k_sweep_spl
             io.epoch_in = s > 0 ? (uint64_t)((i - 1) / sp.slots) << 32 : 0;
             io.epoch_out = (uint64_t)(i / sp.slots) << 32;
             PassResult r;
-            if (!rev) r = sweep<A, G, K, PF, false, true>(a, sm, t, 0, nullptr, io);
-            else r = sweep<A, G, K, PF, true, true>(a, sm, t, f.score, nullptr, io);
+            if (!rev) r = sweep<A, G, K, PF, false, true>(a, sm, t, 0, false, nullptr, io);
+            else r = sweep<A, G, K, PF, true, true>(a, sm, t, f.score, strict, nullptr, io);
             if (p >= 0 && l == 0 && r.key != 0) atomicMax((unsigned long long*)((rev ? rkey : fkey) + ws), r.key);
         }
         if (s > 0) release(i - 1);          // done with the previous strip's rows
