@@ -57,7 +57,7 @@ struct gbsw_batch {
     bool one_shot = false; // a gbsw_align batch: aligned once, never worth a graph
     bool aligned = false;  // results of a gbsw_batch_align are in `out`
     // alignment paths: per-pair tables, run buffers, tightness scratch
-    DeviceBuffer tb_meta, tb_runs, tb_dir, tb_dst, tb_tables;
+    DeviceBuffer tb_meta, tb_temp, tb_runs, tb_dir, tb_dst, tb_tables;
     PinnedBuffer tb_host;
     std::vector<hipEvent_t> tb_events;
     ~gbsw_batch()
@@ -468,114 +468,50 @@ int gbsw_batch_traceback(gbsw_batch* b, const gbsw_scoring* sc, int64_t capacity
         return GBSW_OK;
     }
     hipStream_t st = ctx->ex.stream;
-    // host side in pinned memory, kept with the batch: results (5n int32), then
-    // cap_off (n+1), order (n) and dir_off (n) int64, then run counts (n int32)
-    const size_t hres = sizeof(int32_t) * (size_t)(5 * n), h64 = sizeof(int64_t) * (size_t)(3 * n + 1);
-    GBSW_HIP_TRY(b->tb_host.reserve(hres + h64 + sizeof(int32_t) * (size_t)n));
-    int32_t* res = b->tb_host.as<int32_t>();
-    GBSW_HIP_TRY(hipMemcpyAsync(res, b->out.ptr, hres, hipMemcpyDeviceToHost, st));
-    GBSW_HIP_TRY(hipStreamSynchronize(st));
-    // cells are int32: |values| stay below (rows + columns) x the largest |score|
-    int32_t big = std::max(std::abs(sc->gap_open), std::abs(sc->gap_extend));
-    for (int16_t v : sub) big = std::max<int32_t>(big, std::abs((int32_t)v));
-    // per pair: run capacity (rows + columns) and scratch region
-    constexpr int64_t kTbScratch = (int64_t)4 << 30;
-    int64_t* cap_off = (int64_t*)((uint8_t*)res + hres);
-    int64_t* order = cap_off + n + 1;
-    int64_t* dir_off = order + n;
-    int32_t* nruns = (int32_t*)(dir_off + n);
-    std::vector<int64_t> region((size_t)n);
-    // class of a pair: its stripe count (capped at 127), then its rows in steps of 8
-    // below 2048 and of 128 above (capped): the four pairs of a DP wave run the
-    // largest stripe and row counts of the four, so like pairs go together
-    constexpr int kTbClasses = 128 * 512;
-    std::vector<uint16_t> cls((size_t)n);
-    std::vector<int64_t> cls_count(kTbClasses, 0);
-    cap_off[0] = 0;
-    int64_t max_span = 0; // largest rows + columns of a rectangle
-    for (int64_t p = 0; p < n; ++p) {
-        const bool on = res[(size_t)p] > 0;
-        const int32_t m = on ? res[(size_t)(2 * n + p)] - res[(size_t)(n + p)] : 0;
-        const int32_t w = on ? res[(size_t)(4 * n + p)] - res[(size_t)(3 * n + p)] : 0;
-        if (on && (m <= 0 || w <= 0)) return fail(GBSW_E_INTERNAL, "a pair with a positive score has an empty rectangle");
-        if ((int64_t)(m + w) * big >= ((int64_t)1 << 28)) return fail(GBSW_E_RANGE, "path scores may exceed the int32 cells' range");
-        max_span = std::max<int64_t>(max_span, (int64_t)m + w);
-        cap_off[(size_t)p + 1] = cap_off[(size_t)p] + m + w;
-        region[(size_t)p] = tb_region_bytes(m, w);
-        const int32_t stripes = on ? std::min(127, (w + kTbStripeColumns - 1) / kTbStripeColumns) : 0;
-        const int32_t rows = !on ? 0 : m < 2048 ? m >> 3 : std::min(511, 256 + ((m - 2048) >> 7));
-        const int c = stripes * 512 + rows;
-        cls[(size_t)p] = (uint16_t)c;
-        ++cls_count[(size_t)c];
+    // the int32 cells hold (rows + columns) x the largest |score| below 2^28
+    int64_t big = std::max(std::abs((int64_t)sc->gap_open), std::abs((int64_t)sc->gap_extend));
+    int32_t min_sub = 0;
+    for (int16_t v : sub) {
+        big = std::max<int64_t>(big, std::abs((int32_t)v));
+        min_sub = std::min<int32_t>(min_sub, v);
     }
-    // order: largest classes first (their DP lasts longest; the short ones fill in
-    // behind them), by a counting sort over the classes
-    {
-        std::vector<int64_t> start(kTbClasses);
-        int64_t acc = 0;
-        for (int c = kTbClasses - 1; c >= 0; --c) { start[(size_t)c] = acc; acc += cls_count[(size_t)c]; }
-        for (int64_t p = 0; p < n; ++p) order[(size_t)start[cls[(size_t)p]]++] = p;
-    }
-    // int16 cells when every value stays inside +-32,000: a path value lies within
-    // (rows + columns + 2) x the largest |score| of zero, and each sum formed from
-    // one adds one score more
-    const bool cells16 = (max_span + 4) * big < 32000;
-    // launches in that order: one ends past kTbScratch bytes of scratch (scratch_soft)
-    // once it holds enough waves to fill the GPU twice over (16 per SIMD, against
-    // the DP's seven resident; the largest pairs come first, and a launch of few of
-    // them runs latency-bound; 6, 8, 10, 12, 14 and 16 measured 1,225-1,231, 1,250-
-    // 1,279, 1,271-1,304, 1,277-1,280, 1,301-1,308 and 1,304-1,310 GCUPS on the
-    // 1M-pair DNA mix), at twice that many pairs, and in any case before
-    // scratch_max (or at one pair): 12 GiB, or a third of the free device memory
-    // when less (the scratch of two launches is held at once)
-    size_t free_bytes = 0, total_bytes = 0;
-    if (hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        free_bytes = (size_t)24 << 30;
-    }
-    const int64_t scratch_max =
-        std::max<int64_t>((int64_t)256 << 20, std::min<int64_t>((int64_t)12 << 30, (int64_t)(free_bytes / 3)));
-    const int64_t scratch_soft = std::min(kTbScratch, scratch_max);
-    const int64_t fill_pairs = (int64_t)ctx->num_cu * 4 * 16 * (cells16 ? 8 : 4);
-    std::vector<std::pair<int64_t, int64_t>> launches; // (first position, count)
-    int64_t chunk_first = 0, chunk_bytes = 0, max_chunk = 0;
-    for (int64_t x = 0; x < n; ++x) {
-        const int64_t bytes = region[(size_t)order[(size_t)x]];
-        const int64_t held = x - chunk_first;
-        const bool full = chunk_bytes + bytes > scratch_max ||
-                          (held >= fill_pairs && (chunk_bytes + bytes > scratch_soft || held >= 2 * fill_pairs));
-        if (full && x > chunk_first) {
-            launches.emplace_back(chunk_first, x - chunk_first);
-            max_chunk = std::max(max_chunk, chunk_bytes);
-            chunk_first = x;
-            chunk_bytes = 0;
-        }
-        dir_off[(size_t)x] = chunk_bytes;
-        chunk_bytes += bytes;
-    }
-    launches.emplace_back(chunk_first, n - chunk_first);
-    max_chunk = std::max(max_chunk, chunk_bytes);
-    // device tables: cap_off (n+1), dir_off (n), dst_off (n+1) int64; nruns, path
-    // scores (n) int32; lut and substitution table
-    const size_t meta_bytes = sizeof(int64_t) * (size_t)(4 * n + 2) + sizeof(int32_t) * (size_t)(2 * n);
-    GBSW_HIP_TRY(b->tb_meta.reserve(meta_bytes));
-    GBSW_HIP_TRY(b->tb_runs.reserve(sizeof(uint32_t) * (size_t)std::max<int64_t>(1, cap_off[(size_t)n])));
-    // two scratch halves: the walk of one launch overlaps the DP of the next
-    const size_t half = ((size_t)std::max<int64_t>(8, max_chunk) + 255) & ~(size_t)255;
-    GBSW_HIP_TRY(b->tb_dir.reserve(2 * half));
-    GBSW_HIP_TRY(b->tb_tables.reserve(256 + sizeof(int16_t) * sub.size()));
-    // same order as the host staging: cap_off, order, dir_off (one copy), then dst_off
+    const int64_t go = -(int64_t)sc->gap_open, ge = -(int64_t)sc->gap_extend;
+    // device tables: run capacities and their offsets, offsets of the result (n + 1
+    // int64 each); runs per pair (n + 1), path scores, order and its keys (n int32
+    // each); counts
+    const int64_t n1 = n + 1;
+    GBSW_HIP_TRY(b->tb_meta.reserve(sizeof(int64_t) * (size_t)(3 * n1) + sizeof(int32_t) * (size_t)(n1 + 5 * n) +
+                                    sizeof(TbCounts) + 64));
     int64_t* d_cap = b->tb_meta.as<int64_t>();
-    int64_t* d_order = d_cap + n + 1;
-    int64_t* d_dir_off = d_order + n;
-    int64_t* d_dst_off = d_dir_off + n;
-    int32_t* d_nruns = (int32_t*)(d_dst_off + n + 1);
-    int32_t* d_score = d_nruns + n;
+    int64_t* d_cap_off = d_cap + n1;
+    int64_t* d_dst_off = d_cap_off + n1;
+    int32_t* d_nruns = (int32_t*)(d_dst_off + n1);
+    int32_t* d_score = d_nruns + n1;
+    int32_t* d_vals = d_score + n;
+    int32_t* d_order = d_vals + n;
+    uint32_t* d_keys = (uint32_t*)(d_order + n);
+    uint32_t* d_keys_sorted = d_keys + n;
+    TbCounts* d_counts = (TbCounts*)(d_keys_sorted + n);
+    size_t sort_bytes = 0, scan_bytes = 0, scan32_bytes = 0;
+    GBSW_HIP_TRY(sort_pairs(nullptr, sort_bytes, d_keys, d_keys_sorted, d_vals, d_order, (int)n, kTbKeyBits, st));
+    GBSW_HIP_TRY(tb_scan(nullptr, scan_bytes, d_cap, d_cap_off, n1, st));
+    GBSW_HIP_TRY(tb_scan(nullptr, scan32_bytes, d_nruns, d_dst_off, n1, st));
+    size_t temp_bytes = std::max({sort_bytes, scan_bytes, scan32_bytes, (size_t)16});
+    GBSW_HIP_TRY(b->tb_temp.reserve(temp_bytes));
+    GBSW_HIP_TRY(b->tb_tables.reserve(256 + sizeof(int16_t) * sub.size()));
+    // pinned host memory, kept with the batch: the tables to upload and the counts, later
+    // the result's offsets and the path scores
+    const size_t tables = 256 + sizeof(int16_t) * sub.size();
+    const size_t host_words = sizeof(int64_t) * (size_t)n1 + sizeof(int32_t) * (size_t)n;
+    GBSW_HIP_TRY(b->tb_host.reserve(std::max(host_words, 4096 + sizeof(TbCounts) + sizeof(int64_t))));
+    uint8_t* h_tables = b->tb_host.as<uint8_t>();
+    TbCounts& counts = *(TbCounts*)(h_tables + 4096);
+    int64_t& cap_total = *(int64_t*)(h_tables + 4096 + sizeof(TbCounts));
+    static_assert(sizeof(TbCounts) % 8 == 0, "cap_total is aligned");
+    if (tables > 4096) return fail(GBSW_E_INTERNAL, "residue alphabet too large");
+    std::memcpy(h_tables, b->lut, 256);
+    std::memcpy(h_tables + 256, sub.data(), sizeof(int16_t) * sub.size());
     uint8_t* d_lut = b->tb_tables.as<uint8_t>();
-    int16_t* d_sub = (int16_t*)(d_lut + 256);
-    GBSW_HIP_TRY(hipMemcpyAsync(d_cap, cap_off, sizeof(int64_t) * (size_t)(3 * n + 1), hipMemcpyHostToDevice, st));
-    GBSW_HIP_TRY(hipMemcpyAsync(d_lut, b->lut, 256, hipMemcpyHostToDevice, st));
-    GBSW_HIP_TRY(hipMemcpyAsync(d_sub, sub.data(), sizeof(int16_t) * sub.size(), hipMemcpyHostToDevice, st));
     TbArgs a{};
     a.ref = b->ref.as<uint8_t>();
     a.qry = b->qry.as<uint8_t>();
@@ -584,56 +520,183 @@ int gbsw_batch_traceback(gbsw_batch* b, const gbsw_scoring* sc, int64_t capacity
     a.out = b->out.as<int32_t>();
     a.n = n;
     a.lut = d_lut;
-    a.sub = d_sub;
+    a.sub = (const int16_t*)(d_lut + 256);
     a.alpha = job.alpha;
     a.gap_open = sc->gap_open;
     a.gap_extend = sc->gap_extend;
-    a.dir = b->tb_dir.as<uint8_t>();
-    a.cap_off = d_cap;
-    a.runs = b->tb_runs.as<uint32_t>();
+    a.max_sub = max_sub;
+    a.order = d_order;
+    a.cap_off = d_cap_off;
     a.nruns = d_nruns;
     a.path_score = d_score;
-    a.order = d_order;
-    a.cells16 = cells16 ? 1 : 0;
     Exec& ex = ctx->ex;
-    // Two pipelines, the launches at even and at odd positions, each with its own
-    // scratch half, DP stream and walk stream (the context stream and three
-    // auxiliary ones): launch c's walk waits for its DP, and launch c + 2's DP
-    // (same half) for that walk.  A launch lasts as long as its longest wave (the
-    // largest pairs come first), so the other pipeline's launches fill the GPU
-    // while one runs out its tail.
-    if (int rc = ex.ensure_streams(4)) return rc;
+    constexpr int kTbStreams = 4;
+    if (int rc = ex.ensure_streams(kTbStreams)) return rc;
     GBSW_HIP_TRY(hipEventRecord(ex.ev_start, st));
-    const hipStream_t dp_st[2] = {st, ex.aux[1]}, walk_st[2] = {ex.aux[0], ex.aux[2]};
-    const size_t nev = 2 * launches.size() + 1; // DP c done, walk c done; the tables uploaded
-    while (b->tb_events.size() < nev) {
+    GBSW_HIP_TRY(hipMemcpyAsync(d_lut, h_tables, tables, hipMemcpyHostToDevice, st));
+    GBSW_HIP_TRY(hipMemsetAsync(d_counts, 0, sizeof(TbCounts), st));
+    GBSW_HIP_TRY(tb_keys(a, d_keys, d_vals, d_cap, d_counts, st));
+    GBSW_HIP_TRY(hipMemcpyAsync(&counts, d_counts, sizeof(TbCounts), hipMemcpyDeviceToHost, st));
+    GBSW_HIP_TRY(tb_scan(b->tb_temp.ptr, temp_bytes, d_cap, d_cap_off, n1, st));
+    GBSW_HIP_TRY(hipMemcpyAsync(&cap_total, d_cap_off + n, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    GBSW_HIP_TRY(sort_pairs(b->tb_temp.ptr, temp_bytes, d_keys, d_keys_sorted, d_vals, d_order, (int)n, kTbKeyBits, st));
+    GBSW_HIP_TRY(hipStreamSynchronize(st));
+    if (counts.bad) return fail(GBSW_E_INTERNAL, "a pair with a positive score has an empty rectangle");
+    if ((int64_t)counts.span * big >= ((int64_t)1 << 28))
+        return fail(GBSW_E_RANGE, "path scores may exceed the int32 cells' range");
+    GBSW_HIP_TRY(b->tb_runs.reserve(sizeof(uint32_t) * (size_t)std::max<int64_t>(1, cap_total)));
+    a.runs = b->tb_runs.as<uint32_t>();
+
+    // Substitution scores, biased by o + g: bytes of four times that (in registers for up
+    // to four codes) where they fit, else words.
+    const int64_t lo = min_sub + go + ge, hi = max_sub + go + ge;
+    const int form = lo >= 0 && hi <= 63 ? (job.alpha <= kRegAlpha ? kProfRegs : kProfBytes) : kProfWords;
+    const bool words16 = lo >= -8000 && hi <= 8000;
+    // no 16-bit value is negative: H >= -2 o (all of one sequence, then all of the
+    // other, against gaps), Ho >= H - o, and a diagonal sum adds at least min_sub to Ho
+    const int64_t base = 1 + std::max(3 * go, 2 * go - min_sub);
+    a.base = (int32_t)std::min<int64_t>(base, 1 << 28);
+    // cells of a class: the narrowest that holds its largest value bound
+    auto cells_of = [&](int64_t value) {
+        const int64_t top = value + base + 1;
+        return !words16 || top >= kTbTop16Wide ? kTbCells32 : top >= kTbTop16 ? kTbCells16Wide : kTbCells16;
+    };
+
+    // Launches: stretches of classes, largest first, of one cell type, one group width
+    // and regions that do not differ much, in turn on four streams with a quarter of the
+    // scratch each: the tail of one runs beside the next.  All scratch: at most 12 GiB, or a
+    // third of the free device memory when less (but room for one pair).
+    // (12 waves per CU: 8, 12 and 16 took 4.84, 4.43 and 4.38 ms for 300k pairs of the DNA
+    // mix, 15.5, 14.3 and 14.1 for a million, and scratch is per wave.  One stream less
+    // than needed is worse: on two the 300k pairs took 5.4 ms.)
+    struct Launch {
+        int cells, G, kmax, grid, lds;
+        int64_t p0, count, region;
+    };
+    size_t free_bytes = 0, total_bytes = 0;
+    if (hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        free_bytes = (size_t)24 << 30;
+    }
+    free_bytes += b->tb_dir.bytes;
+    const int64_t part_max =
+        std::max<int64_t>((int64_t)64 << 20, std::min<int64_t>((int64_t)3 << 30, (int64_t)(free_bytes / 12)));
+    // 64 lanes per two pairs take more steps in all than 16 per two (a stripe's
+    // anti-diagonals are longer) but a quarter of the time of each: the classes from
+    // `wide_from` on use them, where that makes the sum per SIMD or the longest set,
+    // whichever is larger, least.  A lone wave issues at about half a SIMD's rate.
+    int wide_from = kTbAreas;
+    {
+        const double simds = 4.0 * ctx->num_cu;
+        double best = 1e300, work64 = 0.0, work16 = 0.0, long64 = 0.0;
+        std::vector<double> w16(kTbAreas), w64(kTbAreas), l16(kTbAreas + 1, 0.0), l64(kTbAreas);
+        for (int c = 0; c < kTbAreas; ++c) {
+            const double k = counts.pairs[c];
+            const int kmax = tb_kmax(cells_of(counts.value[c]), form);
+            // a class spans a factor of two in area: its mean lies near 0.7 of the largest
+            const double s16 = k ? tb_set_cost((int)counts.rows[c], (int)counts.cols[c], 16, kmax) : 0.0;
+            const double s64 = k ? tb_set_cost((int)counts.rows[c], (int)counts.cols[c], 64, kmax) : 0.0;
+            w16[c] = std::ceil(k / 8) * s16;
+            w64[c] = std::ceil(k / 2) * s64;
+            l16[c + 1] = std::max(l16[c], s16);
+            l64[c] = s64;
+            work16 += w16[c];
+        }
+        for (int x = kTbAreas; x >= 0; --x) { // classes x and up with 64 lanes
+            if (x < kTbAreas) {
+                work64 += w64[x];
+                work16 -= w16[x];
+                long64 = std::max(long64, l64[x]);
+            }
+            const double t = std::max((work64 + work16) / simds, 2.0 * std::max(long64, l16[x])) +
+                             0.25 * (work64 + work16) / simds;
+            if (t < best * 0.999) {
+                best = t;
+                wide_from = x;
+            }
+        }
+    }
+    std::vector<Launch> launches;
+    int64_t part_bytes[kTbStreams] = {};
+    {
+        int64_t at = 0;
+        uint32_t top_value[kTbAreas]; // largest bound of a class and those below it
+        for (int c = 0; c < kTbAreas; ++c) top_value[c] = std::max(counts.value[c], c ? top_value[c - 1] : 0u);
+        for (int c = kTbAreas - 1; c >= 0;) {
+            if (!counts.pairs[c]) {
+                --c;
+                continue;
+            }
+            Launch L{};
+            L.cells = cells_of(top_value[c]);
+            L.G = c >= wide_from ? 64 : 16;
+            L.kmax = tb_kmax(L.cells, form);
+            L.p0 = at;
+            L.lds = tb_lds_bytes(L.cells, L.G, form, L.kmax, job.alpha);
+            const int64_t slots =
+                (int64_t)ctx->num_cu * std::min(12, tb_occupancy(L.cells, L.G, form, L.lds));
+            const int np = 2 * (64 / L.G);
+            auto region_of = [&](int x) { // room for a set of the class, if that is not out of proportion
+                const int64_t one = (int64_t)counts.scratch[L.G == 64][x] << 8;
+                const int64_t set =
+                    tb_region_bytes((int)counts.rows[x], (int)counts.cols[x], L.G, L.kmax, L.cells, np / 2);
+                return (std::max(one, std::min({set, np * one, part_max})) + 255) & ~(int64_t)255;
+            };
+            const int64_t first = region_of(c);
+            const bool last = launches.size() + 1 == kTbLaunches;
+            for (; c >= 0; --c) {
+                if (!counts.pairs[c]) continue;
+                const int64_t r = region_of(c);
+                if (L.count && !last && (cells_of(top_value[c]) != L.cells || (c >= wide_from ? 64 : 16) != L.G ||
+                                         (2 * r < first && first * slots > part_max / 4)))
+                    break;
+                L.count += counts.pairs[c];
+                L.region = std::max(L.region, r);
+            }
+            at += L.count;
+            const int64_t sets = (L.count + np - 1) / np;
+            L.grid = (int)std::max<int64_t>(1, std::min({slots, sets, part_max / L.region}));
+            int64_t& part = part_bytes[launches.size() % kTbStreams];
+            part = std::max(part, L.region * L.grid);
+            launches.push_back(L);
+        }
+    }
+    int64_t part_at[kTbStreams + 1] = {};
+    for (int x = 0; x < kTbStreams; ++x) part_at[x + 1] = part_at[x] + part_bytes[x];
+    GBSW_HIP_TRY(b->tb_dir.reserve((size_t)std::max<int64_t>(256, part_at[kTbStreams])));
+    while (b->tb_events.size() < kTbStreams) {
         hipEvent_t e;
         GBSW_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         b->tb_events.push_back(e);
     }
-    hipEvent_t uploaded = b->tb_events[nev - 1];
-    GBSW_HIP_TRY(hipEventRecord(uploaded, st));
-    for (int x = 0; x < 3; ++x) GBSW_HIP_TRY(hipStreamWaitEvent(ex.aux[x], uploaded, 0));
+    const int streams = (int)std::min<size_t>(launches.size(), kTbStreams);
+    if (streams > 1) GBSW_HIP_TRY(hipEventRecord(b->tb_events[0], st));
+    for (int x = 1; x < streams; ++x) GBSW_HIP_TRY(hipStreamWaitEvent(ex.aux[x - 1], b->tb_events[0], 0));
     for (size_t c = 0; c < launches.size(); ++c) {
-        const size_t h = c & 1;
-        a.p0 = launches[c].first;
-        a.dir_off = d_dir_off + launches[c].first;
-        a.dir = b->tb_dir.as<uint8_t>() + h * half;
-        if (c >= 2) GBSW_HIP_TRY(hipStreamWaitEvent(dp_st[h], b->tb_events[2 * (c - 2) + 1], 0));
-        GBSW_HIP_TRY(tb_launch_dp(a, launches[c].second, dp_st[h]));
-        GBSW_HIP_TRY(hipEventRecord(b->tb_events[2 * c], dp_st[h]));
-        GBSW_HIP_TRY(hipStreamWaitEvent(walk_st[h], b->tb_events[2 * c], 0));
-        GBSW_HIP_TRY(tb_launch_walk(a, launches[c].second, walk_st[h]));
-        GBSW_HIP_TRY(hipEventRecord(b->tb_events[2 * c + 1], walk_st[h]));
+        const Launch& L = launches[c];
+        const int x = (int)(c % kTbStreams);
+        a.p0 = L.p0;
+        a.count = L.count;
+        a.kmax = L.kmax;
+        a.region_bytes = L.region;
+        a.queue = d_counts->queue + c;
+        a.dir = b->tb_dir.as<uint8_t>() + part_at[x];
+        GBSW_HIP_TRY(tb_launch(a, L.cells, L.G, form, L.grid, L.lds, x ? ex.aux[x - 1] : st));
     }
-    for (size_t c = launches.size() >= 2 ? launches.size() - 2 : 0; c < launches.size(); ++c)
-        GBSW_HIP_TRY(hipStreamWaitEvent(st, b->tb_events[2 * c + 1], 0));
+    for (int x = 1; x < streams; ++x) {
+        GBSW_HIP_TRY(hipEventRecord(b->tb_events[x], ex.aux[x - 1]));
+        GBSW_HIP_TRY(hipStreamWaitEvent(st, b->tb_events[x], 0));
+    }
+    GBSW_HIP_TRY(tb_scan(b->tb_temp.ptr, temp_bytes, d_nruns, d_dst_off, n1, st));
     GBSW_HIP_TRY(hipEventRecord(ex.ev_stop, st)); // device_ms: the path kernels
-    GBSW_HIP_TRY(hipMemcpyAsync(nruns, d_nruns, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToHost, st));
+    int64_t* h_off = b->tb_host.as<int64_t>();
+    int32_t* h_score = (int32_t*)(h_off + n1);
+    GBSW_HIP_TRY(hipMemcpyAsync(h_off, d_dst_off, sizeof(int64_t) * (size_t)n1, hipMemcpyDeviceToHost, st));
     if (path_score)
-        GBSW_HIP_TRY(hipMemcpyAsync(path_score, d_score, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToHost, st));
+        GBSW_HIP_TRY(hipMemcpyAsync(h_score, d_score, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToHost, st));
     GBSW_HIP_TRY(hipStreamSynchronize(st));
-    for (int64_t p = 0; p < n; ++p) cigar_offsets[p + 1] = cigar_offsets[p] + nruns[p];
+    std::memcpy(cigar_offsets, h_off, sizeof(int64_t) * (size_t)n1);
+    if (path_score) std::memcpy(path_score, h_score, sizeof(int32_t) * (size_t)n);
     const int64_t total = cigar_offsets[n];
     if (device_ms) {
         float ms = 0.f;
@@ -645,10 +708,7 @@ int gbsw_batch_traceback(gbsw_batch* b, const gbsw_scoring* sc, int64_t capacity
                                       " words needed (cigar_offsets holds the layout)");
     }
     GBSW_HIP_TRY(b->tb_dst.reserve(sizeof(uint32_t) * (size_t)std::max<int64_t>(1, total)));
-    // the offsets through pinned memory (the order and dir_off staging is free now)
-    std::memcpy(order, cigar_offsets, sizeof(int64_t) * (size_t)(n + 1));
-    GBSW_HIP_TRY(hipMemcpyAsync(d_dst_off, order, sizeof(int64_t) * (size_t)(n + 1), hipMemcpyHostToDevice, st));
-    GBSW_HIP_TRY(tb_compact(a.runs, d_cap, d_nruns, d_dst_off, b->tb_dst.as<uint32_t>(), n, st));
+    GBSW_HIP_TRY(tb_compact(a.runs, d_cap_off, d_nruns, d_dst_off, b->tb_dst.as<uint32_t>(), n, st));
     if (total)
         GBSW_HIP_TRY(hipMemcpyAsync(cigar, b->tb_dst.ptr, sizeof(uint32_t) * (size_t)total, hipMemcpyDeviceToHost, st));
     GBSW_HIP_TRY(hipStreamSynchronize(st));

@@ -92,24 +92,46 @@ struct TbArgs {
     const int16_t* sub;     // alpha x alpha, s(row code, column code)
     int32_t alpha;
     int32_t gap_open, gap_extend;
-    int64_t p0;             // first position of the launch in `order`
-    const int64_t* order;   // pairs by position (longest first)
-    const int64_t* dir_off; // per position of the launch: byte offset of its region in dir
-    uint8_t* dir;           // tightness bytes and boundary columns of the launch's pairs
+    int32_t max_sub;        // largest substitution score, at least 0
+    int32_t base;           // added to every 16-bit cell value (none is negative then)
+    int32_t kmax;           // most columns per lane (tb_kmax)
+    const int32_t* order;   // pairs by position, largest first
+    int64_t p0, count;      // the launch's positions
+    uint32_t* queue;        // sets taken (0 at launch)
+    uint8_t* dir;           // scratch of region_bytes per workgroup: path bits, boundary columns
+    int64_t region_bytes;
     const int64_t* cap_off; // per pair: offset of its run capacity (rows + columns) in runs
     uint32_t* runs;         // run-length ops, last run first
-    int32_t* nruns;         // per pair: runs written
+    int32_t* nruns;         // per pair: runs written (n + 1 entries, the last 0)
     int32_t* path_score;    // per pair: score of the path
-    int32_t cells16;        // 1: every path value fits int16 (k_tb_dp16), 0: int32 cells (k_tb_dp)
 };
-// Columns of one stripe of the traceback DP.
-constexpr int kTbStripeColumns = 64;
-// Scratch bytes of a pair with an m x n rectangle (0 when empty).
-int64_t tb_region_bytes(int32_t m, int32_t n);
-// Tightness bytes of the pairs at positions p0 .. p0 + count - 1 of `order`.
-hipError_t tb_launch_dp(const TbArgs& a, int64_t count, hipStream_t stream);
-// Their paths (run-length ops, last run first), from the bytes tb_launch_dp wrote.
-hipError_t tb_launch_walk(const TbArgs& a, int64_t count, hipStream_t stream);
+// Classes of pairs by rows x columns (two per factor of two), and what k_tb_keys finds
+// in each; counters of the launches.
+constexpr int kTbAreas = 128, kTbKeyBits = 21, kTbLaunches = 64;
+struct TbCounts {
+    uint32_t pairs[kTbAreas], value[kTbAreas], rows[kTbAreas], cols[kTbAreas];
+    uint32_t scratch[2][kTbAreas]; // of one pair, in 256 bytes (16 and 64 lanes)
+    uint32_t span, bad;            // largest rows + columns; a pair with an empty rectangle
+    uint32_t queue[kTbLaunches];
+};
+// Cells: 16 bits with values below 7,936 (maxima through f16 patterns) or 16,384, 32 bits.
+enum { kTbCells16 = 0, kTbCells16Wide = 1, kTbCells32 = 2 };
+constexpr int64_t kTbTop16 = 7936, kTbTop16Wide = 16384;
+// Columns per lane at most.
+int tb_kmax(int cells, int form);
+// Scratch of a set of `groups` pairs of pairs with rectangles up to rows x cols, in any
+// geometry it may take; the set's work; LDS and resident workgroups of a kernel.
+int64_t tb_region_bytes(int32_t rows, int32_t cols, int G, int kmax, int cells, int groups);
+double tb_set_cost(int32_t rows, int32_t cols, int G, int kmax);
+int tb_lds_bytes(int cells, int G, int form, int kmax, int alpha);
+int tb_occupancy(int cells, int G, int form, int lds);
+// Per pair its order key, index and run capacity; class counts (counts: zero before).
+hipError_t tb_keys(const TbArgs& a, uint32_t* keys, int32_t* vals, int64_t* cap, TbCounts* counts, hipStream_t stream);
+// Paths of the pairs at positions p0 .. p0 + count - 1 of `order`.
+hipError_t tb_launch(const TbArgs& a, int cells, int G, int form, int grid, int lds, hipStream_t stream);
+// Exclusive sums of n entries (temp == nullptr: only the scratch size).
+hipError_t tb_scan(void* temp, size_t& temp_bytes, const int64_t* in, int64_t* out, int64_t n, hipStream_t stream);
+hipError_t tb_scan(void* temp, size_t& temp_bytes, const int32_t* in, int64_t* out, int64_t n, hipStream_t stream);
 // dst[dst_off[p] ...] = runs of pair p in path order.
 hipError_t tb_compact(const uint32_t* runs, const int64_t* cap_off, const int32_t* nruns, const int64_t* dst_off,
                       uint32_t* dst, int64_t n, hipStream_t stream);
