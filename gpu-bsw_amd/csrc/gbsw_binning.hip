@@ -1,11 +1,12 @@
 // gbsw_binning.hip -- device-side length binning of a batch (batched form).
 //
 // Every pair gets a 15-bit key: its length class, longest first (6 bits), then
-// 511 - (longer length / 32) (9 bits, capped).  A stable radix sort of (key, pair
-// index) yields the work order: classes of longer pairs first, inside a class the
-// most rows first (longest-processing-time order for the persistent work queues),
-// so the pairs of a wave have like column and step counts.  The reference has no
-// counterpart: it launches pairs in input order (driver.cpp:176-185).
+// 511 - (longer length / 32) (9 bits, capped).  Sorting (key, pair index) yields the
+// work order: classes of longer pairs first, inside a class the most rows first
+// (longest-processing-time order for the persistent work queues), so the pairs of a
+// wave have like column and step counts.  The order of pairs with one key is open: no
+// result depends on it.  The reference has no counterpart: it launches pairs in input
+// order (driver.cpp:176-185).
 #include <algorithm>
 
 #include <hip/hip_runtime.h>
@@ -16,17 +17,103 @@
 
 namespace gbsw {
 
-__global__ void k_bin_keys(const uint64_t* ref_off, const uint64_t* qry_off, int64_t n, uint32_t* keys, int32_t* vals)
+__device__ __forceinline__ uint32_t sort_key(const PrepareArgs& a, int64_t p)
 {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    const uint32_t la = (uint32_t)(ref_off[p + 1] - ref_off[p]);
-    const uint32_t lb = (uint32_t)(qry_off[p + 1] - qry_off[p]);
+    const uint32_t la = (uint32_t)(a.ref_off[p + 1] - a.ref_off[p]);
+    const uint32_t lb = (uint32_t)(a.qry_off[p + 1] - a.qry_off[p]);
     const uint32_t m = la < lb ? la : lb, M = la < lb ? lb : la;
     const uint32_t c = (uint32_t)(kClasses - 1 - length_class((int)m));
     const uint32_t top = (1u << kRowBits) - 1u, r = M >> 5;
-    keys[p] = (c << kRowBits) | (top - (r < top ? r : top));
-    vals[p] = (int32_t)p;
+    return (c << kRowBits) | (top - (r < top ? r : top));
+}
+
+// Everything a job needs on the device before its kernels, in one launch: the small
+// tables (read from pinned host memory), cleared status words, queues and split
+// bookkeeping by the first `helpers` workgroups; and by the rest
+//  - SMALL, up to kSmallSort pairs: the whole counting sort in one workgroup.  A
+//    counter of 16 bits per key in LDS (51 KB); an atomic add gives a pair its rank
+//    among those of its key, a scan of the counters every key's first place.
+//  - otherwise the keys and pair indices for the radix sort, as far as there are pairs.
+// Bound by latency: for 10,000 pairs the three copies, three clears, key and five sort
+// kernels that did this took 82 us from the first to the alignment's start (graph
+// replay), with launch gaps of 3 to 8 us each; as one launch, 400 us of the 437 us that
+// 10,000 short reads took are left, and 315 of 400 us for a call of one read.
+constexpr int kBins = kClasses << kRowBits;
+constexpr int kSmallThreads = 1024, kSmallEach = kSmallSort / kSmallThreads;
+constexpr int kScanEach = (kBins / 2 + kSmallThreads - 1) / kSmallThreads; // dwords (two counters) per thread
+static_assert((kScanEach & 1) == 1, "an odd stride is free of bank conflicts");
+static_assert(kSmallSort <= 32767, "ranks and places are 16-bit");
+
+template <bool SMALL>
+__global__ __launch_bounds__(SMALL ? kSmallThreads : 256) void k_prepare(PrepareArgs a)
+{
+    constexpr int T = SMALL ? kSmallThreads : 256;
+    const int tid = threadIdx.x, b = blockIdx.x;
+    if (b < a.helpers) {
+        const int64_t step = (int64_t)a.helpers * T;
+        for (int64_t x = (int64_t)b * T + tid; x < a.nsplit; x += step) a.split[x] = 0;
+        if (b > 0) return;
+        for (int x = tid; x < a.nsub; x += T) a.sub[x] = a.h_sub[x];
+        for (int x = tid; x < 256; x += T) a.lut[x] = a.h_lut[x];
+        for (int x = tid; x < a.alpha; x += T) a.colmax[x] = a.h_colmax[x];
+        for (int x = tid; x < a.nstatus; x += T) a.status[x] = 0;
+        for (int x = tid; x < a.nqueue; x += T) a.queue[x] = 0;
+        return;
+    }
+    if constexpr (!SMALL) {
+        const int64_t p = (int64_t)(b - a.helpers) * T + tid;
+        if (p >= a.n) return;
+        a.keys[p] = sort_key(a, p);
+        a.vals[p] = (int32_t)p;
+    } else {
+        __shared__ uint32_t count[kScanEach * kSmallThreads];
+        __shared__ uint32_t wave_sum[kSmallThreads / 64];
+        for (int x = tid; x < kScanEach * kSmallThreads; x += T) count[x] = 0;
+        __syncthreads();
+        const int n = (int)a.n;
+        uint32_t key[kSmallEach]; // key, then rank << 16
+#pragma unroll
+        for (int e = 0; e < kSmallEach; ++e)
+            if (e * T + tid < n) key[e] = sort_key(a, e * T + tid);
+#pragma unroll
+        for (int e = 0; e < kSmallEach; ++e)
+            if (e * T + tid < n) {
+                const int sh = 16 * (int)(key[e] & 1u);
+                const uint32_t old = atomicAdd(&count[key[e] >> 1], 1u << sh);
+                key[e] |= ((old >> sh) & 0xFFFFu) << 16;
+            }
+        __syncthreads();
+        // exclusive sums over the counters
+        uint32_t mine = 0;
+#pragma unroll
+        for (int x = 0; x < kScanEach; ++x) {
+            const uint32_t w = count[tid * kScanEach + x];
+            mine += (w & 0xFFFFu) + (w >> 16);
+        }
+        uint32_t upto = mine;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t v = (uint32_t)__shfl_up((int)upto, o);
+            if ((tid & 63) >= o) upto += v;
+        }
+        if ((tid & 63) == 63) wave_sum[tid >> 6] = upto;
+        __syncthreads();
+        uint32_t at = upto - mine;
+        for (int w = 0; w < (tid >> 6); ++w) at += wave_sum[w];
+#pragma unroll
+        for (int x = 0; x < kScanEach; ++x) {
+            const uint32_t w = count[tid * kScanEach + x];
+            count[tid * kScanEach + x] = at | (at + (w & 0xFFFFu)) << 16;
+            at += (w & 0xFFFFu) + (w >> 16);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < kSmallEach; ++e)
+            if (e * T + tid < n) {
+                const uint32_t k = key[e] & 0xFFFFu;
+                a.order[((count[k >> 1] >> (16 * (k & 1u))) & 0xFFFFu) + (key[e] >> 16)] = e * T + tid;
+            }
+    }
 }
 
 // Which byte values occur in p[0, n): bit b of mask[b / 32].  Each thread reads
@@ -73,11 +160,15 @@ hipError_t byte_presence(const uint8_t* p, uint64_t n, uint32_t* mask, hipStream
     return hipGetLastError();
 }
 
-hipError_t bin_keys(const uint64_t* ref_off, const uint64_t* qry_off, int64_t n, uint32_t* keys, int32_t* vals,
-                    hipStream_t stream)
+hipError_t prepare_job(const PrepareArgs& args, hipStream_t stream)
 {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_bin_keys, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, ref_off, qry_off, n, keys, vals);
+    PrepareArgs a = args;
+    a.helpers = (int32_t)std::max<int64_t>(1, std::min<int64_t>(64, a.nsplit / 8192));
+    if (a.order)
+        hipLaunchKernelGGL(k_prepare<true>, dim3((unsigned)a.helpers + 1), dim3(kSmallThreads), 0, stream, a);
+    else
+        hipLaunchKernelGGL(k_prepare<false>, dim3((unsigned)(a.helpers + (a.keys ? (a.n + 255) / 256 : 0))), dim3(256), 0,
+                           stream, a);
     return hipGetLastError();
 }
 

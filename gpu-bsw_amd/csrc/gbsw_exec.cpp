@@ -137,6 +137,27 @@ int launch_timed(Exec& ex, hipStream_t stream, int kind, int K, int grid, int ld
     return GBSW_OK;
 }
 
+// Tables (staged in pinned memory) and status words; the caller adds the rest.
+PrepareArgs prepare_args(const Exec& ex, const Job& job, size_t sub_bytes)
+{
+    PrepareArgs p{};
+    const uint8_t* th = ex.tables_host.as<uint8_t>();
+    p.n = job.n;
+    p.h_sub = (const int16_t*)th;
+    p.h_lut = th + 2048;
+    p.h_colmax = (const int16_t*)(th + 2304);
+    p.sub = ex.sub.as<int16_t>();
+    p.lut = ex.lut.as<uint8_t>();
+    p.colmax = ex.colmax.as<int16_t>();
+    p.status = ex.status.as<uint32_t>();
+    p.queue = ex.queue.as<uint32_t>();
+    p.split = ex.split_buf.as<uint32_t>();
+    p.nsub = (int32_t)(sub_bytes / sizeof(int16_t));
+    p.alpha = job.alpha;
+    p.nstatus = kStatusWords;
+    return p;
+}
+
 KernelArgs base_args(const Exec& ex, const Job& job, const gbsw_scoring* sc)
 {
     KernelArgs a;
@@ -769,25 +790,30 @@ int set_split_args(const Exec& ex, const BucketPlan& b, KernelArgs& a)
 int record_batched(Exec& ex, const Job& job, KernelArgs a, const std::vector<BucketPlan>& plan, size_t sub_bytes)
 {
     hipStream_t st0 = ex.stream;
-    const uint8_t* th = ex.tables_host.as<uint8_t>();
-    GBSW_HIP_TRY(hipMemcpyAsync(ex.sub.ptr, th, sub_bytes, hipMemcpyHostToDevice, st0));
-    GBSW_HIP_TRY(hipMemcpyAsync(ex.lut.ptr, th + 2048, 256, hipMemcpyHostToDevice, st0));
-    GBSW_HIP_TRY(hipMemcpyAsync(ex.colmax.ptr, th + 2304, sizeof(int16_t) * (size_t)job.alpha, hipMemcpyHostToDevice,
-                                st0));
-    GBSW_HIP_TRY(zero_u32(ex.status.as<uint32_t>(), kStatusWords, st0));
-    // device binning: keys, then a stable radix sort into the work order
-    GBSW_HIP_TRY(bin_keys(job.ref_off, job.qry_off, job.n, job.keys, job.vals, st0));
-    size_t tb = job.sort_temp_bytes;
-    GBSW_HIP_TRY(sort_pairs(job.sort_temp, tb, job.keys, job.keys_sorted, job.vals, job.order, (int)job.n, kSortBits,
-                            st0));
     const size_t nb = plan.size();
-    GBSW_HIP_TRY(zero_u32(ex.queue.as<uint32_t>(), (int)(kXcds * nb), st0));
-    size_t split_words = 0;
+    PrepareArgs pre = prepare_args(ex, job, sub_bytes);
+    pre.ref_off = job.ref_off;
+    pre.qry_off = job.qry_off;
+    pre.nqueue = (int32_t)(kXcds * nb);
     for (const BucketPlan& b : plan)
-        if (plan_is_split(b)) split_words = std::max(split_words, b.split_at + split_words_of(b));
-    if (split_words) GBSW_HIP_TRY(zero_u32(ex.split_buf.as<uint32_t>(), (int)split_words, st0));
-    const int ns = std::max(1, std::min(kAuxStreams + 1, ex.streams));
-    GBSW_HIP_TRY(hipEventRecord(ex.ev_fork, st0));
+        if (plan_is_split(b)) pre.nsplit = std::max(pre.nsplit, (int64_t)(b.split_at + split_words_of(b)));
+    // the work order: up to kSmallSort pairs by one workgroup of the preparing launch
+    // (10k pairs: 57 us less than keys and radix sort from launch to launch); more by a
+    // radix sort on the whole GPU
+    if (job.n <= kSmallSort) {
+        pre.order = job.order;
+    } else {
+        pre.keys = job.keys;
+        pre.vals = job.vals;
+    }
+    GBSW_HIP_TRY(prepare_job(pre, st0));
+    if (pre.keys) {
+        size_t tb = job.sort_temp_bytes;
+        GBSW_HIP_TRY(sort_pairs(job.sort_temp, tb, job.keys, job.keys_sorted, job.vals, job.order, (int)job.n, kSortBits,
+                                st0));
+    }
+    const int ns = std::max(1, std::min({kAuxStreams + 1, ex.streams, (int)nb}));
+    if (ns > 1) GBSW_HIP_TRY(hipEventRecord(ex.ev_fork, st0));
     for (int i = 0; i < ns - 1; ++i) GBSW_HIP_TRY(hipStreamWaitEvent(ex.aux[i], ex.ev_fork, 0));
     // each launch (in the plan's order) goes to the stream with the least estimated
     // work queued so far (its share of the whole GPU, or its longest item): a short
@@ -882,8 +908,8 @@ int enqueue_job(Exec& ex, const Job& job, const gbsw_scoring* sc, int mode)
     for (int c = 0; c < job.alpha; ++c)
         for (int r = 0; r < job.alpha; ++r)
             colmax[(size_t)c] = std::max<int16_t>(colmax[(size_t)c], sub[(size_t)(r * job.alpha + c)]);
-    // small tables through pinned staging (the previous job of this Exec has
-    // completed, so its staging is free): the copies stay asynchronous
+    // small tables in pinned memory, read by the preparing launch (the previous job of
+    // this Exec has completed, so its staging is free)
     uint8_t* th = ex.tables_host.as<uint8_t>();
     std::memcpy(th, sub.data(), sizeof(int16_t) * sub.size());
     std::memcpy(th + 2048, job.lut_host, 256);
@@ -892,10 +918,7 @@ int enqueue_job(Exec& ex, const Job& job, const gbsw_scoring* sc, int mode)
     KernelArgs a = base_args(ex, job, sc);
     if (mode == GBSW_PLAIN) {
         GBSW_HIP_TRY(hipEventRecord(ex.ev_start, st0));
-        GBSW_HIP_TRY(hipMemcpyAsync(ex.sub.ptr, th, sizeof(int16_t) * sub.size(), hipMemcpyHostToDevice, st0));
-        GBSW_HIP_TRY(hipMemcpyAsync(ex.lut.ptr, th + 2048, 256, hipMemcpyHostToDevice, st0));
-        GBSW_HIP_TRY(hipMemcpyAsync(ex.colmax.ptr, th + 2304, sizeof(int16_t) * colmax.size(), hipMemcpyHostToDevice, st0));
-        GBSW_HIP_TRY(zero_u32(ex.status.as<uint32_t>(), kStatusWords, st0));
+        GBSW_HIP_TRY(prepare_job(prepare_args(ex, job, sizeof(int16_t) * sub.size()), st0));
         // one geometry for the whole batch, sized by its longest shorter sequence;
         // with profiles (DNA) the occupancy model's narrower strips cost the long
         // pairs more than the extra waves gain (793 vs 593 GCUPS on the 1M-pair

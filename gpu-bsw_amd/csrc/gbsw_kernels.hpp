@@ -60,8 +60,29 @@ hipError_t kernel_launch(int kind, int K, int grid, int lds_bytes, hipStream_t s
 hipError_t zero_u32(uint32_t* p, int n, hipStream_t stream);
 
 // gbsw_binning.hip
-hipError_t bin_keys(const uint64_t* ref_off, const uint64_t* qry_off, int64_t n, uint32_t* keys, int32_t* vals,
-                    hipStream_t stream);
+// Work of the launch that precedes a job's kernels.
+constexpr int kSmallSort = 16384; // pairs sorted by one workgroup
+struct PrepareArgs {
+    const uint64_t* ref_off;
+    const uint64_t* qry_off;
+    int64_t n;
+    int32_t* order;          // not null: the work order of n <= kSmallSort pairs
+    uint32_t* keys;          // else, not null: sort keys and
+    int32_t* vals;           // pair indices of the n pairs
+    const int16_t* h_sub;    // tables in pinned host memory, and their device copies
+    const uint8_t* h_lut;
+    const int16_t* h_colmax;
+    int16_t* sub;
+    uint8_t* lut;
+    int16_t* colmax;
+    uint32_t* status;        // cleared: status, queues, split bookkeeping
+    uint32_t* queue;
+    uint32_t* split;
+    int64_t nsplit;
+    int32_t nsub, alpha, nstatus, nqueue;
+    int32_t helpers;         // workgroups for tables and clearing (set by prepare_job)
+};
+hipError_t prepare_job(const PrepareArgs& a, hipStream_t stream);
 // OR into mask[8] the set of byte values in p[0, n) (p 16-byte aligned).
 hipError_t byte_presence(const uint8_t* p, uint64_t n, uint32_t* mask, hipStream_t stream);
 hipError_t sort_pairs(void* temp, size_t& temp_bytes, const uint32_t* kin, uint32_t* kout, const int32_t* vin,
