@@ -8,10 +8,13 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "gbsw_internal.hpp"
@@ -41,14 +44,24 @@ struct gbsw_context {
     Exec nx;
     gbsw_batch* nbatch = nullptr;
     std::string nx_error;          // why the allocation-free set-up failed ("" if it did not)
+    // staging of large uploads from pageable memory, shared by the context's batches
+    std::mutex up_mu;
+    PinnedBuffer up_ring;
+    std::vector<hipEvent_t> up_events;
+    ~gbsw_context()
+    {
+        for (hipEvent_t e : up_events) (void)hipEventDestroy(e);
+    }
 };
 
 struct gbsw_batch {
     gbsw_context* ctx = nullptr;
     Job job;
+    DeviceBuffer input;                       // one block: ref_off, qry_off, ref, qry (views)
     DeviceBuffer ref, ref_off, qry, qry_off, out, order;
+    PinnedBuffer stage;                       // a small input block
+    PinnedBuffer results;                     // of a one-shot call
     DeviceBuffer keys, keys_sorted, vals, sort_temp;
-    std::vector<int32_t> len_ref, len_qry;
     uint8_t lut[256];
     uint8_t code_of[24]; // protein: reference code of each residue code present
     gbsw_stats stats{};
@@ -135,10 +148,119 @@ int alphabet_from_mask(int32_t alphabet, const uint32_t* mask, uint8_t* lut, uin
 
 namespace gbsw {
 
+// Device block of a batch's input: byte offsets of its parts.
+struct InputLayout {
+    size_t ref_off, qry_off, ref, qry, total;
+};
+InputLayout input_layout(int64_t n, uint64_t ref_bytes, uint64_t qry_bytes)
+{
+    auto up = [](uint64_t x) { return (size_t)((x + 255) & ~(uint64_t)255); };
+    const uint64_t offs = sizeof(uint64_t) * ((uint64_t)std::max<int64_t>(n, 1) + 1);
+    InputLayout L;
+    L.ref_off = 0;
+    L.qry_off = L.ref_off + up(offs);
+    L.ref = L.qry_off + up(offs);
+    L.qry = L.ref + up(std::max<uint64_t>(ref_bytes, 16));
+    L.total = L.qry + up(std::max<uint64_t>(qry_bytes, 16));
+    return L;
+}
+void input_views(gbsw_batch* b, const InputLayout& L)
+{
+    uint8_t* d = b->input.as<uint8_t>();
+    b->ref_off.view(d + L.ref_off, L.qry_off - L.ref_off);
+    b->qry_off.view(d + L.qry_off, L.ref - L.qry_off);
+    b->ref.view(d + L.ref, L.qry - L.ref);
+    b->qry.view(d + L.qry, L.total - L.qry);
+}
+
+struct HostPart {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+
+// Copy parts to the device.  From pageable memory, large: several threads move pieces
+// into a ring of pinned memory and start each one's transfer, since one thread's copy
+// is slower than the link (100 MB: pinned 1.8 ms, the runtime's pageable copy 3.7 and
+// more for memory it has not pinned before, this 2.4; 2, 4 and 8 MB pieces 2.7, 2.4 and
+// 2.3, two to eight threads alike).  `meanwhile` runs on the calling thread, before it
+// joins in.  Blocks until the sources may be reused.
+constexpr size_t kUpPiece = (size_t)4 << 20;
+constexpr int kUpSlots = 6, kUpThreads = 4;
+template <class F>
+hipError_t upload_large(gbsw_context* ctx, hipStream_t st, const HostPart* parts, int nparts, F&& meanwhile)
+{
+    std::lock_guard<std::mutex> lock(ctx->up_mu);
+    hipError_t e = ctx->up_ring.reserve(kUpPiece * kUpSlots);
+    while (e == hipSuccess && ctx->up_events.size() < (size_t)kUpSlots) {
+        hipEvent_t ev;
+        e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+        if (e == hipSuccess) ctx->up_events.push_back(ev);
+    }
+    if (e != hipSuccess) return e;
+    std::vector<HostPart> pieces;
+    for (int x = 0; x < nparts; ++x)
+        for (size_t at = 0; at < parts[x].bytes; at += kUpPiece)
+            pieces.push_back({(uint8_t*)parts[x].dst + at, (const uint8_t*)parts[x].src + at,
+                              std::min(kUpPiece, parts[x].bytes - at)});
+    std::atomic<size_t> next{0};
+    std::atomic<int> error{(int)hipSuccess};
+    std::atomic<size_t> started[kUpSlots]; // pieces whose transfer from the slot has been started
+    for (auto& v : started) v.store(0);
+    uint8_t* ring = ctx->up_ring.as<uint8_t>();
+    auto work = [&]() {
+        hipError_t me = hipSetDevice(ctx->device);
+        for (;;) {
+            const size_t c = next.fetch_add(1);
+            if (c >= pieces.size()) break;
+            const size_t slot = c % kUpSlots, turn = c / kUpSlots;
+            // the slot's previous piece: its transfer started (by the thread that holds
+            // it, before that thread takes another) and done
+            while (started[slot].load(std::memory_order_acquire) < turn) std::this_thread::yield();
+            if (me == hipSuccess && turn > 0) me = hipEventSynchronize(ctx->up_events[slot]);
+            if (me == hipSuccess && error.load() == (int)hipSuccess) {
+                std::memcpy(ring + slot * kUpPiece, pieces[c].src, pieces[c].bytes);
+                me = hipMemcpyAsync(pieces[c].dst, ring + slot * kUpPiece, pieces[c].bytes, hipMemcpyHostToDevice, st);
+                if (me == hipSuccess) me = hipEventRecord(ctx->up_events[slot], st);
+            }
+            if (me != hipSuccess) error.store((int)me);
+            started[slot].store(turn + 1, std::memory_order_release);
+        }
+    };
+    std::vector<std::thread> helpers;
+    const int want = (int)std::min<size_t>({(size_t)kUpThreads, pieces.size(),
+                                            std::max<size_t>(1, std::thread::hardware_concurrency() / 2)});
+    try {
+        for (int x = 1; x < want; ++x) helpers.emplace_back(work);
+    } catch (...) { // fewer threads, then
+    }
+    meanwhile();
+    work();
+    for (std::thread& t : helpers) t.join();
+    const hipError_t se = hipStreamSynchronize(st); // the ring is free again
+    return error.load() != (int)hipSuccess ? (hipError_t)error.load() : se;
+}
+
+bool is_pinned(const void* p)
+{
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return at.type == hipMemoryTypeHost;
+}
+
 // Upload pairs into batch b (new, or one reused: its device buffers only grow),
-// with ex's stream and geometry model.
-static int batch_fill(gbsw_batch* b, gbsw_context* ctx, Exec& ex, int32_t alphabet, int64_t n, const char* ref,
-                      const uint64_t* ref_off, const char* query, const uint64_t* query_off)
+// with ex's stream and geometry model.  `staged` (not for the allocation-free entry
+// point): through pinned staging; a block of up to kUpStaged bytes is then one
+// transfer, and may still be under way on ex.stream on return.
+constexpr size_t kUpStaged = (size_t)1 << 20, kUpLarge = (size_t)8 << 20;
+// Residues whose set of byte values the host finds (about a byte per cycle: 20 us at
+// most); more are scanned on the device, which costs a launch and a wait (about 30 us).
+constexpr uint64_t kHostScan = 65536;
+static int batch_fill(gbsw_batch* b, gbsw_context* ctx, Exec& ex, bool staged, int32_t alphabet, int64_t n,
+                      const char* ref, const uint64_t* ref_off, const char* query, const uint64_t* query_off)
 {
     if (!ctx || n < 0 || (n > 0 && (!ref_off || !query_off)))
         return fail(GBSW_E_ARGUMENT, "null argument or negative pair count");
@@ -158,26 +280,16 @@ static int batch_fill(gbsw_batch* b, gbsw_context* ctx, Exec& ex, int32_t alphab
     Job& job = b->job;
     job.alphabet = alphabet;
     job.n = n;
-    b->len_ref.resize((size_t)n);
-    b->len_qry.resize((size_t)n);
-    std::vector<uint64_t> ro((size_t)n + 1), qo((size_t)n + 1);
-    for (int64_t p = 0; p <= n; ++p) {
-        ro[(size_t)p] = n ? ref_off[p] - ref_off[0] : 0;
-        qo[(size_t)p] = n ? query_off[p] - query_off[0] : 0;
+    bool valid = true;
+    for (int64_t p = 0; p < n; ++p) { // (a decreasing offset gives a huge length)
+        const uint64_t lr = ref_off[p + 1] - ref_off[p], lq = query_off[p + 1] - query_off[p];
+        valid &= (lr <= 65000) & (lq <= 65000);
     }
-    for (int64_t p = 0; p < n; ++p) {
-        if (ro[(size_t)p + 1] < ro[(size_t)p] || qo[(size_t)p + 1] < qo[(size_t)p]) {
+    for (int64_t p = 0; !valid && p < n; ++p) {
+        if (ref_off[p + 1] < ref_off[p] || query_off[p + 1] < query_off[p])
             return fail(GBSW_E_ARGUMENT, "offsets must be non-decreasing");
-        }
-        const uint64_t lr = ro[(size_t)p + 1] - ro[(size_t)p], lq = qo[(size_t)p + 1] - qo[(size_t)p];
-        if (lr > 65000 || lq > 65000) {
+        if (ref_off[p + 1] - ref_off[p] > 65000 || query_off[p + 1] - query_off[p] > 65000)
             return fail(GBSW_E_RANGE, "sequences longer than 65000 residues are not supported");
-        }
-        b->len_ref[(size_t)p] = (int32_t)lr;
-        b->len_qry[(size_t)p] = (int32_t)lq;
-        job.max_rows = std::max<int32_t>(job.max_rows, (int32_t)std::max(lr, lq));
-        job.max_cols = std::max<int32_t>(job.max_cols, (int32_t)std::min(lr, lq));
-        job.cells += (int64_t)(lr * lq);
     }
     const uint8_t* rp = (const uint8_t*)ref + (n ? ref_off[0] : 0);
     const uint8_t* qp = (const uint8_t*)query + (n ? query_off[0] : 0);
@@ -187,44 +299,97 @@ static int batch_fill(gbsw_batch* b, gbsw_context* ctx, Exec& ex, int32_t alphab
     int rc = sort_scratch_bytes(n, &sort_bytes);
     if (rc) return rc;
     const size_t np = (size_t)std::max<int64_t>(n, 1);
-    hipError_t e = b->ref.reserve(std::max<uint64_t>(ref_bytes, 16));
-    if (e == hipSuccess) e = b->qry.reserve(std::max<uint64_t>(qry_bytes, 16));
-    if (e == hipSuccess) e = b->ref_off.reserve(sizeof(uint64_t) * (np + 1));
-    if (e == hipSuccess) e = b->qry_off.reserve(sizeof(uint64_t) * (np + 1));
+    const InputLayout L = input_layout(n, ref_bytes, qry_bytes);
+    hipStream_t st = ex.stream;
+    hipError_t e = b->input.reserve(L.total);
+    if (e == hipSuccess) input_views(b, L);
     if (e == hipSuccess) e = b->out.reserve(sizeof(int32_t) * 5 * np);
     if (e == hipSuccess) e = b->keys.reserve(std::max<size_t>(4 * np, 32));
     if (e == hipSuccess) e = b->keys_sorted.reserve(4 * np);
     if (e == hipSuccess) e = b->vals.reserve(4 * np);
     if (e == hipSuccess) e = b->order.reserve(4 * np);
     if (e == hipSuccess) e = b->sort_temp.reserve(sort_bytes);
-    if (e == hipSuccess && ref_bytes) e = hipMemcpy(b->ref.ptr, rp, ref_bytes, hipMemcpyHostToDevice);
-    if (e == hipSuccess && qry_bytes) e = hipMemcpy(b->qry.ptr, qp, qry_bytes, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(b->ref_off.ptr, ro.data(), sizeof(uint64_t) * (size_t)(n + 1), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(b->qry_off.ptr, qo.data(), sizeof(uint64_t) * (size_t)(n + 1), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemset(b->out.ptr, 0, sizeof(int32_t) * 5 * np);
-    // The residue codes need the set of byte values in the batch (every distinct
-    // DNA byte is a code; protein bytes must be < 91): a scan of the uploaded
-    // bytes on the device instead of a pass over them on the host.
-    uint32_t seen[8] = {0};
-    if (e == hipSuccess) {
-        hipStream_t st = ex.stream;
-        uint32_t* dmask = b->keys.as<uint32_t>();
-        e = zero_u32(dmask, 8, st);
-        if (e == hipSuccess) e = byte_presence(b->ref.as<uint8_t>(), ref_bytes, dmask, st);
-        if (e == hipSuccess) e = byte_presence(b->qry.as<uint8_t>(), qry_bytes, dmask, st);
-        if (e == hipSuccess) e = hipMemcpyAsync(seen, dmask, sizeof(seen), hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
+    const bool one_block = staged && L.total <= kUpStaged;
+    const bool pinned_offs = staged && b->one_shot; // (kept for the next call)
+    const size_t offs_bytes = L.ref - L.ref_off;
+    const size_t masks_at = one_block ? L.total : pinned_offs ? offs_bytes : 0, masks_bytes = 32 * kPresenceBlocks;
+    if (e == hipSuccess && staged) e = b->stage.reserve(masks_at + masks_bytes);
+    std::vector<uint64_t> offs;
+    uint8_t* h = b->stage.as<uint8_t>();
+    if (e == hipSuccess && !one_block && !pinned_offs) {
+        offs.resize(offs_bytes / sizeof(uint64_t));
+        h = (uint8_t*)offs.data();
     }
-    if (e != hipSuccess)
+    job.buckets.reserve(kClasses); // (no allocation beside running threads)
+    // what takes a pass over the pairs: offsets from 0, classes
+    auto pairs_pass = [&]() {
+        uint64_t *ro = (uint64_t*)(h + L.ref_off), *qo = (uint64_t*)(h + L.qry_off);
+        Bucket classes[kClasses];
+        ro[0] = qo[0] = 0;
+        for (int64_t p = 0; p < n; ++p) {
+            const uint64_t lr = ref_off[p + 1] - ref_off[p], lq = query_off[p + 1] - query_off[p];
+            ro[p + 1] = ro[p] + lr;
+            qo[p + 1] = qo[p] + lq;
+            const int32_t rows = (int32_t)std::max(lr, lq), cols = (int32_t)std::min(lr, lq);
+            job.max_rows = std::max(job.max_rows, rows);
+            job.max_cols = std::max(job.max_cols, cols);
+            job.cells += (int64_t)(lr * lq);
+            classes[length_class(cols)].add(cols, rows);
+        }
+        place_buckets(job, classes);
+    };
+    if (e == hipSuccess) e = hipMemsetAsync(b->out.ptr, 0, sizeof(int32_t) * 5 * np, st);
+    uint8_t* dev = b->input.as<uint8_t>();
+    const HostPart parts[2] = {{dev + L.ref, rp, ref_bytes}, {dev + L.qry, qp, qry_bytes}};
+    if (e == hipSuccess) {
+        if (one_block) {
+            pairs_pass();
+            if (ref_bytes) std::memcpy(h + L.ref, rp, ref_bytes);
+            if (qry_bytes) std::memcpy(h + L.qry, qp, qry_bytes);
+            e = hipMemcpyAsync(dev, h, L.qry + qry_bytes, hipMemcpyHostToDevice, st);
+        } else {
+            if (staged && L.total >= kUpLarge && !(ref_bytes && is_pinned(rp)) && !(qry_bytes && is_pinned(qp))) {
+                e = upload_large(ctx, st, parts, 2, pairs_pass);
+            } else {
+                for (const HostPart& x : parts)
+                    if (e == hipSuccess && x.bytes) e = hipMemcpyAsync(x.dst, x.src, x.bytes, hipMemcpyHostToDevice, st);
+                pairs_pass();
+            }
+            if (e == hipSuccess) e = hipMemcpyAsync(dev, h, offs_bytes, hipMemcpyHostToDevice, st);
+            if (e == hipSuccess) e = hipStreamSynchronize(st);
+        }
+    }
+    // The residue codes need the set of byte values in the batch (every distinct
+    // DNA byte is a code; protein bytes must be < 91).
+    uint32_t seen[8] = {0};
+    if (e == hipSuccess && ref_bytes + qry_bytes <= kHostScan) {
+        uint8_t has[256] = {0};
+        for (uint64_t x = 0; x < ref_bytes; ++x) has[rp[x]] = 1;
+        for (uint64_t x = 0; x < qry_bytes; ++x) has[qp[x]] = 1;
+        for (int x = 0; x < 256; ++x) seen[x >> 5] |= (uint32_t)has[x] << (x & 31);
+    } else if (e == hipSuccess) {
+        // one mask per workgroup, in pinned memory
+        uint32_t* masks = (uint32_t*)(staged ? b->stage.as<uint8_t>() + masks_at : ex.tables_host.as<uint8_t>());
+        std::memset(masks, 0, masks_bytes);
+        e = byte_presence(b->ref.as<uint8_t>(), ref_bytes, b->qry.as<uint8_t>(), qry_bytes, masks, st);
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
+        for (int x = 0; x < 8 * kPresenceBlocks; ++x) seen[x & 7] |= masks[x];
+    }
+    if (e == hipSuccess && one_block && !b->one_shot) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) {
+        (void)hipStreamSynchronize(st);
         return fail(e == hipErrorOutOfMemory ? GBSW_E_MEMORY : GBSW_E_DEVICE,
                     std::string("batch upload: ") + hipGetErrorString(e));
+    }
     {
         const int A = alphabet_from_mask(alphabet, seen, b->lut, b->code_of);
-        if (A < 0) return A;
+        if (A < 0) {
+            (void)hipStreamSynchronize(st);
+            return A;
+        }
         job.alpha = A;
         job.code_of = alphabet == GBSW_PROTEIN ? b->code_of : nullptr;
     }
-    count_buckets(job, b->len_ref.data(), b->len_qry.data());
     job.ref = b->ref.as<uint8_t>();
     job.qry = b->qry.as<uint8_t>();
     job.ref_off = b->ref_off.as<uint64_t>();
@@ -244,8 +409,9 @@ static int batch_fill(gbsw_batch* b, gbsw_context* ctx, Exec& ex, int32_t alphab
 
 namespace {
 
-// Both passes of every pair of batch b on ex's streams, blocking.
-int batch_align_on(gbsw_batch* b, Exec& ex, const gbsw_scoring* sc, int32_t mode)
+// Both passes of every pair of batch b on ex's streams, blocking; the results also to
+// `results` (pinned, 5 n) if given.
+int batch_align_on(gbsw_batch* b, Exec& ex, const gbsw_scoring* sc, int32_t mode, int32_t* results = nullptr)
 {
     if (mode != GBSW_PLAIN && mode != GBSW_BATCHED) return fail(GBSW_E_ARGUMENT, "unknown mode");
     GBSW_HIP_TRY(hipSetDevice(b->ctx->device));
@@ -260,8 +426,15 @@ int batch_align_on(gbsw_batch* b, Exec& ex, const gbsw_scoring* sc, int32_t mode
         (void)hipStreamSynchronize(ex.stream);
         return rc;
     }
+    const size_t bytes = sizeof(int32_t) * 5 * (size_t)b->job.n;
+    if (results && bytes) GBSW_HIP_TRY(hipMemcpyAsync(results, b->out.ptr, bytes, hipMemcpyDeviceToHost, ex.stream));
     double ms = 0.0;
     rc = complete_job(ex, b->job, sc, &ms);
+    if (results && bytes) {
+        if (rc == GBSW_OK && ex.late_results) // (aligned again: recomputed pairs)
+            GBSW_HIP_TRY(hipMemcpyAsync(results, b->out.ptr, bytes, hipMemcpyDeviceToHost, ex.stream));
+        GBSW_HIP_TRY(hipStreamSynchronize(ex.stream));
+    }
     b->launches = ex.launches;
     b->stats.device_ms = ms;
     b->stats.launches = (int32_t)b->launches.size();
@@ -270,6 +443,14 @@ int batch_align_on(gbsw_batch* b, Exec& ex, const gbsw_scoring* sc, int32_t mode
     for (const LaunchRec& L : b->launches) b->stats.main_kernel_ms = std::max(b->stats.main_kernel_ms, L.ms);
     b->aligned = rc == GBSW_OK;
     return rc;
+}
+
+// Five result arrays of n that are one block.
+bool back_to_back(int32_t* const* dst, size_t n)
+{
+    for (int f = 0; f < 5; ++f)
+        if (!dst[0] || dst[f] != dst[0] + f * n) return false;
+    return true;
 }
 
 // Carve the device scratch of gbsw_align_noalloc for one call of n pairs:
@@ -297,10 +478,7 @@ int noalloc_carve(gbsw_context* ctx, int64_t n, uint64_t ref_bytes, uint64_t qry
     take(x.sub, sizeof(int16_t) * 1024);
     take(x.lut, 256);
     take(x.colmax, sizeof(int16_t) * 32);
-    take(b->ref, std::max<uint64_t>(ref_bytes, 16));
-    take(b->qry, std::max<uint64_t>(qry_bytes, 16));
-    take(b->ref_off, sizeof(uint64_t) * (np + 1));
-    take(b->qry_off, sizeof(uint64_t) * (np + 1));
+    take(b->input, input_layout(n, ref_bytes, qry_bytes).total);
     take(b->out, sizeof(int32_t) * 5 * np);
     take(b->keys, std::max<size_t>(4 * np, 32));
     take(b->keys_sorted, 4 * np);
@@ -420,7 +598,7 @@ int gbsw_batch_create(gbsw_context* ctx, int32_t alphabet, int64_t n, const char
     if (!out) return fail(GBSW_E_ARGUMENT, "out is null");
     *out = nullptr;
     gbsw_batch* b = new gbsw_batch();
-    const int rc = ctx ? batch_fill(b, ctx, ctx->ex, alphabet, n, ref, ref_off, query, query_off)
+    const int rc = ctx ? batch_fill(b, ctx, ctx->ex, true, alphabet, n, ref, ref_off, query, query_off)
                        : fail(GBSW_E_ARGUMENT, "context is null");
     if (rc) {
         const std::string err = gbsw_last_error();
@@ -721,10 +899,15 @@ int gbsw_batch_results(gbsw_batch* b, int32_t* score, int32_t* ref_begin, int32_
     if (!b) return fail(GBSW_E_ARGUMENT, "batch is null");
     GBSW_HIP_TRY(hipSetDevice(b->ctx->device));
     int32_t* dst[5] = {score, ref_begin, ref_end, query_begin, query_end};
+    const size_t n = (size_t)b->job.n;
+    if (n && back_to_back(dst, n)) {
+        GBSW_HIP_TRY(hipMemcpy(dst[0], b->out.ptr, sizeof(int32_t) * 5 * n, hipMemcpyDeviceToHost));
+        return GBSW_OK;
+    }
     for (int f = 0; f < 5; ++f)
-        if (dst[f] && b->job.n)
-            GBSW_HIP_TRY(hipMemcpy(dst[f], b->out.as<int32_t>() + (size_t)f * (size_t)b->job.n,
-                                   sizeof(int32_t) * (size_t)b->job.n, hipMemcpyDeviceToHost));
+        if (dst[f] && n)
+            GBSW_HIP_TRY(hipMemcpy(dst[f], b->out.as<int32_t>() + (size_t)f * n, sizeof(int32_t) * n,
+                                   hipMemcpyDeviceToHost));
     return GBSW_OK;
 }
 
@@ -803,9 +986,29 @@ int gbsw_align(gbsw_context* ctx, const gbsw_scoring* sc, int32_t mode, int64_t 
         ctx->oneshot->one_shot = true;
     }
     gbsw_batch* b = ctx->oneshot;
-    int rc = batch_fill(b, ctx, ctx->ex, sc->alphabet, n, ref, ref_off, query, query_off);
-    if (!rc) rc = gbsw_batch_align(b, sc, mode);
-    if (!rc) rc = gbsw_batch_results(b, score, ref_begin, ref_end, query_begin, query_end);
+    int rc = batch_fill(b, ctx, ctx->ex, true, sc->alphabet, n, ref, ref_off, query, query_off);
+    // few results: copied behind the kernels, with the one wait of the call
+    constexpr int64_t kStagedResults = 16384;
+    int32_t* pinned = nullptr;
+    if (!rc && n && n <= kStagedResults) {
+        GBSW_HIP_TRY(b->results.reserve(sizeof(int32_t) * 5 * (size_t)n));
+        pinned = b->results.as<int32_t>();
+    }
+    if (!rc) {
+        rc = batch_align_on(b, ctx->ex, sc, mode, pinned);
+        if (rc) {
+            const std::string err = gbsw_last_error();
+            (void)hipStreamSynchronize(ctx->ex.stream); // (the input block may be under way)
+            set_error(err);
+        }
+    }
+    if (!rc && pinned) {
+        int32_t* dst[5] = {score, ref_begin, ref_end, query_begin, query_end};
+        for (int f = 0; f < 5; ++f)
+            if (dst[f]) std::memcpy(dst[f], pinned + (size_t)f * (size_t)n, sizeof(int32_t) * (size_t)n);
+    } else if (!rc) {
+        rc = gbsw_batch_results(b, score, ref_begin, ref_end, query_begin, query_end);
+    }
     return rc;
 }
 
@@ -820,7 +1023,7 @@ int gbsw_align_noalloc(gbsw_context* ctx, const gbsw_scoring* sc, int32_t mode, 
     const uint64_t qb = n ? query_off[n] - query_off[0] : 0;
     int rc = noalloc_carve(ctx, n, rb, qb);
     gbsw_batch* b = ctx->nbatch;
-    if (!rc) rc = batch_fill(b, ctx, ctx->nx, sc->alphabet, n, ref, ref_off, query, query_off);
+    if (!rc) rc = batch_fill(b, ctx, ctx->nx, false, sc->alphabet, n, ref, ref_off, query, query_off);
     if (!rc) rc = batch_align_on(b, ctx->nx, sc, mode);
     if (!rc) rc = gbsw_batch_results(b, score, ref_begin, ref_end, query_begin, query_end);
     return rc;

@@ -318,16 +318,6 @@ int k_for_cols(int cols, int alpha, int model)
     return best;
 }
 
-void count_buckets(Job& job, const int32_t* len_ref, const int32_t* len_qry)
-{
-    Bucket sum[kClasses];
-    for (int64_t p = 0; p < job.n; ++p) {
-        const int32_t la = len_ref[p], lb = len_qry[p];
-        sum[length_class(std::min(la, lb))].add(std::min(la, lb), std::max(la, lb));
-    }
-    place_buckets(job, sum);
-}
-
 void place_buckets(Job& job, const Bucket* by_class)
 {
     job.buckets.clear();

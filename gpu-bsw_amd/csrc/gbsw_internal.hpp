@@ -192,7 +192,6 @@ int k_for_cols(int cols, int alpha, int model);
 double issue_share(double waves, double threshold);
 // Fill job.buckets from per-pair lengths (host), or from the sums per length class:
 // the classes that occur, in work order (longest first).
-void count_buckets(Job& job, const int32_t* len_ref, const int32_t* len_qry);
 void place_buckets(Job& job, const Bucket* by_class);
 // Workgroups of a full-occupancy one-pair-per-wave launch.
 int wide_grid_cap(const Exec& ex, int alpha);

@@ -83,8 +83,11 @@ struct PrepareArgs {
     int32_t helpers;         // workgroups for tables and clearing (set by prepare_job)
 };
 hipError_t prepare_job(const PrepareArgs& a, hipStream_t stream);
-// OR into mask[8] the set of byte values in p[0, n) (p 16-byte aligned).
-hipError_t byte_presence(const uint8_t* p, uint64_t n, uint32_t* mask, hipStream_t stream);
+// Sets of byte values in p[0, n) and p2[0, n2) (16-byte aligned): eight mask words per
+// workgroup of up to kPresenceBlocks, in pinned host memory.
+constexpr int kPresenceBlocks = 128;
+hipError_t byte_presence(const uint8_t* p, uint64_t n, const uint8_t* p2, uint64_t n2, uint32_t* masks,
+                         hipStream_t stream);
 hipError_t sort_pairs(void* temp, size_t& temp_bytes, const uint32_t* kin, uint32_t* kout, const int32_t* vin,
                       int32_t* vout, int n, int end_bit, hipStream_t stream);
 

@@ -245,7 +245,7 @@ class Context:
         n = len(ro) - 1
         if len(qo) - 1 != n:
             raise ValueError("ref and query counts differ")
-        out = np.zeros((5, max(n, 1)), dtype=np.int32)
+        out = np.empty((5, max(n, 1)), dtype=np.int32)
         ptrs = [out[f].ctypes.data for f in range(5)]
         rb = np.ascontiguousarray(rb, dtype=np.uint8)
         qb = np.ascontiguousarray(qb, dtype=np.uint8)
@@ -254,7 +254,7 @@ class Context:
         fn = self._lib.gbsw_align_noalloc if noalloc else self._lib.gbsw_align
         _check(fn(self._h, ctypes.byref(scoring), MODES.get(mode, mode), n, rb.ctypes.data, ro.ctypes.data,
                   qb.ctypes.data, qo.ctypes.data, *ptrs))
-        return {f: out[k][:n].copy() for k, f in enumerate(FIELDS)}
+        return {f: out[k][:n] for k, f in enumerate(FIELDS)}
 
 
 class Batch:
