@@ -321,10 +321,11 @@ static int batch_fill(gbsw_batch* b, gbsw_context* ctx, Exec& ex, bool staged, i
         h = (uint8_t*)offs.data();
     }
     job.buckets.reserve(kClasses); // (no allocation beside running threads)
+    job.fine.reserve(kFineClasses);
     // what takes a pass over the pairs: offsets from 0, classes
     auto pairs_pass = [&]() {
         uint64_t *ro = (uint64_t*)(h + L.ref_off), *qo = (uint64_t*)(h + L.qry_off);
-        Bucket classes[kClasses];
+        Bucket classes[kClasses], fine[kFineClasses];
         ro[0] = qo[0] = 0;
         for (int64_t p = 0; p < n; ++p) {
             const uint64_t lr = ref_off[p + 1] - ref_off[p], lq = query_off[p + 1] - query_off[p];
@@ -334,9 +335,12 @@ static int batch_fill(gbsw_batch* b, gbsw_context* ctx, Exec& ex, bool staged, i
             job.max_rows = std::max(job.max_rows, rows);
             job.max_cols = std::max(job.max_cols, cols);
             job.cells += (int64_t)(lr * lq);
-            classes[length_class(cols)].add(cols, rows);
+            fine[fine_class(cols)].add(cols, rows);
         }
-        place_buckets(job, classes);
+        for (const Bucket& f : fine)
+            if (f.count) classes[length_class(f.max_cols)].add(f);
+        place_buckets(job.buckets, classes, kClasses);
+        place_buckets(job.fine, fine, kFineClasses);
     };
     if (e == hipSuccess) e = hipMemsetAsync(b->out.ptr, 0, sizeof(int32_t) * 5 * np, st);
     uint8_t* dev = b->input.as<uint8_t>();

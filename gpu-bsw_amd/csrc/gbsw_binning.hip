@@ -1,6 +1,6 @@
 // gbsw_binning.hip -- device-side length binning of a batch (batched form).
 //
-// Every pair gets a 15-bit key: its length class, longest first (6 bits), then
+// Every pair gets a 15-bit key: its length class (or fine class), longest first (6 bits), then
 // 511 - (longer length / 32) (9 bits, capped).  Sorting (key, pair index) yields the
 // work order: classes of longer pairs first, inside a class the most rows first
 // (longest-processing-time order for the persistent work queues), so the pairs of a
@@ -22,7 +22,7 @@ __device__ __forceinline__ uint32_t sort_key(const PrepareArgs& a, int64_t p)
     const uint32_t la = (uint32_t)(a.ref_off[p + 1] - a.ref_off[p]);
     const uint32_t lb = (uint32_t)(a.qry_off[p + 1] - a.qry_off[p]);
     const uint32_t m = la < lb ? la : lb, M = la < lb ? lb : la;
-    const uint32_t c = (uint32_t)(kClasses - 1 - length_class((int)m));
+    const uint32_t c = (uint32_t)(a.fine ? kFineClasses - 1 - fine_class((int)m) : kClasses - 1 - length_class((int)m));
     const uint32_t top = (1u << kRowBits) - 1u, r = M >> 5;
     return (c << kRowBits) | (top - (r < top ? r : top));
 }

@@ -107,9 +107,12 @@ int lds_for(int K, int alpha, bool p8, int bnd_bytes = 4)
     return lds_layout(prof_row_bytes(K, p8), alpha, bnd_bytes).total;
 }
 
+// Lanes per pair of the sweep kernel with eight pairs per wave (16 lanes for two).
+constexpr int kLanesPerTwo = kLanesPerPair / 2;
+
 int sweep_lds_for(int K, int alpha, int form, int G)
 {
-    return sweep_lds(G, K, form, alpha, 4).total;
+    return G == kLanesPerTwo ? pairs_lds(K, alpha).total : sweep_lds(G, K, form, alpha, 4).total;
 }
 
 int grid_for(const Exec& ex, int kind, int K, int lds, int64_t nquads)
@@ -324,14 +327,14 @@ int k_for_cols(int cols, int alpha, int model)
     return best;
 }
 
-void place_buckets(Job& job, const Bucket* by_class)
+void place_buckets(std::vector<Bucket>& out, const Bucket* by_class, int classes)
 {
-    job.buckets.clear();
+    out.clear();
     int64_t at = 0;
-    for (int c = kClasses - 1; c >= 0; --c) { // the sort order: longest class first
+    for (int c = classes - 1; c >= 0; --c) { // the sort order: longest class first
         if (by_class[c].count == 0) continue;
-        job.buckets.push_back(by_class[c]);
-        job.buckets.back().begin = at;
+        out.push_back(by_class[c]);
+        out.back().begin = at;
         at += by_class[c].count;
     }
 }
@@ -478,6 +481,11 @@ size_t split_words_of(const BucketPlan& b)
 // 391 / 455 / 602 at K = 5 / 6 / 8 alone); a strip with boundary rows takes more.
 double step_issue(int K, bool ms) { return 25.0 * K + 80 + (ms ? 20 : 0); }
 double step_alone(int K, bool ms) { return 58.0 * K + 135 + (ms ? 55 : 0); }
+// Eight pairs per wave, K columns per lane.  (Short reads, K = 10 against four pairs at
+// K = 5: 5k, 10k, 20k, 30k, 50k, 100k and 300k pairs 0.33, 0.47, 0.59, 0.72, 0.91, 1.55
+// and 4.15 ms against 0.32, 0.34, 0.56, 0.71, 1.01, 1.84 and 4.91.)
+double pairs_issue(int K) { return 29.5 * K + 52; }
+double pairs_alone(int K) { return 56.0 * K + 200; }
 // Forward plus reverse pass, in forward passes.
 constexpr double kPasses = 1.6;
 // A strip of the split form starts once its predecessor has published the rows of
@@ -491,6 +499,7 @@ constexpr int kSweepK64[] = {GBSW_SWEEP_K64(GBSW_ITEM)};
 constexpr int kSweepSplitK[] = {GBSW_SWEEP_K64_SPLIT(GBSW_ITEM)};
 #undef GBSW_ITEM
 constexpr int kSweepNarrowMax = 8; // widest geometry of the narrow four-pair kernel
+static_assert(kPairsCols == kVirtPerPair * kSweepNarrowMax, "eight pairs per wave: the narrow classes");
 
 // Estimates of one class in one geometry: work (wave cycles over all SIMDs) and
 // the longest item's time.
@@ -514,6 +523,17 @@ GeoCost geo_cost(const Exec& ex, const Bucket& bk, int G, int K, bool split)
     return c;
 }
 
+// The same for eight pairs per wave.
+GeoCost pairs_cost(const Exec& ex, const Bucket& bk, int K)
+{
+    GeoCost c;
+    c.K = K;
+    const double n = (double)std::max<int64_t>(1, bk.count);
+    c.work = n / 8 * ((double)bk.rows / n + kLanesPerPair - 1) * pairs_issue(K) * kPasses / (4.0 * ex.num_cu);
+    c.unit = ((double)bk.max_rows + kLanesPerPair - 1) * pairs_alone(K) * kPasses;
+    return c;
+}
+
 // The launches of a job whose scoring runs the sweep kernels.
 //
 // Which geometry a class takes.  Four pairs per wave issue the fewest instructions
@@ -524,10 +544,13 @@ GeoCost geo_cost(const Exec& ex, const Bucket& bk, int G, int K, bool split)
 // geometries), one launch each.  A job lasts at least as long as its instructions
 // take on the whole GPU and as its longest item takes alone; the stretches are
 // those of least max + kOverlap x min of the two.
-void plan_sweeps(const Exec& ex, const Job& job, const SweepChoice& sw, bool may_split, std::vector<BucketPlan>& plan)
+//
+// pairs: the narrow classes with eight pairs per wave (cls: the fine classes).
+// Returns the estimate.
+double plan_sweeps_over(const Exec& ex, const Job& job, const std::vector<Bucket>& cls, const SweepChoice& sw,
+                        bool may_split, bool pairs, std::vector<BucketPlan>& plan)
 {
     constexpr double kOverlap = 0.35;
-    const std::vector<Bucket>& cls = job.buckets;
     const size_t n = cls.size();
     const double thr = occupancy_threshold(job.kmodel);
     auto lds = [&](int G, int K) { return sweep_lds_for(K, job.alpha, sw.form, G); };
@@ -558,13 +581,21 @@ void plan_sweeps(const Exec& ex, const Job& job, const SweepChoice& sw, bool may
     four.work.assign(n + 1, 0.0);
     four.unit.assign(n + 1, 0.0);
     for (size_t i = n; i-- > 0;) {
-        int K = 0;
-        for (int k : kSweepK16)
-            if (cls[i].max_cols <= kVirtPerPair * k) { K = k; break; }
-        const double s = K ? share(K > kSweepNarrowMax ? kWideLanes : 0, kLanesPerPair, K) : 0.0;
+        double s = 0.0;
+        if (pairs && cls[i].max_cols <= kPairsCols) {
+            const int K = std::max(2, (cls[i].max_cols + 15) / 16);
+            s = K > kPairsNarrowMax ? share(kHalfPairs | kWideLanes, kLanesPerTwo, kPairsCols / 16)
+                                    : share(kHalfPairs, kLanesPerTwo, kPairsNarrowMax);
+            four.cost[i] = pairs_cost(ex, cls[i], K);
+        } else {
+            int K = 0;
+            for (int k : kSweepK16)
+                if (cls[i].max_cols <= kVirtPerPair * k) { K = k; break; }
+            if (K) s = share(K > kSweepNarrowMax ? kWideLanes : 0, kLanesPerPair, K);
+            if (K) four.cost[i] = geo_cost(ex, cls[i], kLanesPerPair, K, false);
+        }
         if (s <= 0) break;
         first = i;
-        four.cost[i] = geo_cost(ex, cls[i], kLanesPerPair, K, false);
         four.work[i] = four.work[i + 1] + four.cost[i].work / s;
         four.unit[i] = std::max(four.unit[i + 1], four.cost[i].unit);
     }
@@ -609,6 +640,8 @@ void plan_sweeps(const Exec& ex, const Job& job, const SweepChoice& sw, bool may
     size_t i64 = 0, i16 = n, which_one = 0, which_split = 0;
     // launches beyond the first cost little beside a large job and show in a small one
     constexpr double kLaunch = 12000;
+    // (more pairs than this fill the GPU unsplit)
+    const int64_t most_split = 16 * (int64_t)ex.num_cu;
     for (size_t o = 0; o < one.size(); ++o)
         for (size_t b = first; b <= n; ++b) { // [b, n) four pairs per wave
             std::vector<double> unit_tail(b + 1, 0.0); // longest one-pair item of [i, b)
@@ -626,7 +659,7 @@ void plan_sweeps(const Exec& ex, const Job& job, const SweepChoice& sw, bool may
             };
             consider(0, 0);
             for (size_t s = 0; s < split.size(); ++s)
-                for (size_t a = 1; a <= b; ++a) consider(a, s);
+                for (size_t a = 1; a <= b && cls[a - 1].begin + cls[a - 1].count <= most_split; ++a) consider(a, s);
         }
 
     auto add = [&](size_t from, size_t to, int G, int flags, const Option& o, bool is_split) {
@@ -651,11 +684,40 @@ void plan_sweeps(const Exec& ex, const Job& job, const SweepChoice& sw, bool may
         plan.push_back(b);
     };
     size_t narrow = i16;
-    while (narrow < n && four.cost[narrow].K > kSweepNarrowMax) ++narrow;
+    while (narrow < n && cls[narrow].max_cols > kPairsCols) ++narrow;
     if (i64) add(0, i64, kWave, kWideGroup, split[which_split], true);
     add(i64, i16, kWave, kWideGroup, one[which_one], false);
     add(i16, narrow, kLanesPerPair, kWideLanes, four, false);
-    add(narrow, n, kLanesPerPair, 0, four, false);
+    if (pairs) {
+        size_t few = narrow;
+        while (few < n && four.cost[few].K > kPairsNarrowMax) ++few;
+        add(narrow, few, kLanesPerTwo, kHalfPairs | kWideLanes, four, false);
+        add(few, n, kLanesPerTwo, kHalfPairs, four, false);
+    } else {
+        add(narrow, n, kLanesPerPair, 0, four, false);
+    }
+    return best;
+}
+
+// Eight pairs per wave: jobs with two such waves per SIMD and more (fewer leave SIMDs
+// idle) and register tables, where the estimate is less.
+void plan_sweeps(const Exec& ex, const Job& job, const SweepChoice& sw, bool may_split, bool asym,
+                 std::vector<BucketPlan>& plan)
+{
+    const double t = plan_sweeps_over(ex, job, job.buckets, sw, may_split, false, plan);
+    if (sw.form != kProfRegs || asym || job.fine.empty() || job.n <= kSmallSort ||
+        job.n < 8 * 2 * 4 * (int64_t)ex.num_cu)
+        return;
+    std::vector<BucketPlan> other;
+    if (plan_sweeps_over(ex, job, job.fine, sw, may_split, true, other) < t) plan.swap(other);
+}
+
+// Whether a plan's stretches are those of the fine classes.
+bool plan_is_fine(const std::vector<BucketPlan>& plan)
+{
+    for (const BucketPlan& b : plan)
+        if (b.kind & kHalfPairs) return true;
+    return false;
 }
 
 // The launches of a job on the int16 kernels (scorings outside the sweep kernels'
@@ -730,7 +792,7 @@ int plan_batched(Exec& ex, const Job& job, int max_sub, bool p8, const SweepChoi
     };
     auto make = [&](bool split) {
         plan.clear();
-        if (sw.ok) plan_sweeps(ex, job, sw, split, plan);
+        if (sw.ok) plan_sweeps(ex, job, sw, split, asym, plan);
         else plan_int16(ex, job, max_sub, p8, kclamp, split, plan);
         for (BucketPlan& b : plan) set_grid(b);
         sizes();
@@ -801,6 +863,7 @@ int record_batched(Exec& ex, const Job& job, KernelArgs a, const std::vector<Buc
     } else {
         pre.keys = job.keys;
         pre.vals = job.vals;
+        pre.fine = plan_is_fine(plan) ? 1 : 0;
     }
     GBSW_HIP_TRY(prepare_job(pre, st0));
     if (pre.keys) {

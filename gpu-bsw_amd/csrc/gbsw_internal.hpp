@@ -163,7 +163,8 @@ struct Job {
     const uint8_t* lut_host = nullptr; // 256 entries
     int32_t max_rows = 0, max_cols = 0;
     int64_t cells = 0;
-    std::vector<Bucket> buckets;     // batched form (host counts)
+    std::vector<Bucket> buckets;     // batched form: length classes (host counts)
+    std::vector<Bucket> fine;        // the same by fine classes; empty: not counted
     uint32_t* keys = nullptr;
     uint32_t* keys_sorted = nullptr;
     int32_t* vals = nullptr;
@@ -190,9 +191,8 @@ double occupancy_threshold(int model);
 int k_for_cols(int cols, int alpha, int model);
 // Share of the VALU issue rate that `waves` per SIMD reach under a model's threshold.
 double issue_share(double waves, double threshold);
-// Fill job.buckets from per-pair lengths (host), or from the sums per length class:
-// the classes that occur, in work order (longest first).
-void place_buckets(Job& job, const Bucket* by_class);
+// The classes that occur, in work order (longest first).
+void place_buckets(std::vector<Bucket>& out, const Bucket* by_class, int classes);
 // Workgroups of a full-occupancy one-pair-per-wave launch.
 int wide_grid_cap(const Exec& ex, int alpha);
 // Whether a scoring runs the sweep kernels (gbsw_sweep.hpp), and how: the profile

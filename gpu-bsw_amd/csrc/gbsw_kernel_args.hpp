@@ -97,6 +97,16 @@ __host__ __device__ constexpr int length_class(int m)
            : m <= 16384 ? 29 + (m - 8193) / 1024
                         : 37 + (m - 16385) / 4096;
 }
+// Fine classes: up to 256 in steps of 16 (2 .. 16 columns per lane of the sweep kernel
+// with eight pairs per wave), as above beyond.  Only for jobs that run that kernel: in
+// a small job the order by rows, longest first, counts for more (10k short reads:
+// 348 us with the classes above, 356 with these).
+constexpr int kPairsCols = 256, kFineClasses = kClasses + 8;
+__host__ __device__ constexpr int fine_class(int m)
+{
+    return m <= 32 ? 0 : m <= kPairsCols ? (m - 17) / 16 : length_class(m) + 8;
+}
+static_assert(fine_class(kPairsCols) + 1 == fine_class(kPairsCols + 1) && kFineClasses <= 64, "adjacent classes");
 // Sort key of a pair: classes of longer pairs first, in a class the most rows
 // first (longest-processing-time order for the work queues, and like row counts
 // in a wave).  kRowBits bits of row count in steps of 32.
@@ -241,6 +251,26 @@ __host__ __device__ inline SweepLds sweep_lds(int32_t G, int32_t K, int form, in
     L.ring_bnd_off = L.ring_code_off + 2 * sweep_ring(G) * (form == kProfRegs ? 4 : 2);
     L.group_bytes = align_up(L.ring_bnd_off + (sweep_ring(G) + kSweepUnroll) * bnd_bytes, 128);
     L.total = L.group_off + (kWave / G) * L.group_bytes;
+    return L;
+}
+
+// LDS of the sweep kernel with eight pairs per wave: tables, the row rings (a selector
+// for both pairs of a group, each row twice), the rows of the lanes' bests.
+constexpr int kPairsRing = 2 * kChunk;
+struct PairsLds {
+    int32_t lut_off, sub_off, colmax_off, row_tab_off, col_tab_off, ring_off, snap_off, total;
+};
+__host__ __device__ inline PairsLds pairs_lds(int32_t K, int32_t alpha)
+{
+    PairsLds L;
+    L.lut_off = 0;
+    L.sub_off = 256;
+    L.colmax_off = L.sub_off + align_up(2 * alpha * alpha, 16);
+    L.row_tab_off = L.colmax_off + 2 * 32;
+    L.col_tab_off = align_up(L.row_tab_off + 2 * 257, 4);
+    L.ring_off = align_up(L.col_tab_off + 4 * 257, 128);
+    L.snap_off = L.ring_off + (kWave / kLanesPerPair) * 2 * kPairsRing * 4;
+    L.total = L.snap_off + 2 * (K + 1) * kWave * 2;
     return L;
 }
 

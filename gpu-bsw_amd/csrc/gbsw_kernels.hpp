@@ -28,6 +28,7 @@ inline int with_profile(int kind, bool bytes8) { return bytes8 ? (kind | kBytePr
 constexpr int kWideGroup = 0x200;
 constexpr int kRegTables = 0x400;
 constexpr int kWideLanes = 0x800;
+constexpr int kHalfPairs = 0x2000; // eight pairs per wave, one in each half of 16 lanes' registers
 constexpr int kReportedKind = 0x1FF; // the part of a kind that launch statistics report
 inline int sweep_kind(int kind, int form, int flags)
 {
@@ -37,6 +38,9 @@ inline int sweep_kind(int kind, int form, int flags)
 // Geometries of the sweep kernels.
 #define GBSW_SWEEP_K16(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8)
 #define GBSW_SWEEP_K16_WIDE(X) X(10) X(12) X(14) X(16)
+#define GBSW_SWEEP_PAIRS(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10)
+#define GBSW_SWEEP_PAIRS_WIDE(X) X(11) X(12) X(13) X(14) X(15) X(16)
+constexpr int kPairsNarrowMax = 10;
 #define GBSW_SWEEP_K64(X) X(1) X(2) X(3) X(4) X(5) X(6) X(8)
 #define GBSW_SWEEP_K64_SPLIT(X) X(1) X(2) X(3) X(4) X(6) X(8)
 // kernel of a form, nullptr where it is not compiled (gbsw_sweep_*.hip)
@@ -46,6 +50,7 @@ const void* sweep_kernel_words(int kind, int K);
 const void* sweep_kernel_regs_wide(int kind, int K);
 const void* sweep_kernel_bytes_wide(int kind, int K);
 const void* sweep_kernel_words_wide(int kind, int K);
+const void* sweep_kernel_pairs(int kind);
 // int32 cells (kBatchedWide | kWideGroup, with kSplitStrips the split form)
 constexpr int kSplitStrips = 0x1000;
 #define GBSW_SWEEP_K32(X) X(2) X(4)
@@ -80,6 +85,7 @@ struct PrepareArgs {
     uint32_t* split;
     int64_t nsplit;
     int32_t nsub, alpha, nstatus, nqueue;
+    int32_t fine;            // keys by fine classes (not with `order`)
     int32_t helpers;         // workgroups for tables and clearing (set by prepare_job)
 };
 hipError_t prepare_job(const PrepareArgs& a, hipStream_t stream);

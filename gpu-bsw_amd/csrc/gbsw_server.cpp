@@ -481,7 +481,7 @@ void gbsw_server::admit(Slot& s)
     j.max_rows = max_rows;
     j.max_cols = max_cols;
     j.cells = cells;
-    place_buckets(j, sum);
+    place_buckets(j.buckets, sum, kClasses);
     s.busy = true;
     s.launch_seq = ++launch_counter;
     ++busy_slots;

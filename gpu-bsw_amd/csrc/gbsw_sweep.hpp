@@ -371,8 +371,8 @@ struct SweepRows {
 
 // Row table: byte -> code of its row (register form: its half of the selector).
 // Column table (register form): byte -> the four biased scores of its column.
-template <int PF>
-__device__ __forceinline__ void stage_byte_tables(const KernelArgs& a, const SweepSmem& sm)
+template <int PF, class S>
+__device__ __forceinline__ void stage_byte_tables(const KernelArgs& a, const S& sm)
 {
     const int alpha = a.alpha, sbias = -(a.gap_open + a.gap_extend);
     for (int i = threadIdx.x; i <= kNoRow; i += kWave) {

@@ -116,3 +116,54 @@ def test_scores_around_the_16_bit_range(ctx, letters):
         qrys.append(refs[-1][100:100 + rng.randint(1, 120)])
     exp = check(ctx, refs, qrys, ol.dna_scoring(96, -96, -192, -64), gbsw.dna_scoring(96, -96, -192, -64), letters)
     assert exp["score"].max() > 100_000 and ((exp["score"] > 30_000) & (exp["score"] < 33_000)).sum() > 10
+
+
+PAIRS = 120000  # enough pairs of up to 256 columns for eight per wave (16 lanes for two)
+
+
+@pytest.mark.parametrize("letters,sc", [("ACGT", (3, -3, -6, -1)), ("ACG", (1, -1, -1, -1)), ("ACGT", (112, -16, -32, -2))])
+def test_eight_pairs_per_wave(ctx, letters, sc):
+    # columns around every multiple of 16, rows around a chunk and a ring; equal lengths
+    # (the reverse pass may swap the sequences), pairs past the 16-bit range, no score
+    rng = np.random.default_rng(len(letters) + sc[0])
+    L = np.frombuffer(letters.encode(), np.uint8)
+    edge = np.array([c + d for c in range(16, 257, 16) for d in (-1, 0, 1)])
+    cols = np.where(rng.random(PAIRS) < 0.5, rng.choice(edge[edge <= 256], PAIRS), rng.integers(1, 257, PAIRS))
+    cols[rng.random(PAIRS) < 0.7] //= 3
+    cols = np.maximum(cols, 1)
+    rows = cols + rng.choice([0, 1, 15, 31, 32, 33, 63, 64, 65, 130], PAIRS)
+    refs, qrys = [], []
+    for c, r in zip(cols, rows):
+        a = L[rng.integers(0, len(L), r)]
+        at = int(rng.integers(0, r - c + 1))
+        b = a[at:at + c].copy()
+        u = rng.random()
+        if u < 0.25:
+            b = L[rng.integers(0, len(L), c)]
+        elif u < 0.8:
+            hit = rng.random(c) < 0.1
+            b[hit] = L[rng.integers(0, len(L), int(hit.sum()))]
+            if c > 20 and u < 0.5:  # a short gap
+                k = int(rng.integers(1, 6))
+                b = np.concatenate([b[:c // 2], b[c // 2 + k:], L[rng.integers(0, len(L), k)]])
+        x, y = a.tobytes(), b.tobytes()
+        refs.append(x if rng.random() < 0.7 else y)
+        qrys.append(y if refs[-1] is x else x)
+    refs[5], qrys[5] = b"A" * 60, b"C" * 40
+    ro = np.zeros(PAIRS + 1, np.uint64)
+    qo = np.zeros(PAIRS + 1, np.uint64)
+    np.cumsum([len(x) for x in refs], out=ro[1:])
+    np.cumsum([len(x) for x in qrys], out=qo[1:])
+    rb, qb = np.frombuffer(b"".join(refs), np.uint8), np.frombuffer(b"".join(qrys), np.uint8)
+    exp = ol.align_batch(rb, ro, qb, qo, ol.dna_scoring(*sc))
+    b = ctx.batch(gbsw.DNA, rb, ro, qb, qo)
+    try:
+        b.align(gbsw.dna_scoring(*sc))
+        got, launches = b.results(), b.launches()
+    finally:
+        b.close()
+    # columns per lane of 16 lanes, not of two blocks of 16
+    assert max(x["columns_per_lane"] for x in launches if x["pairs"] > 1000) == 16, launches
+    for f in FIELDS:
+        bad = np.nonzero(exp[f] != got[f])[0]
+        assert len(bad) == 0, (sc, f, len(bad), refs[bad[0]], qrys[bad[0]], exp[f][bad[0]], got[f][bad[0]])
