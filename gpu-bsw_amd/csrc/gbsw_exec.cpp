@@ -462,7 +462,7 @@ struct BucketPlan {
 bool plan_is_split(const BucketPlan& b)
 {
     const int k = b.kind & 0xFF;
-    return k == kSplit || k == kSplitF16;
+    return k == kSplit || k == kSplitF16 || (b.kind & kSplitStrips);
 }
 
 // 32-bit words of a split launch's bookkeeping: keys (2 x count u64), progress
@@ -699,11 +699,68 @@ double plan_sweeps_over(const Exec& ex, const Job& job, const std::vector<Bucket
     return best;
 }
 
+// int32 cells, one pair per wave, K columns per virtual lane (split: strips on several
+// waves).
+constexpr int kMostInt32 = 4; // widest geometry of the int32 kernels
+void int32_geometry(const Job& job, int K, bool split, BucketPlan& b)
+{
+    b.G = kWave;
+    b.K = K;
+    b.kind = kBatchedWide | kWideGroup | (split ? kSplitStrips : 0);
+    b.strips = std::max(1, (b.bk.max_cols + 2 * kWave * K - 1) / (2 * kWave * K));
+    b.lds = sweep_lds(kWave, K, kProfWords, job.alpha, 8).total;
+}
+// The split form in the geometry whose chain of strips is shortest.  (An int32 step
+// takes about twice a 16-bit one.)
+void int32_split_geometry(const Job& job, BucketPlan& b)
+{
+    double best = 1e300;
+    int K = kMostInt32;
+    for (int k = 2; k <= kMostInt32; k += 2) {
+        const double strips = std::ceil(b.bk.max_cols / (2.0 * kWave * k));
+        const double t = (b.bk.max_rows + (strips - 1) * split_lag(kWave)) * step_alone(2 * k, true);
+        if (t < best) { best = t; K = k; }
+    }
+    int32_geometry(job, K, true, b);
+    b.unit = best * kPasses;
+}
+
+// The classes of the longest pairs, as far as one may well pass the 16-bit range (its
+// columns at 0.75 of the best score each, which reads of 10 % errors reach), take int32
+// cells at once, beside the others, where their strips' waves are few (two per SIMD).
+// Recomputed after the others, two of 400 long reads doubled the time, 21.5 ms where
+// this takes 12.2: their chain of strips is as long as everything else.
+size_t plan_int32(const Exec& ex, const Job& job, const SweepChoice& sw, int max_sub, std::vector<BucketPlan>& plan)
+{
+    if (ex.fixed || !sw.wide_ok) return 0;
+    BucketPlan b;
+    size_t n = 0;
+    for (; n < job.buckets.size(); ++n) {
+        const Bucket& bk = job.buckets[n];
+        if (0.75 * max_sub * (double)bk.max_cols < (double)sw.sat_limit) break;
+        b.bk.add(bk);
+    }
+    if (!n) return 0;
+    b.bk.begin = job.buckets[0].begin;
+    int32_split_geometry(job, b);
+    if (b.strips < 2 || b.bk.count * b.strips > 8 * (int64_t)ex.num_cu) return 0;
+    b.sat_limit = INT_MAX;
+    b.ranges.push_back({(int32_t)b.bk.count, b.K});
+    plan.push_back(b);
+    return n;
+}
+
 // Eight pairs per wave: jobs with two such waves per SIMD and more (fewer leave SIMDs
 // idle) and register tables, where the estimate is less.
-void plan_sweeps(const Exec& ex, const Job& job, const SweepChoice& sw, bool may_split, bool asym,
+void plan_sweeps(const Exec& ex, const Job& job, const SweepChoice& sw, int max_sub, bool may_split, bool asym,
                  std::vector<BucketPlan>& plan)
 {
+    const size_t wide = may_split ? plan_int32(ex, job, sw, max_sub, plan) : 0;
+    if (wide) {
+        const std::vector<Bucket> rest(job.buckets.begin() + (std::ptrdiff_t)wide, job.buckets.end());
+        if (!rest.empty()) (void)plan_sweeps_over(ex, job, rest, sw, may_split, false, plan);
+        return;
+    }
     const double t = plan_sweeps_over(ex, job, job.buckets, sw, may_split, false, plan);
     if (sw.form != kProfRegs || asym || job.fine.empty() || job.n <= kSmallSort ||
         job.n < 8 * 2 * 4 * (int64_t)ex.num_cu)
@@ -781,7 +838,11 @@ int plan_batched(Exec& ex, const Job& job, int max_sub, bool p8, const SweepChoi
             b.bnd_at = bnd_words;
             const size_t per_wg = (size_t)b.pairs_per_wave() * (size_t)std::max(1, b.bk.max_rows);
             if (plan_is_split(b)) {
-                bnd_words += (size_t)2 * b.grid * per_wg;
+                // (int32 rows are pairs of 64-bit alignment)
+                const size_t row_words = b.kind & kSplitStrips ? 2 : 1;
+                bnd_words = (bnd_words + 1) & ~(size_t)1;
+                b.bnd_at = bnd_words;
+                bnd_words += (size_t)2 * b.grid * per_wg * row_words;
                 b.split_at = split_words;
                 split_words += split_words_of(b);
             } else if (b.strips > 1) {
@@ -792,7 +853,7 @@ int plan_batched(Exec& ex, const Job& job, int max_sub, bool p8, const SweepChoi
     };
     auto make = [&](bool split) {
         plan.clear();
-        if (sw.ok) plan_sweeps(ex, job, sw, split, asym, plan);
+        if (sw.ok) plan_sweeps(ex, job, sw, max_sub, split, asym, plan);
         else plan_int16(ex, job, max_sub, p8, kclamp, split, plan);
         for (BucketPlan& b : plan) set_grid(b);
         sizes();
@@ -841,6 +902,7 @@ int set_split_args(const Exec& ex, const BucketPlan& b, KernelArgs& a)
         return fail(GBSW_E_INTERNAL, "split bookkeeping of a launch is not 8-byte aligned");
     a.split.strips = b.strips;
     a.split.slots = (int32_t)(nslots / kXcds);
+    a.split.first = b.kind & kSplitStrips ? 1 : 0;
     return GBSW_OK;
 }
 
@@ -1089,29 +1151,11 @@ int redo_int32(Exec& ex, const Job& job, const gbsw_scoring* sc, int64_t count)
     if (sw.wide_ok) {
         // One pair per wave; few pairs (up to a wave per SIMD) as strips of the split
         // form: 400 long reads, a few of them past the range, 773 -> 21.5 ms with
-        // the few no longer on one 16-lane group each.  (An int32 step takes about
-        // twice a 16-bit one.)
+        // the few no longer on one 16-lane group each.
         a.base = sw.base;
-        b.G = kWave;
-        auto geometry = [&](int K, bool split) {
-            b.K = K;
-            b.kind = kBatchedWide | kWideGroup | (split ? kSplitStrips : 0);
-            b.strips = std::max(1, (job.max_cols + 2 * kWave * K - 1) / (2 * kWave * K));
-            b.lds = sweep_lds(kWave, K, kProfWords, job.alpha, 8).total;
-        };
-        constexpr int kMost = 4; // widest geometry of the int32 kernels
-        geometry(kMost, false);
+        int32_geometry(job, kMostInt32, false, b);
         const bool few = count <= 4 * (int64_t)ex.num_cu;
-        if (few && b.strips > 1 && ex.split && !ex.split_misplaced && !a.asym) {
-            double best = 1e300;
-            int K = kMost;
-            for (int k = 2; k <= kMost; k += 2) {
-                const double strips = std::ceil(job.max_cols / (2.0 * kWave * k));
-                const double t = (job.max_rows + (strips - 1) * split_lag(kWave)) * step_alone(2 * k, true);
-                if (t < best) { best = t; K = k; }
-            }
-            geometry(K, true);
-        }
+        if (few && b.strips > 1 && ex.split && !ex.split_misplaced && !a.asym) int32_split_geometry(job, b);
     } else {
         int nk = 0;
         const int* wk = wide_k_list(&nk);

@@ -55,6 +55,7 @@ struct SplitArgs {
                       // (s + 1: strip s keeps it, kGateDropped: dropped from the rest)
     int32_t strips;   // strip items per quad and pass
     int32_t slots;    // boundary slots per XCD
+    int32_t first;    // 1: before other split launches (int32 cells: the longest chain of a job)
 };
 constexpr uint32_t kGateDropped = 0xFFFFFFFFu;
 constexpr int kXcds = 8;                 // workgroup w is expected on XCD w % 8

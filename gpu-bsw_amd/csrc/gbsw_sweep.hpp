@@ -990,7 +990,9 @@ __global__ __launch_bounds__(64, A::kWide ? 2 : K <= 6 ? 4 : 3) void k_sweep_spl
     const int x = (int)(blockIdx.x % kXcds);
     const SplitArgs& sp = a.split;
     split_check_placement(sp, x, a.status);
-    __builtin_amdgcn_s_setprio(3); // as in k_split: the chain of waits goes first
+    // as in k_split: the chain of waits goes first
+    if (sp.first) __builtin_amdgcn_s_setprio(3);
+    else __builtin_amdgcn_s_setprio(2);
     const int64_t nsets = (a.order_n + PW - 1) / PW;
     const int64_t nsets_x = nsets > x ? (nsets - x + kXcds - 1) / kXcds : 0;
     const int64_t per_pass = nsets_x * sp.strips;

@@ -167,3 +167,39 @@ def test_eight_pairs_per_wave(ctx, letters, sc):
     for f in FIELDS:
         bad = np.nonzero(exp[f] != got[f])[0]
         assert len(bad) == 0, (sc, f, len(bad), refs[bad[0]], qrys[bad[0]], exp[f][bad[0]], got[f][bad[0]])
+
+
+def test_long_pairs_take_int32_cells_at_once(ctx):
+    # a class whose longest pair may pass the 16-bit range runs on int32 cells beside the
+    # rest: one pair that passes it, an unrelated one of its class, shorter ones, and one
+    # that passes it from a shorter class (no errors: recomputed after the rest)
+    rng = np.random.default_rng(77)
+    L = np.frombuffer(b"ACGT", np.uint8)
+
+    def related(n, subst):
+        a = L[rng.integers(0, 4, n)]
+        b = a.copy()
+        hit = rng.random(n) < subst
+        b[hit] = L[rng.integers(0, 4, int(hit.sum()))]
+        return a.tobytes(), np.delete(b, slice(n // 3, n // 3 + 7)).tobytes()
+
+    pairs = [related(13400, 0.08), (L[rng.integers(0, 4, 13500)].tobytes(), L[rng.integers(0, 4, 13350)].tobytes()),
+             related(10300, 0.0)] + [related(int(n), 0.1) for n in rng.integers(200, 3000, 30)]
+    rb, ro = gbsw.pack([p[0] for p in pairs])
+    qb, qo = gbsw.pack([p[1] for p in pairs])
+    exp = ol.align_batch(rb, ro, qb, qo, ol.dna_scoring(3, -3, -6, -1))
+    assert exp["score"][0] > 29000 and exp["score"][2] > 29000 and exp["score"][1] < 28000
+    sc = gbsw.dna_scoring(3, -3, -6, -1)
+    b = ctx.batch(gbsw.DNA, rb, ro, qb, qo)
+    try:
+        for split in (1, 0):  # without the split form every such pair is recomputed
+            ctx.set_option(gbsw.OPT_SPLIT, split)
+            for _ in range(2):
+                b.align(sc)
+                got, wide = b.results(), [x["pairs"] for x in b.launches() if x["kind"] == 3]
+                assert wide == ([2, 1] if split else [2]), wide
+                for f in FIELDS:
+                    assert np.array_equal(exp[f], got[f]), (split, f)
+    finally:
+        ctx.set_option(gbsw.OPT_SPLIT, 1)
+        b.close()
