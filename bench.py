@@ -50,7 +50,7 @@ PEAK_INT_TOPS_PACKED = MI355X_CU * 64 * MI355X_GHZ * 2 / 1000.0  # 78.6 TOP/s (i
 
 # launch kind -> (kernel, cell policy)
 KIND_NAMES = {2: ("k_batched", "Packed16"), 3: ("k_batched", "Wide32"), 4: ("k_sweep", "Sweep16"),
-              5: ("k_split", "Packed16"), 6: ("k_sweep_split", "Sweep16")}
+              5: ("k_split", "Packed16"), 6: ("k_sweep_split", "Sweep16"), 7: ("k_sweep_pairs", "Sweep16")}
 
 
 def log(*a):
@@ -61,7 +61,7 @@ def profiled_traffic(kname):
     """HBM bytes per launch of `kname` (FETCH_SIZE + WRITE_SIZE, calibrated) from
     the committed rocprofv3 summary, or None when it does not cover this kernel."""
     import re
-    path = os.path.join(REPO, "profiles", "k_batched_dna_mix_1m.md")
+    path = os.path.join(REPO, "profiles", "k_sweep_dna_mix_1m.md")
     if not os.path.exists(path):
         return None
     for line in open(path):
@@ -494,9 +494,8 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        # int16 cells; length buckets whose score bound is below 2048 compute in
-        # packed f16 holding integers (exact: every value is an integer below 2048)
-        "dtype": "int16 (f16 integer-exact buckets)",
+        # 16-bit integer cells (maxima through f16 bit patterns, which order as integers)
+        "dtype": "int16",
         "data": "synthetic",
         "config": {"workload": "batched uneven-length DNA mix: %d seeded pairs, query lognormal(median 150) "
                                "[32,1024], ref lognormal(median 600) [64,2048], +3/-3/-6/-1" % w.n,

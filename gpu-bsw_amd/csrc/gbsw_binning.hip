@@ -34,10 +34,10 @@ __device__ __forceinline__ uint32_t sort_key(const PrepareArgs& a, int64_t p)
 //    counter of 16 bits per key in LDS (51 KB); an atomic add gives a pair its rank
 //    among those of its key, a scan of the counters every key's first place.
 //  - otherwise the keys and pair indices for the radix sort, as far as there are pairs.
-// Bound by latency: for 10,000 pairs the three copies, three clears, key and five sort
-// kernels that did this took 82 us from the first to the alignment's start (graph
-// replay), with launch gaps of 3 to 8 us each; as one launch, 400 us of the 437 us that
-// 10,000 short reads took are left, and 315 of 400 us for a call of one read.
+// Bound by latency.  Three copies, three clears, the keys and five sort kernels did this
+// before, with launch gaps of 3 to 8 us between them: 82 us from the first to the
+// alignment's start for 10,000 pairs (graph replay).  As one launch it took 37 us off a
+// batch of 10,000 short reads (437 us) and 84 off a call of one read (399 us).
 constexpr int kBins = kClasses << kRowBits;
 constexpr int kSmallThreads = 1024, kSmallEach = kSmallSort / kSmallThreads;
 constexpr int kScanEach = (kBins / 2 + kSmallThreads - 1) / kSmallThreads; // dwords (two counters) per thread

@@ -129,6 +129,13 @@ int grid_for(const Exec& ex, int kind, int K, int lds, int64_t nquads)
     return (int)std::max<int64_t>(1, std::min<int64_t>(full, nquads));
 }
 
+// A kind as launch statistics report it.
+int reported_kind(int kind)
+{
+    if (kind & kHalfPairs) return kByteProfile | kReportedPairs;
+    return kind & kReportedKind;
+}
+
 // Launch one kernel between two timing events.
 int launch_timed(Exec& ex, hipStream_t stream, int kind, int K, int grid, int lds, KernelArgs& a, void* bnd)
 {
@@ -142,7 +149,7 @@ int launch_timed(Exec& ex, hipStream_t stream, int kind, int K, int grid, int ld
     GBSW_HIP_TRY(hipEventRecord(ex.kev[2 * slot], stream));
     GBSW_HIP_TRY(kernel_launch(kind, K, grid, lds, stream, a));
     GBSW_HIP_TRY(hipEventRecord(ex.kev[2 * slot + 1], stream));
-    ex.launches.push_back({kind & kReportedKind, K, grid, 0, 0, 0.0});
+    ex.launches.push_back({reported_kind(kind), K, grid, 0, 0, 0.0});
     return GBSW_OK;
 }
 

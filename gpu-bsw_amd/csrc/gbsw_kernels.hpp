@@ -30,6 +30,7 @@ constexpr int kRegTables = 0x400;
 constexpr int kWideLanes = 0x800;
 constexpr int kHalfPairs = 0x2000; // eight pairs per wave, one in each half of 16 lanes' registers
 constexpr int kReportedKind = 0x1FF; // the part of a kind that launch statistics report
+constexpr int kReportedPairs = 7;     // and for eight pairs per wave
 inline int sweep_kind(int kind, int form, int flags)
 {
     kind |= flags;

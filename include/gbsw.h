@@ -177,10 +177,11 @@ int gbsw_batch_traceback(gbsw_batch* batch, const gbsw_scoring* scoring, int64_t
 /* One kernel launch of the last gbsw_batch_align (index 0 .. stats.launches-1). */
 typedef struct {
     int32_t kind;             /* 0 plain forward, 1 plain reverse, 2 batched fwd+rev
-                                 int16, 3 batched int32 (saturated pairs), 4 batched
-                                 f16; +256: scores from the substitution table
-                                 (alphabets of 8+ codes) instead of a profile       */
-    int32_t columns_per_lane; /* K: columns per virtual lane (strip = 32*K columns)  */
+                                 int16, 3 batched int32 (pairs past the 16-bit
+                                 range, or that may pass it), 4 batched sweep kernel,
+                                 5 / 6 the split forms of 2 / 4, 7 sweep kernel with
+                                 eight pairs per wave; +256: scores held as bytes   */
+    int32_t columns_per_lane; /* K: columns per (virtual) lane, the widest of the launch */
     int32_t workgroups;       /* grid size (64-lane workgroups)                       */
     int64_t pairs;            /* pairs processed by the launch                        */
     int64_t cells;            /* their sum of |ref|*|query| (0 for the reverse launch)*/
