@@ -50,35 +50,17 @@ __device__ __forceinline__ uint32_t bfi(uint32_t m, uint32_t a, uint32_t b)
     asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "v"(m), "v"(a), "v"(b));
     return r;
 }
-// ---- integer-valued packed f16 (exact for |x| <= 2048)
+// ---- f16 bit patterns of non-negative numbers, which order as integers
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ f16x2 as_h(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
 __device__ __forceinline__ uint32_t raw(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
-// v_pk_add_f16
-__device__ __forceinline__ uint32_t pk_add_f16(uint32_t a, uint32_t b) { return raw(as_h(a) + as_h(b)); }
-// IEEE maximum of both halves (llvm.maximum: v_pk_maximum3_f16 on gfx950, with no
-// canonicalising max per operand, unlike maxnum).  The operands are integers,
-// never NaN, and -0 does not arise (a sum is -0 only if both terms are).
-__device__ __forceinline__ uint32_t pk_max_f16(uint32_t a, uint32_t b)
-{
-    return raw(__builtin_elementwise_maximum(as_h(a), as_h(b)));
-}
-// v_pk_maximum3_f16 (gfx950): max of three per half.
+// v_pk_maximum3_f16 (gfx950): max of three per half.  The IEEE maximum (unlike maxnum)
+// takes no canonicalising max per operand; the operands are never NaN.
 __device__ __forceinline__ uint32_t pk_max3_f16(uint32_t a, uint32_t b, uint32_t c)
 {
     return raw(__builtin_elementwise_maximum(__builtin_elementwise_maximum(as_h(a), as_h(b)), as_h(c)));
 }
-// 0xFFFF in each half where a < b, else 0: the sign of a - b (exact, and +0 when
-// equal), spread by v_pk_ashrrev_i16.
-__device__ __forceinline__ uint32_t pk_lt_mask_f16(uint32_t a, uint32_t b)
-{
-    return raw(as_s(raw(as_h(a) - as_h(b))) >> (s16x2){15, 15});
-}
 __host__ __device__ inline uint16_t f16_bits(int32_t x) { return __builtin_bit_cast(uint16_t, (_Float16)x); }
-__device__ __forceinline__ int32_t f16_int(uint32_t bits16)
-{
-    return (int32_t)__builtin_bit_cast(_Float16, (uint16_t)bits16);
-}
 
 // v_bfi_b32 with a wave-uniform (SGPR) second operand.
 __device__ __forceinline__ uint32_t bfi_s(uint32_t m, uint32_t a, uint32_t b)
