@@ -995,8 +995,8 @@ int gbsw_align(gbsw_context* ctx, const gbsw_scoring* sc, int32_t mode, int64_t 
     constexpr int64_t kStagedResults = 16384;
     int32_t* pinned = nullptr;
     if (!rc && n && n <= kStagedResults) {
-        GBSW_HIP_TRY(b->results.reserve(sizeof(int32_t) * 5 * (size_t)n));
-        pinned = b->results.as<int32_t>();
+        if (b->results.reserve(sizeof(int32_t) * 5 * (size_t)n) == hipSuccess) pinned = b->results.as<int32_t>();
+        else (void)hipGetLastError(); // (copied after the job, then)
     }
     if (!rc) {
         rc = batch_align_on(b, ctx->ex, sc, mode, pinned);
