@@ -866,6 +866,8 @@ int plan_batched(Exec& ex, const Job& job, int max_sub, bool p8, const SweepChoi
         sizes();
     };
     make(may_split);
+    for (const BucketPlan& b : plan)
+        if (b.ranges.size() > (size_t)kMaxRanges) return fail(GBSW_E_INTERNAL, "a launch has too many geometry ranges");
     if (ex.fixed) {
         // preallocated buffers (a serving slot): without the split form where its
         // boundary slots and bookkeeping do not fit
@@ -959,7 +961,7 @@ int record_batched(Exec& ex, const Job& job, KernelArgs a, const std::vector<Buc
         a.queue = ex.queue.as<uint32_t>() + kXcds * i;
         a.bnd_rows = std::max(1, bk.max_rows);
         a.kmax = b.K;
-        a.nranges = (int32_t)std::min<size_t>(kMaxRanges, b.ranges.size());
+        a.nranges = (int32_t)b.ranges.size(); // (plan_batched: at most kMaxRanges)
         for (int32_t r = 0; r < a.nranges; ++r) a.ranges[r] = b.ranges[(size_t)r];
         a.sat_limit = b.sat_limit;
         std::memset(&a.split, 0, sizeof(a.split));

@@ -116,8 +116,11 @@ constexpr int kSortBits = 6 + kRowBits;
 static_assert(kClasses <= 64, "class bits of the sort key");
 
 // Work of a sweep launch: sets of pairs in work order, the sets that start below
-// pair `end` in geometry K (columns per virtual lane).
-constexpr int kMaxRanges = 16;
+// pair `end` in geometry K (columns per virtual lane).  Room for a range per class:
+// neighbouring classes may well differ (with one pair per wave the K of the fewest
+// strips goes 8, 6, 8, 5, ... along classes of 512 columns).
+constexpr int kMaxRanges = kFineClasses;
+static_assert(kMaxRanges >= kClasses, "a range per class");
 struct SetRange {
     int32_t end, K;
 };
