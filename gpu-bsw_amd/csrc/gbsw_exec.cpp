@@ -788,14 +788,14 @@ bool plan_is_fine(const std::vector<BucketPlan>& plan)
 // range, option F16 off): one per geometry.  A multi-strip launch is split when it
 // has too few quads to keep every workgroup busy for two rounds (on the 200k-pair
 // DNA mix: 1765 vs 827 GCUPS at 1.4 quads per workgroup; 988 vs 1275 on protein at
-// 2.7).
-void plan_int16(const Exec& ex, const Job& job, int max_sub, bool p8, int kclamp, bool may_split,
+// 2.7).  one_launch: all pairs in one launch, in the geometry of the longest.
+void plan_int16(const Exec& ex, const Job& job, int max_sub, bool p8, int kclamp, bool may_split, bool one_launch,
                 std::vector<BucketPlan>& plan)
 {
     for (const Bucket& bk : job.buckets) {
-        const int K = std::min(kclamp, k_for_cols(bk.max_cols, job.alpha, job.kmodel));
+        const int K = std::min(kclamp, k_for_cols(one_launch ? job.max_cols : bk.max_cols, job.alpha, job.kmodel));
         const int strips = std::max(1, (bk.max_cols + kVirtPerPair * K - 1) / (kVirtPerPair * K));
-        if (plan.empty() || plan.back().K != K || (plan.back().strips > 1) != (strips > 1)) {
+        if (plan.empty() || (!one_launch && (plan.back().K != K || (plan.back().strips > 1) != (strips > 1)))) {
             plan.push_back(BucketPlan{});
             BucketPlan& b = plan.back();
             b.bk.begin = bk.begin;
@@ -858,10 +858,10 @@ int plan_batched(Exec& ex, const Job& job, int max_sub, bool p8, const SweepChoi
             }
         }
     };
-    auto make = [&](bool split) {
+    auto make = [&](bool split, bool one_launch = false) {
         plan.clear();
         if (sw.ok) plan_sweeps(ex, job, sw, max_sub, split, asym, plan);
-        else plan_int16(ex, job, max_sub, p8, kclamp, split, plan);
+        else plan_int16(ex, job, max_sub, p8, kclamp, split, one_launch, plan);
         for (BucketPlan& b : plan) set_grid(b);
         sizes();
     };
@@ -878,6 +878,13 @@ int plan_batched(Exec& ex, const Job& job, int max_sub, bool p8, const SweepChoi
             BucketPlan* w = nullptr;
             for (BucketPlan& b : plan)
                 if (!plan_is_split(b) && b.strips > 1 && b.grid > 1 && (!w || b.grid > w->grid)) w = &b;
+            if (!w && plan.size() > 1 && !sw.ok) {
+                // a workgroup per launch is too much still: all pairs in one launch, which
+                // needs the rows of one workgroup (a server's slots hold that much at
+                // least; sweep plans have one launch with boundary rows anyway)
+                make(false, true);
+                continue;
+            }
             if (!w) return fail(GBSW_E_RANGE, "strip boundary rows exceed the preallocated scratch");
             w->grid = std::max(1, w->grid / 2);
             sizes();

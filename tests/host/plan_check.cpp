@@ -118,6 +118,37 @@ const char* check(std::vector<Len> v, int alphabet, bool split, bool fixed, int*
     return nullptr;
 }
 
+// A serving slot of `bnd_bytes` of boundary rows and a scoring of the int16 kernels:
+// the job is planned, not refused.
+const char* check_slot(const std::vector<Len>& v, int alphabet, size_t bnd_bytes)
+{
+    const int alpha = alphabet == GBSW_DNA ? 5 : 24;
+    Job j = job_of(v, alphabet, alpha);
+    Exec ex;
+    ex.num_cu = 256;
+    ex.fixed = true;
+    // (views: sizes count, nothing is read or written)
+    ex.bnd.view((void*)256, bnd_bytes);
+    ex.queue.view((void*)256, 4 * kXcds * 64);
+    ex.split_buf.view((void*)256, (size_t)1 << 30);
+    SweepChoice sw;
+    sw.ok = false;
+    std::vector<BucketPlan> plan;
+    if (plan_batched(ex, j, 3, alphabet == GBSW_PROTEIN, sw, false, 1 << 30, plan)) return last_error_text();
+    size_t end = 0;
+    int64_t pairs = 0;
+    for (const BucketPlan& b : plan) {
+        const size_t rows = 4 * (size_t)kPairsPerWave * (size_t)b.bk.max_rows * (size_t)b.grid * (plan_is_split(b) ? 2 : 1);
+        if (b.grid < 1) return "an empty grid";
+        if (b.strips > 1) end = std::max(end, 4 * b.bnd_at + rows);
+        if ((b.bk.max_cols + kVirtPerPair * b.K - 1) / (kVirtPerPair * b.K) > b.strips) return "more strips than planned";
+        pairs += b.bk.count;
+    }
+    if (end > bnd_bytes) return "boundary rows past the slot's";
+    if (pairs != j.n) return "not every pair in a launch";
+    return nullptr;
+}
+
 } // namespace
 } // namespace gbsw
 
@@ -155,6 +186,11 @@ int main()
         for (int x = 0; x < n; ++x) {
             const int c = (int)std::exp(lo + (hi - lo) * real());
             v.push_back({std::min(65000, (int)(c * (1 + 3 * real() * real()))), std::max(0, c - (mix % 7 == 0 && x == 0 ? c : 0))});
+        }
+        // (4 x 65,000 x 4: the least a server takes)
+        if (const char* e = check_slot(v, mix & 1, (size_t)4 * 65000 * 4)) {
+            std::printf("a slot of the least boundary rows, pairs %zu: %s\n", v.size(), e);
+            return 1;
         }
         if (!run(v, mix & 1 ? GBSW_PROTEIN : GBSW_DNA, "random mix")) return 1;
     }
