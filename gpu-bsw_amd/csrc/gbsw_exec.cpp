@@ -389,6 +389,10 @@ SweepChoice sweep_choice(const std::vector<int16_t>& sub, int alpha, int32_t gap
     // and one substitution on top of its best; the strict reverse pass keeps kRevLow
     // below zero)
     c.sat_limit = (int32_t)(0x7C00 - kRevLow - offset - 2 * ge - max_sub - 4);
+    double same = 0, all = 0;
+    for (int r = 0; r < alpha; ++r) same += sub[(size_t)(r * alpha + r)];
+    for (int16_t v : sub) all += v;
+    c.typical = 0.875 * same / alpha + (alpha > 1 ? 0.125 * (all - same) / ((double)alpha * (alpha - 1)) : 0.0);
     return c;
 }
 
@@ -732,19 +736,24 @@ void int32_split_geometry(const Job& job, BucketPlan& b)
     b.unit = best * kPasses;
 }
 
-// The classes of the longest pairs, as far as one may well pass the 16-bit range (its
-// columns at 0.75 of the best score each, which reads of 10 % errors reach), take int32
-// cells at once, beside the others, where their strips' waves are few (two per SIMD).
-// Recomputed after the others, two of 400 long reads doubled the time, 21.5 ms where
-// this takes 12.2: their chain of strips is as long as everything else.
-size_t plan_int32(const Exec& ex, const Job& job, const SweepChoice& sw, int max_sub, std::vector<BucketPlan>& plan)
+// The classes of the longest pairs, as far as an alike pair of them passes the 16-bit
+// range (SweepChoice::typical per column, one residue in eight changed: 2.25 of +3/-3,
+// 4.9 of BLOSUM62), take int32 cells at once, beside the others, where their strips'
+// waves are few (two per SIMD).  Recomputed after the others, two of 400 long reads
+// doubled the time, 21.5 ms where this takes 12.2, and 36 of 100 alike proteins of up to
+// 8,192 columns 15.3 ms where this takes 8.2: their chain of strips is as long as
+// everything else.  Pairs that are not alike pay for it: 100 unrelated proteins of up to
+// 8,192 columns 8.3 ms, 7.2 in 16 bits.  (By the largest score of the table, 11 of W
+// against W, proteins from 3,576 columns on paid too: 20, 100 and 500 of up to 4,096
+// columns 4.8, 5.7 and 8.0 ms instead of 4.4, 4.8 and 6.7.)
+size_t plan_int32(const Exec& ex, const Job& job, const SweepChoice& sw, std::vector<BucketPlan>& plan)
 {
     if (ex.fixed || !sw.wide_ok) return 0;
     BucketPlan b;
     size_t n = 0;
     for (; n < job.buckets.size(); ++n) {
         const Bucket& bk = job.buckets[n];
-        if (0.75 * max_sub * (double)bk.max_cols < (double)sw.sat_limit) break;
+        if (sw.typical * (double)bk.max_cols < (double)sw.sat_limit) break;
         b.bk.add(bk);
     }
     if (!n) return 0;
@@ -759,10 +768,10 @@ size_t plan_int32(const Exec& ex, const Job& job, const SweepChoice& sw, int max
 
 // Eight pairs per wave: jobs with two such waves per SIMD and more (fewer leave SIMDs
 // idle) and register tables, where the estimate is less.
-void plan_sweeps(const Exec& ex, const Job& job, const SweepChoice& sw, int max_sub, bool may_split, bool asym,
+void plan_sweeps(const Exec& ex, const Job& job, const SweepChoice& sw, bool may_split, bool asym,
                  std::vector<BucketPlan>& plan)
 {
-    const size_t wide = may_split ? plan_int32(ex, job, sw, max_sub, plan) : 0;
+    const size_t wide = may_split ? plan_int32(ex, job, sw, plan) : 0;
     if (wide) {
         const std::vector<Bucket> rest(job.buckets.begin() + (std::ptrdiff_t)wide, job.buckets.end());
         if (!rest.empty()) (void)plan_sweeps_over(ex, job, rest, sw, may_split, false, plan);
@@ -860,7 +869,7 @@ int plan_batched(Exec& ex, const Job& job, int max_sub, bool p8, const SweepChoi
     };
     auto make = [&](bool split, bool one_launch = false) {
         plan.clear();
-        if (sw.ok) plan_sweeps(ex, job, sw, max_sub, split, asym, plan);
+        if (sw.ok) plan_sweeps(ex, job, sw, split, asym, plan);
         else plan_int16(ex, job, max_sub, p8, kclamp, split, one_launch, plan);
         for (BucketPlan& b : plan) set_grid(b);
         sizes();

@@ -203,6 +203,7 @@ struct SweepChoice {
     bool wide_ok = false; // the int32 sweep kernels
     int form = 0; // ProfileForm
     int32_t base = 0, sat_limit = 0;
+    double typical = 0; // score per column of a pair with one residue in eight changed
 };
 SweepChoice sweep_choice(const std::vector<int16_t>& sub, int alpha, int32_t gap_open, int32_t gap_extend,
                          int32_t max_sub, bool bytes);

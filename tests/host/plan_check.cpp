@@ -75,7 +75,7 @@ const char* check(std::vector<Len> v, int alphabet, bool split, bool fixed, int*
     ex.num_cu = 256;
     ex.fixed = fixed;
     std::vector<BucketPlan> plan;
-    plan_sweeps(ex, j, sw, max_sub, split, false, plan);
+    plan_sweeps(ex, j, sw, split, false, plan);
     // the work order (k_prepare): classes of longer pairs first, then rows
     const bool fine = plan_is_fine(plan);
     std::sort(v.begin(), v.end(), [&](const Len& x, const Len& y) {
@@ -116,6 +116,24 @@ const char* check(std::vector<Len> v, int alphabet, bool split, bool fixed, int*
     for (int t : taken)
         if (t != 1) return "a pair in no launch, or in two";
     return nullptr;
+}
+
+// Pairs that a plan puts on int32 cells at once: a table's mean identical and mean other
+// score, the rest of the diagonal alike but for one code of `rare`.
+int64_t int32_pairs(const std::vector<Len>& v, int alphabet, int alpha, int16_t same, int16_t other, int16_t rare)
+{
+    Job j = job_of(v, alphabet, alpha);
+    std::vector<int16_t> sub((size_t)(alpha * alpha), other);
+    for (int c = 0; c < alpha; ++c) sub[(size_t)(c * alpha + c)] = same;
+    sub[0] = rare;
+    Exec ex;
+    ex.num_cu = 256;
+    std::vector<BucketPlan> plan;
+    plan_sweeps(ex, j, sweep_choice(sub, alpha, -6, -1, std::max(same, rare), true), true, false, plan);
+    int64_t n = 0;
+    for (const BucketPlan& b : plan)
+        if ((b.kind & 0xFF) == kBatchedWide) n += b.bk.count;
+    return n;
 }
 
 // A serving slot of `bnd_bytes` of boundary rows and a scoring of the int16 kernels:
@@ -177,6 +195,28 @@ int main()
         return 1;
     }
     g_occupancy = 16;
+    // 20 to 300 proteins of up to 4,096 columns stay in 16 bits though one residue scores 11
+    // with itself (identical ones of 4,096 score about 22,000); ten of 8,000 do not, nor do
+    // ten reads of 16,000 at +3/-3
+    for (int n : {20, 100, 300}) {
+        std::vector<Len> v;
+        for (int x = 0; x < n; ++x) v.push_back({8000, 1024 + 3072 * x / (n - 1)});
+        if (const int64_t k = int32_pairs(v, GBSW_PROTEIN, 20, 5, -1, 11)) {
+            std::printf("%d of %d proteins on int32 cells\n", (int)k, n);
+            return 1;
+        }
+    }
+    {
+        std::vector<Len> aa(10, Len{9000, 8000}), reads(10, Len{20000, 16000});
+        for (int x = 0; x < 50; ++x) {
+            aa.push_back({3000, 2000});
+            reads.push_back({6000, 4000});
+        }
+        if (int32_pairs(aa, GBSW_PROTEIN, 20, 5, -1, 11) != 10 || int32_pairs(reads, GBSW_DNA, 4, 3, -3, 3) != 10) {
+            std::printf("pairs that pass the 16-bit range not on int32 cells\n");
+            return 1;
+        }
+    }
     std::mt19937 rng(5);
     auto real = [&]() { return std::uniform_real_distribution<double>(0.0, 1.0)(rng); };
     for (int mix = 0; mix < 3000; ++mix) {
