@@ -958,10 +958,16 @@ int gbsw_batch_autotune(gbsw_batch* b, const gbsw_scoring* sc, int32_t repeats, 
     const int current = job.kmodel;
     int best = -1;
     double best_ms = 1e300;
+    std::vector<std::string> tried;
     for (int i = 0; i < kGeometryModels; ++i) {
         const int m = i == 0 ? current : (i <= current ? i - 1 : i);
         use_model(m);
-        int rc = GBSW_OK;
+        // models whose plan is one already timed add nothing
+        std::string plan;
+        int rc = batched_plan_text(ctx->ex, job, sc, &plan);
+        if (rc) return rc;
+        if (std::find(tried.begin(), tried.end(), plan) != tried.end()) continue;
+        tried.push_back(std::move(plan));
         double m_ms = 1e300;
         for (int r = 0; !rc && r < repeats + 1; ++r) {
             rc = gbsw_batch_align(b, sc, GBSW_BATCHED);

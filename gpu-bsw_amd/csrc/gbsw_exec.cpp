@@ -998,6 +998,20 @@ int record_batched(Exec& ex, const Job& job, KernelArgs a, const std::vector<Buc
     return GBSW_OK;
 }
 
+// Every launch of a plan, as bytes.
+std::string plan_text(const std::vector<BucketPlan>& plan)
+{
+    std::string k;
+    for (const BucketPlan& b : plan) {
+        const Bucket& bk = b.bk;
+        const int64_t f[] = {b.kind, b.K, b.grid, b.lds, b.strips, (int64_t)b.bnd_at, (int64_t)b.split_at,
+                             bk.begin, bk.count, bk.max_cols, bk.max_rows};
+        k.append((const char*)f, sizeof(f));
+        k.append((const char*)b.ranges.data(), sizeof(SetRange) * b.ranges.size());
+    }
+    return k;
+}
+
 // What a captured graph depends on besides the batch's bytes: the scoring, the
 // options, the addresses of the context buffers it writes, and each bucket's
 // slice of the sort order (baked into the captured launch arguments; another
@@ -1016,18 +1030,42 @@ std::string graph_key(const Exec& ex, const Job& job, const gbsw_scoring* sc, co
     k.append((const char*)opts, sizeof(opts));
     const int64_t jf[] = {job.kmodel, job.n, (int64_t)(uintptr_t)job.order};
     k.append((const char*)jf, sizeof(jf));
-    for (size_t i = 0; i < plan.size(); ++i) {
-        const BucketPlan& b = plan[i];
-        const Bucket& bk = b.bk;
-        const int64_t f[] = {b.kind, b.K, b.grid, b.lds, b.strips, (int64_t)b.bnd_at, (int64_t)b.split_at,
-                             bk.begin, bk.count, bk.max_cols, bk.max_rows};
-        k.append((const char*)f, sizeof(f));
-        k.append((const char*)b.ranges.data(), sizeof(SetRange) * b.ranges.size());
-    }
-    return k;
+    return k + plan_text(plan);
+}
+
+// Geometries are chosen for the byte profile of a large alphabet; scores outside int8
+// take the int16 profile, in the widest geometry that fits.
+int widest_k(const Job& job, bool p8)
+{
+    return (byte_profile_alphabet(job.alpha) && !p8) ? max_k_for(job.alpha, false) : 1 << 30;
+}
+
+// The plan of the batched form for a job and the tables of a scoring (prepare_scoring).
+int plan_scored(Exec& ex, const Job& job, const gbsw_scoring* sc, const std::vector<int16_t>& sub, int max_sub, bool p8,
+                bool f16p8, SweepChoice& sw, std::vector<BucketPlan>& plan)
+{
+    // scores of the sweep kernels: bytes where they fit an int8 profile (large
+    // alphabets) or have at most three significant bits (small ones), else 16 bits
+    sw = sweep_choice(sub, job.alpha, sc->gap_open, sc->gap_extend, max_sub,
+                      byte_profile_alphabet(job.alpha) ? p8 : f16p8);
+    sw.ok = sw.ok && ex.f16;
+    return plan_batched(ex, job, max_sub, p8, sw, table_is_asymmetric(sc, job), widest_k(job, p8), plan);
 }
 
 } // namespace
+
+int batched_plan_text(Exec& ex, const Job& job, const gbsw_scoring* sc, std::string* text)
+{
+    std::vector<int16_t> sub;
+    std::vector<BucketPlan> plan;
+    int max_sub = 0;
+    bool p8 = false, f16p8 = false;
+    SweepChoice sw;
+    int rc = prepare_scoring(job, sc, sub, &max_sub, &p8, &f16p8);
+    if (!rc) rc = plan_scored(ex, job, sc, sub, max_sub, p8, f16p8, sw, plan);
+    if (!rc) *text = plan_text(plan);
+    return rc;
+}
 
 int enqueue_job(Exec& ex, const Job& job, const gbsw_scoring* sc, int mode)
 {
@@ -1040,9 +1078,7 @@ int enqueue_job(Exec& ex, const Job& job, const gbsw_scoring* sc, int mode)
     if (rc) return rc;
     ex.max_sub = max_sub;
     ex.p8 = p8;
-    // geometries were chosen for the byte profile of a large alphabet; scores
-    // outside int8 take the int16 profile, in the widest geometry that fits
-    const int kclamp = (byte_profile_alphabet(job.alpha) && !p8) ? max_k_for(job.alpha, false) : 1 << 30;
+    const int kclamp = widest_k(job, p8);
     hipStream_t st0 = ex.stream;
     if (job.n == 0) {
         GBSW_HIP_TRY(hipEventRecord(ex.ev_start, st0));
@@ -1100,14 +1136,10 @@ int enqueue_job(Exec& ex, const Job& job, const gbsw_scoring* sc, int mode)
         return GBSW_OK;
     }
     std::vector<BucketPlan> plan;
-    // scores of the sweep kernels: bytes where they fit an int8 profile (large
-    // alphabets) or have at most three significant bits (small ones), else 16 bits
-    SweepChoice sw = sweep_choice(sub, job.alpha, sc->gap_open, sc->gap_extend, max_sub,
-                                  byte_profile_alphabet(job.alpha) ? p8 : f16p8);
-    sw.ok = sw.ok && ex.f16;
-    a.base = sw.base;
-    rc = plan_batched(ex, job, max_sub, p8, sw, a.asym != 0, kclamp, plan);
+    SweepChoice sw;
+    rc = plan_scored(ex, job, sc, sub, max_sub, p8, f16p8, sw, plan);
     if (rc) return rc;
+    a.base = sw.base;
     const size_t sub_bytes = sizeof(int16_t) * sub.size();
     if (!ex.graphs || ex.fixed || !job.graph) {
         GBSW_HIP_TRY(hipEventRecord(ex.ev_start, st0));

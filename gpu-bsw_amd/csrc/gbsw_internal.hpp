@@ -232,6 +232,9 @@ void* noalloc_scratch(int device);
 // Asynchronous: ex.ev_stop is recorded after the last kernel and the status words
 // are copied to ex.status_host.
 int enqueue_job(Exec& ex, const Job& job, const gbsw_scoring* sc, int mode);
+// The launches of the batched form for a job (kernels, geometries, grids), as bytes: equal
+// for two geometry models that make one plan.
+int batched_plan_text(Exec& ex, const Job& job, const gbsw_scoring* sc, std::string* text);
 // After ex.ev_stop completed: recompute int16-saturated pairs with the int32
 // kernel (synchronously, rare), check the status words and collect timings.
 int complete_job(Exec& ex, const Job& job, const gbsw_scoring* sc, double* device_ms);
