@@ -184,20 +184,26 @@ struct HostPart {
 // is slower than the link (100 MB: pinned 1.8 ms, the runtime's pageable copy 3.7 and
 // more for memory it has not pinned before, this 2.4; 2, 4 and 8 MB pieces 2.7, 2.4 and
 // 2.3, two to eight threads alike).  `meanwhile` runs on the calling thread, before it
-// joins in.  Blocks until the sources may be reused.
+// joins in.  Blocks until the sources may be reused.  False: there is no pinned memory
+// for the ring, and nothing was done.
 constexpr size_t kUpPiece = (size_t)4 << 20;
 constexpr int kUpSlots = 6, kUpThreads = 4;
 template <class F>
-hipError_t upload_large(gbsw_context* ctx, hipStream_t st, const HostPart* parts, int nparts, F&& meanwhile)
+bool upload_large(gbsw_context* ctx, hipStream_t st, const HostPart* parts, int nparts, F&& meanwhile, hipError_t* result)
 {
     std::lock_guard<std::mutex> lock(ctx->up_mu);
     hipError_t e = ctx->up_ring.reserve(kUpPiece * kUpSlots);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
     while (e == hipSuccess && ctx->up_events.size() < (size_t)kUpSlots) {
         hipEvent_t ev;
         e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
         if (e == hipSuccess) ctx->up_events.push_back(ev);
     }
-    if (e != hipSuccess) return e;
+    *result = e;
+    if (e != hipSuccess) return true;
     std::vector<HostPart> pieces;
     for (int x = 0; x < nparts; ++x)
         for (size_t at = 0; at < parts[x].bytes; at += kUpPiece)
@@ -238,7 +244,8 @@ hipError_t upload_large(gbsw_context* ctx, hipStream_t st, const HostPart* parts
     work();
     for (std::thread& t : helpers) t.join();
     const hipError_t se = hipStreamSynchronize(st); // the ring is free again
-    return error.load() != (int)hipSuccess ? (hipError_t)error.load() : se;
+    *result = error.load() != (int)hipSuccess ? (hipError_t)error.load() : se;
+    return true;
 }
 
 bool is_pinned(const void* p)
@@ -254,7 +261,8 @@ bool is_pinned(const void* p)
 // Upload pairs into batch b (new, or one reused: its device buffers only grow),
 // with ex's stream and geometry model.  `staged` (not for the allocation-free entry
 // point): through pinned staging; a block of up to kUpStaged bytes is then one
-// transfer, and may still be under way on ex.stream on return.
+// transfer, and may still be under way on ex.stream on return.  Where pinned memory is
+// not to be had, the same copies go from pageable memory.
 constexpr size_t kUpStaged = (size_t)1 << 20, kUpLarge = (size_t)8 << 20;
 // Residues whose set of byte values the host finds (about a byte per cycle: 20 us at
 // most); more are scanned on the device, which costs a launch and a wait (about 30 us).
@@ -309,11 +317,16 @@ static int batch_fill(gbsw_batch* b, gbsw_context* ctx, Exec& ex, bool staged, i
     if (e == hipSuccess) e = b->vals.reserve(4 * np);
     if (e == hipSuccess) e = b->order.reserve(4 * np);
     if (e == hipSuccess) e = b->sort_temp.reserve(sort_bytes);
-    const bool one_block = staged && L.total <= kUpStaged;
-    const bool pinned_offs = staged && b->one_shot; // (kept for the next call)
-    const size_t offs_bytes = L.ref - L.ref_off;
-    const size_t masks_at = one_block ? L.total : pinned_offs ? offs_bytes : 0, masks_bytes = 32 * kPresenceBlocks;
-    if (e == hipSuccess && staged) e = b->stage.reserve(masks_at + masks_bytes);
+    const size_t offs_bytes = L.ref - L.ref_off, masks_bytes = 32 * kPresenceBlocks;
+    bool one_block = staged && L.total <= kUpStaged;
+    bool pinned_offs = staged && b->one_shot; // (kept for the next call)
+    bool host_scan = ref_bytes + qry_bytes <= kHostScan;
+    const size_t masks_at = one_block ? L.total : pinned_offs ? offs_bytes : 0;
+    if (staged && b->stage.reserve(masks_at + masks_bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        staged = one_block = pinned_offs = false;
+        host_scan = true; // (nowhere for the device's masks)
+    }
     std::vector<uint64_t> offs;
     uint8_t* h = b->stage.as<uint8_t>();
     if (e == hipSuccess && !one_block && !pinned_offs) {
@@ -352,9 +365,8 @@ static int batch_fill(gbsw_batch* b, gbsw_context* ctx, Exec& ex, bool staged, i
             if (qry_bytes) std::memcpy(h + L.qry, qp, qry_bytes);
             e = hipMemcpyAsync(dev, h, L.qry + qry_bytes, hipMemcpyHostToDevice, st);
         } else {
-            if (staged && L.total >= kUpLarge && !(ref_bytes && is_pinned(rp)) && !(qry_bytes && is_pinned(qp))) {
-                e = upload_large(ctx, st, parts, 2, pairs_pass);
-            } else {
+            if (!(staged && L.total >= kUpLarge && !(ref_bytes && is_pinned(rp)) && !(qry_bytes && is_pinned(qp)) &&
+                  upload_large(ctx, st, parts, 2, pairs_pass, &e))) {
                 for (const HostPart& x : parts)
                     if (e == hipSuccess && x.bytes) e = hipMemcpyAsync(x.dst, x.src, x.bytes, hipMemcpyHostToDevice, st);
                 pairs_pass();
@@ -366,7 +378,7 @@ static int batch_fill(gbsw_batch* b, gbsw_context* ctx, Exec& ex, bool staged, i
     // The residue codes need the set of byte values in the batch (every distinct
     // DNA byte is a code; protein bytes must be < 91).
     uint32_t seen[8] = {0};
-    if (e == hipSuccess && ref_bytes + qry_bytes <= kHostScan) {
+    if (e == hipSuccess && host_scan) {
         uint8_t has[256] = {0};
         for (uint64_t x = 0; x < ref_bytes; ++x) has[rp[x]] = 1;
         for (uint64_t x = 0; x < qry_bytes; ++x) has[qp[x]] = 1;
