@@ -876,7 +876,8 @@ int plan_batched(Exec& ex, const Job& job, int max_sub, bool p8, const SweepChoi
     };
     make(may_split);
     for (const BucketPlan& b : plan)
-        if (b.ranges.size() > (size_t)kMaxRanges) return fail(GBSW_E_INTERNAL, "a launch has too many geometry ranges");
+        if (sw.ok && (b.ranges.empty() || b.ranges.size() > (size_t)kMaxRanges || b.ranges.back().end != b.bk.count))
+            return fail(GBSW_E_INTERNAL, "the geometry ranges of a launch do not hold its pairs");
     if (ex.fixed) {
         // preallocated buffers (a serving slot): without the split form where its
         // boundary slots and bookkeeping do not fit
