@@ -365,30 +365,49 @@ bool f16_high_byte_exact(int32_t s)
 }
 
 SweepChoice sweep_choice(const std::vector<int16_t>& sub, int alpha, int32_t gap_open, int32_t gap_extend,
-                         int32_t max_sub, bool bytes)
+                         int32_t max_sub, bool bytes, int32_t max_cols)
 {
     SweepChoice c;
-    const int32_t ge = -gap_extend, go = -gap_open, bias = ge + go;
+    const int32_t ge = -gap_extend, go = -gap_open, cost = ge + go;
     int32_t lo = 1 << 30, hi = -(1 << 30);
     for (int r = 0; r < alpha; ++r)
         for (int q = 0; q < alpha; ++q) {
-            lo = std::min<int32_t>(lo, sub[(size_t)(r * alpha + q)] + bias);
-            hi = std::max<int32_t>(hi, sub[(size_t)(r * alpha + q)] + bias);
+            lo = std::min<int32_t>(lo, sub[(size_t)(r * alpha + q)]);
+            hi = std::max<int32_t>(hi, sub[(size_t)(r * alpha + q)]);
         }
+    // Tables hold score + bias; 0 is padding, which must score below zero.  The step adds
+    // score + open + extend: as it stands in the tables where that fits (bias = cost),
+    // else, as bytes, from the smallest score up, the rest by `shift` (Sweep16Shifted).
+    // (100,000 proteins with gaps of -2/-1 8.2 ms, with a 16-bit profile 11.6; a million
+    // reads with gaps that cost nothing 27.9 ms, with a 16-bit profile 39.8, on the int16
+    // kernels 47.6.)
+    c.bias = cost;
+    int32_t pad = cost > 0 ? -cost : -1; // (16-bit tables hold a padding word)
+    c.form = kProfWords;
+    if (bytes && cost > 0 && lo + cost >= 0 && hi + cost <= 255) {
+        c.form = kProfBytes;
+    } else if (bytes && hi - std::min(lo, -1) <= 255) {
+        c.form = kProfBytes;
+        c.bias = -std::min(lo, -1);
+        pad = -c.bias;
+    }
+    if (c.form == kProfBytes && alpha <= kRegAlpha) c.form = kProfRegs;
+    c.shift = cost - c.bias;
     // every value stays non-negative: the smallest is a zero cell's Ho plus the
-    // smallest biased score
-    c.base = go + std::max(0, -lo) + 4;
+    // smallest score
+    c.base = go + std::max(0, -(std::min(lo, pad) + cost)) + 4;
     const int64_t offset = (int64_t)c.base + (int64_t)ge * (kRebase + 40);
-    // the padding scores -(open + extend), which must be negative; the running
-    // offset and the scores leave most of the range to the cell values
-    c.ok = bias >= 1 && offset <= 8192 && max_sub <= 4096 && lo > -16384 && hi < 16384;
     // int32 cells: any range; the profile holds the biased scores in 16 bits
-    c.wide_ok = bias >= 1 && lo > -32768 && hi < 32768;
-    c.form = (bytes && lo >= 0 && hi <= 255) ? (alpha <= kRegAlpha ? kProfRegs : kProfBytes) : kProfWords;
+    c.wide_ok = cost >= 1 && lo + cost > -32768 && hi + cost < 32768;
     // a pair below this never formed a value past 0x7C00 (largest offset, gap step
     // and one substitution on top of its best; the strict reverse pass keeps kRevLow
     // below zero)
     c.sat_limit = (int32_t)(0x7C00 - kRevLow - offset - 2 * ge - max_sub - 4);
+    // The running offset and the scores leave most of the range to the cell values, or
+    // enough for any pair of the job.  (A million reads with gaps of -600/-100 25.4 ms, on
+    // the int16 kernels 33.7.)
+    c.ok = (offset <= 8192 || (offset <= 24576 && (int64_t)max_cols * max_sub < c.sat_limit)) && max_sub <= 4096 &&
+           lo + cost > -16384 && hi + cost < 16384;
     double same = 0, all = 0;
     for (int r = 0; r < alpha; ++r) same += sub[(size_t)(r * alpha + r)];
     for (int16_t v : sub) all += v;
@@ -565,11 +584,12 @@ double plan_sweeps_over(const Exec& ex, const Job& job, const std::vector<Bucket
     const size_t n = cls.size();
     const double thr = occupancy_threshold(job.kmodel);
     auto lds = [&](int G, int K) { return sweep_lds_for(K, job.alpha, sw.form, G); };
+    auto kind_of = [&](int kind, int flags) { return sweep_kind(kind, sw.form, sw.shift ? flags | kShifted : flags); };
     // share of the issue rate of a launch whose widest geometry is K
     auto share = [&](int flags, int G, int K) {
         const int l = lds(G, K);
         if (l > 65536) return 0.0;
-        return issue_share(kernel_occupancy(sweep_kind(kBatchedF16, sw.form, flags), K, l) / 4.0, thr);
+        return issue_share(kernel_occupancy(kind_of(kBatchedF16, flags), K, l) / 4.0, thr);
     };
     struct Option {
         std::vector<GeoCost> cost; // per class
@@ -636,7 +656,7 @@ double plan_sweeps_over(const Exec& ex, const Job& job, const std::vector<Bucket
     if (may_split)
         for (int K : kSweepSplitK) {
             if (lds(kWave, K) > 65536) break;
-            const int kind = sweep_kind(kSplitF16, sw.form, kWideGroup);
+            const int kind = kind_of(kSplitF16, kWideGroup);
             const double s = issue_share(kernel_occupancy(kind, K, lds(kWave, K)) / 4.0, thr);
             Option o;
             o.cap = K;
@@ -690,7 +710,7 @@ double plan_sweeps_over(const Exec& ex, const Job& job, const std::vector<Bucket
             if (!b.ranges.empty() && b.ranges.back().K == c.K) b.ranges.back().end = end;
             else b.ranges.push_back({end, c.K});
         }
-        b.kind = sweep_kind(is_split ? kSplitF16 : kBatchedF16, sw.form, flags);
+        b.kind = kind_of(is_split ? kSplitF16 : kBatchedF16, flags);
         b.lds = lds(G, b.K);
         plan.push_back(b);
     };
@@ -1048,7 +1068,7 @@ int plan_scored(Exec& ex, const Job& job, const gbsw_scoring* sc, const std::vec
     // scores of the sweep kernels: bytes where they fit an int8 profile (large
     // alphabets) or have at most three significant bits (small ones), else 16 bits
     sw = sweep_choice(sub, job.alpha, sc->gap_open, sc->gap_extend, max_sub,
-                      byte_profile_alphabet(job.alpha) ? p8 : f16p8);
+                      byte_profile_alphabet(job.alpha) ? p8 : f16p8, job.max_cols);
     sw.ok = sw.ok && ex.f16;
     return plan_batched(ex, job, max_sub, p8, sw, table_is_asymmetric(sc, job), widest_k(job, p8), plan);
 }
@@ -1141,6 +1161,8 @@ int enqueue_job(Exec& ex, const Job& job, const gbsw_scoring* sc, int mode)
     rc = plan_scored(ex, job, sc, sub, max_sub, p8, f16p8, sw, plan);
     if (rc) return rc;
     a.base = sw.base;
+    a.bias = sw.bias;
+    a.shift = sw.shift;
     const size_t sub_bytes = sizeof(int16_t) * sub.size();
     if (!ex.graphs || ex.fixed || !job.graph) {
         GBSW_HIP_TRY(hipEventRecord(ex.ev_start, st0));
@@ -1205,7 +1227,7 @@ int redo_int32(Exec& ex, const Job& job, const gbsw_scoring* sc, int64_t count)
     bool p8 = false, f16p8 = false;
     int rc = prepare_scoring(job, sc, sub, &max_sub, &p8, &f16p8);
     if (rc) return rc;
-    const SweepChoice sw = sweep_choice(sub, job.alpha, sc->gap_open, sc->gap_extend, max_sub, false);
+    const SweepChoice sw = sweep_choice(sub, job.alpha, sc->gap_open, sc->gap_extend, max_sub, false, job.max_cols);
     if (sw.wide_ok) {
         // One pair per wave; few pairs (up to a wave per SIMD) as strips of the split
         // form: 400 long reads, a few of them past the range, 773 -> 21.5 ms with

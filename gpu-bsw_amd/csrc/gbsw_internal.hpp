@@ -197,16 +197,18 @@ void place_buckets(std::vector<Bucket>& out, const Bucket* by_class, int classes
 int wide_grid_cap(const Exec& ex, int alpha);
 // Whether a scoring runs the sweep kernels (gbsw_sweep.hpp), and how: the profile
 // form, the offset of all cell values, and the score from which a pair may have
-// left the 16-bit range.  bytes: the scores may be held as bytes.
+// left the 16-bit range.  bytes: the scores may be held as bytes; max_cols: the job's
+// longest shorter sequence.
 struct SweepChoice {
     bool ok = false;
     bool wide_ok = false; // the int32 sweep kernels
     int form = 0; // ProfileForm
     int32_t base = 0, sat_limit = 0;
+    int32_t bias = 0, shift = 0; // added to the scores in the tables, and by the step
     double typical = 0; // score per column of a pair with one residue in eight changed
 };
 SweepChoice sweep_choice(const std::vector<int16_t>& sub, int alpha, int32_t gap_open, int32_t gap_extend,
-                         int32_t max_sub, bool bytes);
+                         int32_t max_sub, bool bytes, int32_t max_cols);
 // Scratch bytes of the radix sort for n pairs.
 int sort_scratch_bytes(int64_t n, size_t* bytes);
 

@@ -154,6 +154,7 @@ struct KernelArgs {
     int32_t nranges;
     SetRange ranges[kMaxRanges];
     SplitArgs split;           // split forms only
+    int32_t bias, shift;       // shifted sweep kernels: added to the scores in the tables, and by the step
 };
 
 // Dynamic LDS layout of one 64-lane workgroup; W = profile columns per row

@@ -1067,6 +1067,7 @@ static const void* kernel_for(int kind, int K)
     if (base == kBatchedWide && (kind & kWideGroup)) return sweep_kernel_int32(kind, K);
     if (base == kBatchedF16 || base == kSplitF16) {
         const bool wide = (kind & kWideGroup) != 0;
+        if (kind & kShifted) return wide ? sweep_kernel_shifted_wide(kind, K) : sweep_kernel_shifted(kind);
         if (kind & kHalfPairs) return sweep_kernel_pairs(kind);
         if (kind & kRegTables) return wide ? sweep_kernel_regs_wide(kind, K) : sweep_kernel_regs(kind, K);
         if (kind & kByteProfile) return wide ? sweep_kernel_bytes_wide(kind, K) : sweep_kernel_bytes(kind, K);

@@ -29,6 +29,7 @@ constexpr int kWideGroup = 0x200;
 constexpr int kRegTables = 0x400;
 constexpr int kWideLanes = 0x800;
 constexpr int kHalfPairs = 0x2000; // eight pairs per wave, one in each half of 16 lanes' registers
+constexpr int kShifted = 0x4000;   // byte tables hold the scores from the smallest one up
 constexpr int kReportedKind = 0x1FF; // the part of a kind that launch statistics report
 constexpr int kReportedPairs = 7;     // and for eight pairs per wave
 inline int sweep_kind(int kind, int form, int flags)
@@ -52,6 +53,8 @@ const void* sweep_kernel_regs_wide(int kind, int K);
 const void* sweep_kernel_bytes_wide(int kind, int K);
 const void* sweep_kernel_words_wide(int kind, int K);
 const void* sweep_kernel_pairs(int kind);
+const void* sweep_kernel_shifted(int kind);
+const void* sweep_kernel_shifted_wide(int kind, int K);
 // int32 cells (kBatchedWide | kWideGroup, with kSplitStrips the split form)
 constexpr int kSplitStrips = 0x1000;
 #define GBSW_SWEEP_K32(X) X(2) X(4)

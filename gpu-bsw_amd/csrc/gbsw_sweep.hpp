@@ -13,7 +13,8 @@
 // Recurrence.  With g the cost of extending a gap, o that of opening one, every
 // value is held with the offset phi(s, k) = base + g (t + k), t = 1 + s mod
 // kRebase, k the column within the lane:
-//   D  = Ho(s-1, k-1) + S''            S'' = s(row, col) + o + g (in the tables)
+//   D  = Ho(s-1, k-1) + S''            S'' = s(row, col) + o + g (in the tables; where
+//                                      bytes do not hold it, less a constant: Sweep16Shifted)
 //   H  = max3(D, E, F)
 //   Ho = H + (g - o)                   the state, in place of H
 //   E' = max3(E, Ho, floor(s, k+1))    (next column)
@@ -140,7 +141,7 @@ struct Sweep16 {
     using V = uint32_t;
     using U = uint32_t;
     using B = uint32_t; // strip boundary entry: H | E << 16
-    static constexpr bool kWide = false;
+    static constexpr bool kWide = false, kShifts = false;
     __device__ static U uni(int32_t x) { return (uint32_t)x * 0x00010001u; }
     __device__ static V from(U u) { return u; }
     __device__ static V splat(int32_t x) { return uni(x); }
@@ -151,7 +152,7 @@ struct Sweep16 {
     __device__ static V sub_each(V a, U u) { return raw(as_u(a) - as_u(u)); } // no borrow between the halves
     // + scores: 32-bit while they are non-negative, else per half
     template <bool SIGNED>
-    __device__ static V add(V a, V b)
+    __device__ static V add(V a, V b, U)
     {
         if constexpr (SIGNED) return raw(as_u(a) + as_u(b));
         else return a + b;
@@ -209,6 +210,20 @@ struct Sweep16 {
     __device__ static B zero_bnd() { return 0u; }
 };
 
+// The same where the byte tables hold the scores from the smallest one up: the rest of
+// score + open + extend (KernelArgs::shift) is the third operand of the addition, whose
+// halves do not carry or borrow either.  Apart from Sweep16, since the longer encoding
+// costs every step (1M-pair DNA mix 21.9 -> 22.1 ms, 10k long proteins 64.0 -> 65.4).
+struct Sweep16Shifted : Sweep16 {
+    static constexpr bool kShifts = true;
+    template <bool SIGNED>
+    __device__ static V add(V a, V b, U shift)
+    {
+        static_assert(!SIGNED, "byte forms");
+        return a + b + shift;
+    }
+};
+
 // Sweep32: the same two virtual lanes as two int32 registers, for pairs whose score
 // may exceed the 16-bit range.
 struct Sweep32 {
@@ -217,7 +232,7 @@ struct Sweep32 {
     };
     using U = int32_t;
     using B = uint2; // (H, E)
-    static constexpr bool kWide = true;
+    static constexpr bool kWide = true, kShifts = false;
     __device__ static U uni(int32_t x) { return x; }
     __device__ static V from(U u) { return V{u, u}; }
     __device__ static V splat(int32_t x) { return V{x, x}; }
@@ -226,7 +241,7 @@ struct Sweep32 {
     __device__ static V subu(V a, U u) { return V{a.l - u, a.h - u}; }
     __device__ static V sub_each(V a, U u) { return subu(a, u); }
     template <bool SIGNED>
-    __device__ static V add(V a, V b) { return V{a.l + b.l, a.h + b.h}; }
+    __device__ static V add(V a, V b, U) { return V{a.l + b.l, a.h + b.h}; }
     __device__ static V vmax(V a, V b) { return V{max(a.l, b.l), max(a.h, b.h)}; }
     __device__ static V max3(V a, V b, V c) { return V{max(max(a.l, b.l), c.l), max(max(a.h, b.h), c.h)}; }
     __device__ static V max3u(V a, V b, U c) { return V{max(max(a.l, b.l), c), max(max(a.h, b.h), c)}; }
@@ -369,12 +384,19 @@ struct SweepRows {
     }
 };
 
+// What the tables add to the scores.
+template <class A>
+__device__ __forceinline__ int table_bias(const KernelArgs& a)
+{
+    return A::kShifts ? a.bias : -(a.gap_open + a.gap_extend);
+}
+
 // Row table: byte -> code of its row (register form: its half of the selector).
 // Column table (register form): byte -> the four biased scores of its column.
-template <int PF, class S>
+template <class A, int PF, class S>
 __device__ __forceinline__ void stage_byte_tables(const KernelArgs& a, const S& sm)
 {
-    const int alpha = a.alpha, sbias = -(a.gap_open + a.gap_extend);
+    const int alpha = a.alpha, sbias = table_bias<A>(a);
     for (int i = threadIdx.x; i <= kNoRow; i += kWave) {
         int c = i < kNoRow ? (int)sm.lut()[i] : alpha;
         c = c > alpha ? alpha : c; // bytes outside the alphabet read the padding row
@@ -449,7 +471,7 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
     constexpr int UN = K <= 8 ? kSweepUnroll : 2;
     const int lane = threadIdx.x, g = lane / G, l = lane & (G - 1);
     const int alpha = a.alpha;
-    const int ge = -a.gap_extend, go = -a.gap_open, sbias = ge + go;
+    const int ge = -a.gap_extend, go = -a.gap_open, sbias = table_bias<A>(a);
     // offset of the floor (base) and of zero scores (zero)
     const int base = a.base, low = REV && strict ? kRevLow : 0, zero = base + low;
     const GroupFix fix = group_fix(l);
@@ -475,7 +497,7 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
     const bool multi_strip = G == kWave && strips_max > 1;
     const int strip_lo = SPLIT ? io.strip : 0;
 
-    const U gs = A::uni(ge), cs = A::uni(ge - go), hand_u = A::uni(ge * (K - 1));
+    const U gs = A::uni(ge), cs = A::uni(ge - go), hand_u = A::uni(ge * (K - 1)), shift = A::uni(a.shift);
     // (opaque: kept in vector registers, where the DPP subtraction takes it)
     V hand = A::from(hand_u);
     A::keep(hand);
@@ -514,7 +536,9 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
             return code < alpha ? code : -1;
         };
 
-        // ---- scores of the strip's columns (a score of 0 after the bias: padding)
+        // ---- scores of the strip's columns (a score of 0 after the bias: padding; -1
+        // where the bias is 0, so that padding scores are negative)
+        const int pad = PF == kProfWords && sbias == 0 ? -1 : 0;
         __syncthreads();
         uint32_t tlo[PF == kProfRegs ? K : 1], thi[PF == kProfRegs ? K : 1];
         if constexpr (PF == kProfRegs) {
@@ -537,7 +561,7 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
                     uint32_t w = 0;
 #pragma unroll
                     for (int b = 0; b < 4; b += P::COLB) {
-                        const int sc = (code[b] >= 0 && r < alpha) ? sub[r * alpha + code[b]] + sbias : 0;
+                        const int sc = (code[b] >= 0 && r < alpha) ? sub[r * alpha + code[b]] + sbias : pad;
                         w |= ((uint32_t)sc & (P::COLB == 1 ? 0xFFu : 0xFFFFu)) << (8 * b);
                     }
                     *(uint32_t*)(gb + r * rowstride + j4 * 4) = w;
@@ -718,7 +742,7 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
                         } else {
                             S = A::words(in.w, in.w + SweepProf<G, K, PF>::NW, k);
                         }
-                        const V D = A::template add<PF == kProfWords>(Hd, S);
+                        const V D = A::template add<PF == kProfWords>(Hd, S, shift);
                         Hd = Ho[k];
                         const V H = A::max3(D, E, F[k]);
                         const V ho = A::addu(H, cs);
@@ -945,7 +969,7 @@ __global__ __launch_bounds__(64, sweep_group_waves<A>(G, WIDE)) void k_sweep(Ker
     constexpr int PW = kWave / G;
     const SweepSmem sm = sweep_smem<A, G, PF>(smem_raw, a);
     stage_tables(a, sm);
-    stage_byte_tables<PF>(a, sm);
+    stage_byte_tables<A, PF>(a, sm);
     const int g = threadIdx.x / G;
     typename A::B* bnd_g = (typename A::B*)a.bnd + ((int64_t)blockIdx.x * PW + g) * a.bnd_rows;
     const int64_t nsets = (a.order_n + PW - 1) / PW;
@@ -987,7 +1011,7 @@ __global__ __launch_bounds__(64, A::kWide ? 2 : K <= 6 ? 4 : 3) void k_sweep_spl
     constexpr int PW = kWave / G;
     const SweepSmem sm = sweep_smem<A, G, PF>(smem_raw, a);
     stage_tables(a, sm);
-    stage_byte_tables<PF>(a, sm);
+    stage_byte_tables<A, PF>(a, sm);
     const int l = threadIdx.x & (G - 1), g = threadIdx.x / G;
     const int x = (int)(blockIdx.x % kXcds);
     const SplitArgs& sp = a.split;

@@ -5,7 +5,7 @@ namespace gbsw {
 
 const void* sweep_kernel_pairs(int kind)
 {
-    return (kind & kWideLanes) ? (const void*)&k_sweep_pairs<true> : (const void*)&k_sweep_pairs<false>;
+    return (kind & kWideLanes) ? (const void*)&k_sweep_pairs<Sweep16, true> : (const void*)&k_sweep_pairs<Sweep16, false>;
 }
 
 } // namespace gbsw

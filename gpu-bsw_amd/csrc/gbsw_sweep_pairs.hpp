@@ -56,11 +56,10 @@ __device__ __forceinline__ void row_left(uint32_t x, uint32_t y, uint32_t d, uin
 
 // One pass for the two pairs of every group of the wave (REV: the reverse one); key:
 // their winner keys, as in gbsw_pass.hpp.
-template <int K, bool REV>
+template <class A, int K, bool REV>
 __device__ __forceinline__ void sweep_pairs(const KernelArgs& a, const PairsSmem& sm, const Task (&t)[2],
                                             const int32_t (&target)[2], bool strict, uint64_t (&key)[2])
 {
-    using A = Sweep16;
     using V = uint32_t;
     constexpr int G = kLanesPerPair, R = kPairsRing, N = kChunk / G;
     constexpr int UN = K <= 8 ? kSweepUnroll : 2;
@@ -82,7 +81,7 @@ __device__ __forceinline__ void sweep_pairs(const KernelArgs& a, const PairsSmem
     steps_max = max(steps_max, __shfl_xor(steps_max, 32));
     steps_max = __builtin_amdgcn_readfirstlane(steps_max);
 
-    const uint32_t gs = A::uni(ge), cs = A::uni(ge - go);
+    const uint32_t gs = A::uni(ge), cs = A::uni(ge - go), shift = A::uni(a.shift);
     // (opaque: kept in a vector register, where the DPP subtraction takes it)
     V hand = A::uni(ge * (K - 1));
     A::keep(hand);
@@ -215,7 +214,7 @@ __device__ __forceinline__ void sweep_pairs(const KernelArgs& a, const PairsSmem
             V E = xE, Hd = Hd0;
 #pragma unroll
             for (int k = 0; k < K; ++k) {
-                const V D = Hd + __builtin_amdgcn_perm(th[k], tl[k], code);
+                const V D = A::template add<false>(Hd, __builtin_amdgcn_perm(th[k], tl[k], code), shift);
                 Hd = Ho[k];
                 const V H = A::max3(D, E, F[k]);
                 const V ho = H + cs;
@@ -328,7 +327,7 @@ __device__ __forceinline__ void sweep_pairs(const KernelArgs& a, const PairsSmem
 }
 
 // Both passes of the wave's pairs, and their results.
-template <int K>
+template <class A, int K>
 __device__ __forceinline__ void sweep_pairs_set(const KernelArgs& a, const PairsSmem& sm, const int64_t (&p)[2])
 {
     const int l = threadIdx.x & (kLanesPerPair - 1);
@@ -338,7 +337,7 @@ __device__ __forceinline__ void sweep_pairs_set(const KernelArgs& a, const Pairs
     Task t[2];
     {
         const Task tf[2] = {forward_task(a, p[0]), forward_task(a, p[1])};
-        sweep_pairs<K, false>(a, sm, tf, none, false, key);
+        sweep_pairs<A, K, false>(a, sm, tf, none, false, key);
     }
     int32_t target[2];
     bool swaps = false;
@@ -351,7 +350,7 @@ __device__ __forceinline__ void sweep_pairs_set(const KernelArgs& a, const Pairs
         swaps |= p[h] >= 0 && f[h].score > 0 && reverse_swaps(a, p[h], f[h]);
     }
     const bool strict = __ballot(swaps) == 0;
-    sweep_pairs<K, true>(a, sm, t, target, strict, key);
+    sweep_pairs<A, K, true>(a, sm, t, target, strict, key);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         int32_t rb, qb;
@@ -370,14 +369,14 @@ __device__ __forceinline__ void sweep_pairs_set(const KernelArgs& a, const Pairs
 // gives their geometries, as in k_sweep.
 // WIDE: the geometries of K > kPairsNarrowMax; apart, since their registers spill more
 // outside the loops (one kernel for all: 14.6 ms for the 858k pairs, two 14.4).
-template <bool WIDE>
+template <class A, bool WIDE>
 __global__ __launch_bounds__(64, 4) void k_sweep_pairs(KernelArgs a)
 {
     extern __shared__ __align__(16) uint8_t smem_raw[];
     constexpr int PW = 8;
     const PairsSmem sm{smem_raw, pairs_lds(a.kmax, a.alpha)};
     stage_tables(a, sm);
-    stage_byte_tables<kProfRegs>(a, sm);
+    stage_byte_tables<A, kProfRegs>(a, sm);
     const int g = threadIdx.x / kLanesPerPair;
     const int64_t nsets = (a.order_n + PW - 1) / PW;
     for (;;) {
@@ -389,7 +388,7 @@ __global__ __launch_bounds__(64, 4) void k_sweep_pairs(KernelArgs a)
         int K = a.ranges[a.nranges - 1].K;
         for (int r = a.nranges - 2; r >= 0; --r)
             if ((int64_t)q * PW < a.ranges[r].end) K = a.ranges[r].K;
-#define GBSW_CASE(k) case k: sweep_pairs_set<k>(a, sm, p); break;
+#define GBSW_CASE(k) case k: sweep_pairs_set<A, k>(a, sm, p); break;
         if constexpr (WIDE) {
             switch (K) { GBSW_SWEEP_PAIRS_WIDE(GBSW_CASE) }
         } else {

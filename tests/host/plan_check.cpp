@@ -70,7 +70,7 @@ const char* check(std::vector<Len> v, int alphabet, bool split, bool fixed, int*
     std::vector<int16_t> sub((size_t)(alpha * alpha), (int16_t)(dna ? -3 : -4));
     for (int c = 0; c < alpha; ++c) sub[(size_t)(c * alpha + c)] = dna ? 3 : 6;
     const int max_sub = dna ? 3 : 6;
-    const SweepChoice sw = sweep_choice(sub, alpha, -6, -1, max_sub, true);
+    const SweepChoice sw = sweep_choice(sub, alpha, -6, -1, max_sub, true, j.max_cols);
     Exec ex;
     ex.num_cu = 256;
     ex.fixed = fixed;
@@ -129,7 +129,7 @@ int64_t int32_pairs(const std::vector<Len>& v, int alphabet, int alpha, int16_t 
     Exec ex;
     ex.num_cu = 256;
     std::vector<BucketPlan> plan;
-    plan_sweeps(ex, j, sweep_choice(sub, alpha, -6, -1, std::max(same, rare), true), true, false, plan);
+    plan_sweeps(ex, j, sweep_choice(sub, alpha, -6, -1, std::max(same, rare), true, j.max_cols), true, false, plan);
     int64_t n = 0;
     for (const BucketPlan& b : plan)
         if ((b.kind & 0xFF) == kBatchedWide) n += b.bk.count;
