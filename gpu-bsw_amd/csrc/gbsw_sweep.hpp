@@ -31,8 +31,8 @@
 // (all 2^21 random triples of such patterns gave the integer maximum).  base
 // keeps every value non-negative, and a pair whose score comes near the top of
 // that range is recomputed with int32 cells: cell values grow by at most one
-// substitution per cell, so the best score passes sat_limit before any value
-// passes 0x7C00, and whatever the halves hold after that, the recorded best stays.
+// substitution per cell, so some lane's threshold passes sat_limit before any value
+// passes 0x7C00, and whatever the halves hold after that, thresholds only rise.
 //
 // Scores: with at most four residue codes a lane keeps, per column, the four
 // scores S'' as the bytes of one register, and one v_perm picks the scores of both
@@ -900,6 +900,13 @@ __device__ __forceinline__ PassResult sweep(const KernelArgs& a, const SweepSmem
         const uint64_t o = ((uint64_t)(uint32_t)__shfl_xor((int)(uint32_t)(key >> 32), x) << 32) |
                            (uint32_t)__shfl_xor((int)(uint32_t)key, x);
         key = o > key ? o : key;
+    }
+    if constexpr (!REV && !A::kWide) {
+        // The thresholds never fall (but by one from strip to strip).  A row that a lane
+        // kept may have been replaced where the pair is past its range, by padding rows or
+        // columns, whose values then mean nothing: such a pair is recomputed.
+        const int32_t top = A::lo(A::template group_max<G>(bt)) + strips_g;
+        if (strips_g > strip_lo && top >= a.sat_limit) key = max(key, (uint64_t)top << 40);
     }
     PassResult r;
     r.key = key;

@@ -289,6 +289,13 @@ __device__ __forceinline__ void sweep_pairs(const KernelArgs& a, const PairsSmem
     }
 
     // ---- candidates, reduced over each group
+    V most = bt; // forward: the groups' highest thresholds (see sweep)
+    if constexpr (!REV) {
+        most = pk_max(most, row_ror<1>(most));
+        most = pk_max(most, row_ror<2>(most));
+        most = pk_max(most, row_ror<4>(most));
+        most = pk_max(most, row_ror<8>(most));
+    }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         uint64_t k64 = 0;
@@ -322,6 +329,8 @@ __device__ __forceinline__ void sweep_pairs(const KernelArgs& a, const PairsSmem
                                (uint32_t)__shfl_xor((int)(uint32_t)k64, x);
             k64 = o > k64 ? o : k64;
         }
+        const int32_t top = h ? A::hi(most) : A::lo(most);
+        if (!REV && live[h] && top >= a.sat_limit) k64 = max(k64, (uint64_t)top << 40);
         key[h] = k64;
     }
 }
