@@ -787,7 +787,7 @@ int gbsw_batch_traceback(gbsw_batch* b, const gbsw_scoring* sc, int64_t capacity
         for (int c = 0; c < kTbAreas; ++c) {
             const double k = counts.pairs[c];
             const int kmax = tb_kmax(cells_of(counts.value[c]), form);
-            // a class spans a factor of two in area: its mean lies near 0.7 of the largest
+            // (every set as its class's largest rows and columns)
             const double s16 = k ? tb_set_cost((int)counts.rows[c], (int)counts.cols[c], 16, kmax) : 0.0;
             const double s64 = k ? tb_set_cost((int)counts.rows[c], (int)counts.cols[c], 64, kmax) : 0.0;
             w16[c] = std::ceil(k / 8) * s16;

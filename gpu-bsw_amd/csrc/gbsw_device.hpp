@@ -55,12 +55,12 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ f16x2 as_h(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
 __device__ __forceinline__ uint32_t raw(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
 // v_pk_maximum3_f16 (gfx950): max of three per half.  The IEEE maximum (unlike maxnum)
-// takes no canonicalising max per operand; the operands are never NaN.
+// takes no canonicalising max per operand.  Patterns past 0x7C00 are NaN: they come up
+// only in pairs that are past their range and recomputed.
 __device__ __forceinline__ uint32_t pk_max3_f16(uint32_t a, uint32_t b, uint32_t c)
 {
     return raw(__builtin_elementwise_maximum(__builtin_elementwise_maximum(as_h(a), as_h(b)), as_h(c)));
 }
-__host__ __device__ inline uint16_t f16_bits(int32_t x) { return __builtin_bit_cast(uint16_t, (_Float16)x); }
 
 // v_bfi_b32 with a wave-uniform (SGPR) second operand.
 __device__ __forceinline__ uint32_t bfi_s(uint32_t m, uint32_t a, uint32_t b)

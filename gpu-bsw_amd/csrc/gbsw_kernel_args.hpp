@@ -185,9 +185,8 @@ __host__ __device__ constexpr int32_t kstride(int32_t K) { return K / 8 * 8 + kr
 // the (alpha+1)-row profile of a strip takes half the LDS and leaves room for
 // more waves per CU.  Layout of one row: K/16 blocks of 16 columns for all 32
 // virtual lanes (one b128 read each), then the K%16 remaining columns padded to
-// a b32/b64/b96/b128 read (kremstride8).  With the f16 kernels (DNA-like
-// tables whose scores are f16 values with a zero low byte) a byte is the high
-// byte of the score's f16 bits instead.
+// a b32/b64/b96/b128 read (kremstride8).  The sweep kernels lay their byte profiles
+// out alike, with biased scores (0: padding).
 constexpr int kByteProfileAlpha = 8;
 __host__ __device__ constexpr int32_t kremstride8(int32_t K)
 {

@@ -1077,7 +1077,6 @@ static const void* kernel_for(int kind, int K)
                                  : kernel_for_profile<false>(kind, K);
 }
 
-bool kernel_supported(int K) { return kernel_for(kPlainForward, K) != nullptr; }
 bool kernel_has(int kind, int K) { return kernel_for(kind, K) != nullptr; }
 
 const int* wide_k_list(int* count)

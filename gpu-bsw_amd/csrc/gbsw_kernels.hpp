@@ -60,7 +60,6 @@ constexpr int kSplitStrips = 0x1000;
 #define GBSW_SWEEP_K32(X) X(2) X(4)
 const void* sweep_kernel_int32(int kind, int K);
 
-bool kernel_supported(int K);
 bool kernel_has(int kind, int K);
 const int* kernel_k_list(int* count); // K values with compiled kernels, ascending
 const int* wide_k_list(int* count);   // K values of the int32 (kBatchedWide) kernel

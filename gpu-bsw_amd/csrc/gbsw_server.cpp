@@ -401,7 +401,8 @@ void gbsw_server::admit(Slot& s)
     Bucket sum[kClasses];
     int64_t pairs = 0, res = 0, wide = 0, cells = 0;
     int32_t max_rows = 0, max_cols = 0;
-    // boundary rows: one workgroup per pair of several strips, up to a full grid
+    // boundary rows: one workgroup per pair of several strips, up to a full grid (the
+    // plan shrinks its grids, and drops the split form, until they fit)
     auto bnd_need = [&](int64_t wide, int32_t rows) {
         return std::min<int64_t>(T.wide_full, std::max<int64_t>(1, wide)) * (int64_t)std::max(1, rows) * 4;
     };

@@ -27,8 +27,8 @@
 // steps the state drops the g x kRebase it has accumulated.
 //
 // The maxima are v_pk_maximum3_f16 on integers: the bit patterns of non-negative
-// f16 values up to infinity (0x7C00) order as integers do, denormals included
-// (all 2^21 random triples of such patterns gave the integer maximum).  base
+// f16 values up to infinity (0x7C00) order as integers do, denormals (below 0x400,
+// where most values of short pairs lie) included: the instruction keeps them.  base
 // keeps every value non-negative, and a pair whose score comes near the top of
 // that range is recomputed with int32 cells: cell values grow by at most one
 // substitution per cell, so some lane's threshold passes sat_limit before any value

@@ -117,8 +117,9 @@ EXPORTED = (
     "gbsw_context_set_option", "gbsw_batch_traceback", "gbsw_align_noalloc",
 )
 OPT_STREAMS, OPT_F16, OPT_GEOMETRY, OPT_SPLIT, OPT_GRAPHS = 1, 2, 3, 4, 5
-# launch kinds (gbsw_launch_stat.kind): plain forward, plain reverse, batched
-# int16, batched int32, batched f16; plus KIND_BYTE_PROFILE for int8 profiles
+# launch kinds (gbsw_launch_stat.kind): plain forward, plain reverse, batched int16,
+# batched int32, sweep kernels, their split forms, eight pairs per wave; plus
+# KIND_BYTE_PROFILE where scores are held as bytes
 KIND_PLAIN_FORWARD, KIND_PLAIN_REVERSE, KIND_BATCHED, KIND_BATCHED_WIDE, KIND_BATCHED_F16 = 0, 1, 2, 3, 4
 KIND_SPLIT, KIND_SPLIT_F16, KIND_BATCHED_PAIRS = 5, 6, 7
 KIND_BYTE_PROFILE = 256
