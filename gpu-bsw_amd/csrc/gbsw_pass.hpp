@@ -327,6 +327,7 @@ __device__ __forceinline__ void reverse_plan_finish(const KernelArgs& a, int64_t
     if (r.target <= 0) r.t = empty_task(a, 1);
     if (r.target >= a.sat_limit) {
         r.saturated = true;
+        r.target = 0; // (nothing to reach in this pass)
         r.t = empty_task(a, 1);
         if ((threadIdx.x & (G - 1)) == 0) {
             const int32_t slot = atomicAdd(a.status + kStatusSaturated, 1);
