@@ -788,6 +788,14 @@ size_t plan_int32(const Exec& ex, const Job& job, const SweepChoice& sw, std::ve
     return n;
 }
 
+// Whether a plan's stretches are those of the fine classes.
+bool plan_is_fine(const std::vector<BucketPlan>& plan)
+{
+    for (const BucketPlan& b : plan)
+        if (b.kind & kHalfPairs) return true;
+    return false;
+}
+
 // Eight pairs per wave: jobs with two such waves per SIMD and more (fewer leave SIMDs
 // idle) and register tables, where the estimate is less.
 void plan_sweeps(const Exec& ex, const Job& job, const SweepChoice& sw, bool may_split, bool asym,
@@ -804,15 +812,8 @@ void plan_sweeps(const Exec& ex, const Job& job, const SweepChoice& sw, bool may
         job.n < 8 * 2 * 4 * (int64_t)ex.num_cu)
         return;
     std::vector<BucketPlan> other;
-    if (plan_sweeps_over(ex, job, job.fine, sw, may_split, true, other) < t) plan.swap(other);
-}
-
-// Whether a plan's stretches are those of the fine classes.
-bool plan_is_fine(const std::vector<BucketPlan>& plan)
-{
-    for (const BucketPlan& b : plan)
-        if (b.kind & kHalfPairs) return true;
-    return false;
+    // (only with that kernel in it: the pairs are then sorted by the fine classes)
+    if (plan_sweeps_over(ex, job, job.fine, sw, may_split, true, other) < t && plan_is_fine(other)) plan.swap(other);
 }
 
 // The launches of a job on the int16 kernels (scorings outside the sweep kernels'

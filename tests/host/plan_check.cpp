@@ -106,6 +106,7 @@ const char* check(std::vector<Len> v, int alphabet, bool split, bool fixed, int*
             for (int64_t x = q * PW; x < std::min((q + 1) * PW, b.bk.count); ++x) {
                 const Len& l = v[(size_t)(b.bk.begin + x)];
                 const int lanes = pairs ? kLanesPerPair : 2 * b.G;
+                if (l.rows > b.bk.max_rows) return "a pair of more rows than the launch has boundary rows for";
                 if ((pairs || b.G != kWave) && l.cols > lanes * K) return "a pair wider than its one strip";
                 if (b.G == kWave && (l.cols + lanes * K - 1) / (lanes * K) > std::max(1, b.strips))
                     return "a pair of more strips than the launch has boundary rows for";
